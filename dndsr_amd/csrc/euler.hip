@@ -62,33 +62,43 @@ __global__ void __launch_bounds__(256) kDtFace(DevMesh m, GasParams gp, const re
     dLamF[f] = max3(fabs(dvn + aR - aL), fabs(dvn - aR + aL), fabs(aL - aR));
 }
 
+// Loads issued together as in kRHSGather; blockDim.x is a power of two of at most 256.
+template <int KM>
 __global__ void __launch_bounds__(256) kDtCell(DevMesh m, real CFL, real maxDt, const real *__restrict__ lam,
                                                const real *__restrict__ dLamF, real *__restrict__ dt,
                                                real *__restrict__ dlc, real *__restrict__ partMin)
 {
     __shared__ real sm[256];
-    idx i = blockIdx.x * blockDim.x + threadIdx.x;
+    const idx i = xcdTile(blockIdx.x, gridDim.x) * (idx)blockDim.x + threadIdx.x;
     real d = 3e200;
     if (i < m.N)
     {
-        real lc = 0, dl = 0;
-        for (int k = 0; k < m.K; k++)
+        idx f[KM];
+#pragma unroll
+        for (int k = 0; k < KM; k++)
+            f[k] = k < m.K ? m.c2f[(size_t)k * m.N + i] : idx(-1);
+        const real vs = CFL * m.vol[i] * m.smooth[i];
+        real l[KM], A[KM], dl[KM];
+#pragma unroll
+        for (int k = 0; k < KM; k++)
         {
-            idx f = m.c2f[(size_t)k * m.N + i];
-            if (f < 0)
-                continue;
-            lc += lam[f] * m.farea[f];
-            dl = fmax(dl, dLamF[f]);
+            const idx ff = f[k] < 0 ? 0 : f[k];
+            l[k] = lam[ff], A[k] = m.farea[ff], dl[k] = dLamF[ff];
         }
-        d = fmin(CFL * m.vol[i] * m.smooth[i] / (lc + 1e-100), maxDt);
+        real lc = 0, dm = 0;
+#pragma unroll
+        for (int k = 0; k < KM; k++)
+            if (f[k] >= 0)
+                lc += l[k] * A[k], dm = fmax(dm, dl[k]);
+        d = fmin(vs / (lc + 1e-100), maxDt);
         if (dt)
             dt[i] = d;
         if (dlc)
-            dlc[i] = dl;
+            dlc[i] = dm;
     }
     sm[threadIdx.x] = d;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1)
+    for (int s = blockDim.x / 2; s > 0; s >>= 1)
     {
         if (threadIdx.x < s)
             sm[threadIdx.x] = fmin(sm[threadIdx.x], sm[threadIdx.x + s]);
@@ -132,17 +142,21 @@ void launchEvalDt(Ctx &c, const GasParams &gp, const real *u, real CFL, real max
         kDtFace<<<gridFor(m.F, 256), 256, 0, c.stream>>>(m, gp, u, lambdaFace, c.faceLamTmp);
         DNDSR_HIP_CHECK(hipGetLastError());
     }
-    int nb = gridFor(m.N, 256);
+    const int bs = cellBlock(m.N), nb = gridFor(m.N, bs);
     {
         KernelTimer kt(c, K_DT_CELL);
-        kDtCell<<<nb, 256, 0, c.stream>>>(m, CFL, maxDt, lambdaFace, c.faceLamTmp, dt, deltaLambdaCell, c.red);
+        if (m.K <= 4)
+            kDtCell<4><<<nb, bs, 0, c.stream>>>(m, CFL, maxDt, lambdaFace, c.faceLamTmp, dt, deltaLambdaCell, c.red);
+        else
+            kDtCell<kMaxFC><<<nb, bs, 0, c.stream>>>(m, CFL, maxDt, lambdaFace, c.faceLamTmp, dt, deltaLambdaCell,
+                                                     c.red);
         DNDSR_HIP_CHECK(hipGetLastError());
     }
     kReduceMin<<<1, 256, 0, c.stream>>>(c.red, nb, dtMinDev);
     DNDSR_HIP_CHECK(hipGetLastError());
     if (!useLocalDt && dt)
     {
-        kFillFromScalar<<<nb, 256, 0, c.stream>>>(m.N, dtMinDev, dt);
+        kFillFromScalar<<<gridFor(m.N, 256), 256, 0, c.stream>>>(m.N, dtMinDev, dt);
         DNDSR_HIP_CHECK(hipGetLastError());
     }
 }
@@ -457,28 +471,50 @@ kRHSFace(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__rest
     }
 }
 
+// Gather of the face fluxes into the residual, one thread per cell.  The kernel is bound by the
+// latency of its dependent loads (face index -> flux) when the mesh is small and by the gathers'
+// cache lines when it is large, so a thread issues all its face indices and side flags at once and
+// then all 5 K fluxes (KM >= K slots, unrolled; a slot past K or without a face reads a valid row
+// with weight 0: a load under a branch would wait for every earlier one at the join), and divides
+// the sum by the volume once.  The side comes from the slot flags, not from a load that depends on
+// the face index.
+template <int KM>
 __global__ void __launch_bounds__(256) kRHSGather(DevMesh m, const real *__restrict__ fflux, real *__restrict__ rhs,
                                                   StageUpdate st, int *__restrict__ nonFinite)
 {
-    idx i = blockIdx.x * blockDim.x + threadIdx.x;
+    const idx i = xcdTile(blockIdx.x, gridDim.x) * (idx)blockDim.x + threadIdx.x;
     if (i >= m.N)
         return;
     const size_t N = m.N, F = m.F;
-    real vol = m.vol[i];
-    real acc[5] = {0, 0, 0, 0, 0};
-    for (int k = 0; k < m.K; k++)
+    idx f[KM];
+    real w[KM];
+#pragma unroll
+    for (int k = 0; k < KM; k++)
     {
-        idx f = m.c2f[(size_t)k * N + i];
-        if (f < 0)
-            continue;
-        bool back = m.f2c[f] == i;
+        const size_t q = (size_t)(k < m.K ? k : 0) * N + i;
+        f[k] = m.c2f[q];
+        w[k] = (m.c2flag[q] & 1) ? -1.0 : 1.0; // bit 0: the cell is the face's front side
+        if (k >= m.K || f[k] < 0)
+            w[k] = 0, f[k] = 0;
+    }
+    const real vol = m.vol[i];
+    const real dt = st.u && st.dtDev ? st.dtDev[0] : 1.0;
+    real fv[KM][5];
+#pragma unroll
+    for (int k = 0; k < KM; k++)
 #pragma unroll
         for (int v = 0; v < 5; v++)
-        {
-            real fv = fflux[v * F + f];
-            acc[v] += (back ? fv : -fv) / vol;
-        }
-    }
+            fv[k][v] = fflux[v * F + f[k]];
+    real acc[5] = {0, 0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < KM; k++)
+        if (w[k] != 0) // an unused slot contributes nothing, whatever face 0 holds
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+                acc[v] += w[k] * fv[k][v];
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+        acc[v] /= vol;
     // the reference asserts on non-finite fluxes (EulerEvaluator_EvaluateRHS.hxx:387-398, 782-788);
     // here the first one raises a flag the host reads at its next synchronisation
     if (nonFinite && !(isfinite(acc[0]) && isfinite(acc[1]) && isfinite(acc[2]) && isfinite(acc[3]) && isfinite(acc[4])))
@@ -491,7 +527,6 @@ __global__ void __launch_bounds__(256) kRHSGather(DevMesh m, const real *__restr
     }
     if (st.u) // same arithmetic as kAxpby(a, u, b, y, cdt, rhs, dt)
     {
-        const real dt = st.dtDev ? st.dtDev[0] : 1.0;
 #pragma unroll
         for (int v = 0; v < 5; v++)
         {
@@ -1312,8 +1347,13 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
         DNDSR_HIP_CHECK(hipGetLastError());
     }
     KernelTimer kt2(c, K_RHS_GATHER);
-    kRHSGather<<<gridFor(m.N, 256), 256, 0, c.stream>>>(m, ff, rhs, stage ? *stage : StageUpdate{},
-                                                         flagNonFinite ? c.nonFinite : nullptr);
+    const int bs = cellBlock(m.N), nb2 = gridFor(m.N, bs);
+    const StageUpdate su = stage ? *stage : StageUpdate{};
+    int *flag = flagNonFinite ? c.nonFinite : nullptr;
+    if (m.K <= 4)
+        kRHSGather<4><<<nb2, bs, 0, c.stream>>>(m, ff, rhs, su, flag);
+    else
+        kRHSGather<kMaxFC><<<nb2, bs, 0, c.stream>>>(m, ff, rhs, su, flag);
     DNDSR_HIP_CHECK(hipGetLastError());
 }
 

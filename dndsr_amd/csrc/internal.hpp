@@ -357,6 +357,9 @@ T *devAlloc(Ctx &c, size_t n)
 }
 
 inline int gridFor(idx n, int block) { return (int)((n + block - 1) / block); }
+// Block size of the one-thread-per-cell gathers: one wavefront while 256-thread blocks would leave
+// CUs without any (fewer than 512 of them), so that a small mesh spreads over the device
+inline int cellBlock(idx n) { return n < 512 * 256 ? 64 : 256; }
 
 // Skipped colour passes of the symmetric Gauss-Seidel sweeps: a sweep may skip its first colour
 // (fCol; its current values stay in the array the sweep reads) and read the colour the previous
