@@ -225,17 +225,80 @@ static void vrIterDiffM(Ctx &c, int nVars, const real *x, real *y)
 // MODE 0: Jacobi (scale = relax); 1: recordInc (scale = -1); 2: the Jacobian action
 // (uB(uBL + D0phi x) - uB(uBL) in place of uB - u_i, scale = -1).
 // ---------------------------------------------------------------------------
-// BCC of boundary face f of cell i (mom, cen, isc: the cell's moments, centre and scale;
-// um its mean): the own block is read through rec(v, j) and, for LIN, the Jacobian
-// direction through dx(v, j).
+// Point g of boundary face f of cell i (mom, cen, isc: the cell's moments, centre and scale; um its
+// mean): the basis values phi and inc = uB - u_i (LIN: the ghost's change along dx).  The own block
+// is read through rec(v, j) and, for LIN, the Jacobian direction through dx(v, j).
 template <int DIM, int NDOF, int NV, bool LIN, class Rec, class Dx>
-__device__ inline void boundaryFaceBCC(const DevMesh &m, idx f, const real *mom, const real *cen, real isc,
-                                       const real *um, Rec rec, Dx dx, real (&BCC)[NDOF - 1][NV])
+__device__ inline void boundaryPointInc(const DevMesh &m, idx f, int g, const real *mom, const real *cen, real isc,
+                                        const real *um, Rec rec, Dx dx, real (&phi)[NDOF - 1], real (&inc)[NV])
 {
     constexpr int M = NDOF - 1;
     const size_t F = m.F;
     const bool euler = NV == 5 && m.bcType != nullptr;
-    const int zone = m.fzone[f];
+    real xs[3];
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+    {
+        xs[r] = m.fpts[((size_t)g * 3 + r) * F + f] - cen[r];
+        if (DIM == 3 || r < 2)
+            xs[r] *= isc;
+    }
+    basisRow0<DIM, NDOF>(xs, mom, phi);
+    if (euler)
+    {
+        const int zone = m.fzone[f];
+        real uBL[5], n[3], ULf[5], uB[5];
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            real r = 0;
+#pragma unroll
+            for (int j = 0; j < M; j++)
+                r += phi[j] * rec(v, j);
+            uBL[v] = r;
+        }
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+            n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
+        const real *far = m.bcVal + (size_t)zone * 5;
+        const int type = m.bcType[zone];
+        compressRecPart(um, uBL, ULf);
+        bcGhost(type, ULf, n, far, m.bcGamma, uB);
+        if constexpr (LIN)
+        {
+            real in2[5], ULp[5], uBp[5];
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+            {
+                real r = 0;
+#pragma unroll
+                for (int j = 0; j < M; j++)
+                    r += phi[j] * dx(v, j);
+                in2[v] = uBL[v] + r;
+            }
+            compressRecPart(um, in2, ULp);
+            bcGhost(type, ULp, n, far, m.bcGamma, uBp);
+#pragma unroll
+            for (int v = 0; v < NV; v++)
+                inc[v] = uBp[v] - uB[v];
+        }
+        else
+#pragma unroll
+            for (int v = 0; v < NV; v++)
+                inc[v] = uB[v] - um[v];
+    }
+    else
+#pragma unroll
+        for (int v = 0; v < NV; v++)
+            inc[v] = LIN ? 0.0 : m.dirVal[((size_t)v * m.G + g) * F + f] - um[v];
+}
+
+// BCC of boundary face f of cell i, its points one after the other (the SOR sweep)
+template <int DIM, int NDOF, int NV, class Rec>
+__device__ inline void boundaryFaceBCC(const DevMesh &m, idx f, const real *mom, const real *cen, real isc,
+                                       const real *um, Rec rec, real (&BCC)[NDOF - 1][NV])
+{
+    constexpr int M = NDOF - 1;
     const real w0 = m.faceW[f]; // order-0 weight; faceL^0 = 1
     const real w2 = w0 * w0;
 #pragma unroll
@@ -245,63 +308,9 @@ __device__ inline void boundaryFaceBCC(const DevMesh &m, idx f, const real *mom,
             BCC[j][v] = 0;
     for (int g = 0; g < m.G; g++)
     {
-        real xs[3], phi[M];
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-        {
-            xs[r] = m.fpts[((size_t)g * 3 + r) * F + f] - cen[r];
-            if (DIM == 3 || r < 2)
-                xs[r] *= isc;
-        }
-        basisRow0<DIM, NDOF>(xs, mom, phi);
-        real inc[NV];
-        if (euler)
-        {
-            real uBL[5], n[3], ULf[5], uB[5];
-#pragma unroll
-            for (int v = 0; v < 5; v++)
-            {
-                real r = 0;
-#pragma unroll
-                for (int j = 0; j < M; j++)
-                    r += phi[j] * rec(v, j);
-                uBL[v] = r;
-            }
-#pragma unroll
-            for (int r = 0; r < 3; r++)
-                n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
-            const real *far = m.bcVal + (size_t)zone * 5;
-            const int type = m.bcType[zone];
-            compressRecPart(um, uBL, ULf);
-            bcGhost(type, ULf, n, far, m.bcGamma, uB);
-            if constexpr (LIN)
-            {
-                real in2[5], ULp[5], uBp[5];
-#pragma unroll
-                for (int v = 0; v < 5; v++)
-                {
-                    real r = 0;
-#pragma unroll
-                    for (int j = 0; j < M; j++)
-                        r += phi[j] * dx(v, j);
-                    in2[v] = uBL[v] + r;
-                }
-                compressRecPart(um, in2, ULp);
-                bcGhost(type, ULp, n, far, m.bcGamma, uBp);
-#pragma unroll
-                for (int v = 0; v < NV; v++)
-                    inc[v] = uBp[v] - uB[v];
-            }
-            else
-#pragma unroll
-                for (int v = 0; v < NV; v++)
-                    inc[v] = uB[v] - um[v];
-        }
-        else
-#pragma unroll
-            for (int v = 0; v < NV; v++)
-                inc[v] = LIN ? 0.0 : m.dirVal[((size_t)v * m.G + g) * F + f] - um[v];
-        const real fac = m.fwj[(size_t)g * F + f];
+        real phi[M], inc[NV];
+        boundaryPointInc<DIM, NDOF, NV, false>(m, f, g, mom, cen, isc, um, rec, rec, phi, inc);
+        const real fac = m.fwj[(size_t)g * m.F + f];
 #pragma unroll
         for (int j = 0; j < M; j++)
 #pragma unroll
@@ -310,70 +319,151 @@ __device__ inline void boundaryFaceBCC(const DevMesh &m, idx f, const real *mom,
     }
 }
 
-// The boundary term in two passes.  kVRBndFace: one thread per boundary face, A^-1 BCC of the
-// face (BCC from the owner cell's block, A^-1 = the cell's slot-0 block) into vrBnd; kVRBndCell:
-// one thread per boundary cell adds scale times its faces' terms in slot order.  (One thread per
-// boundary cell doing both would run, in every wave, each slot that any lane has on the
-// boundary.)
+// The boundary term in two passes.  kVRBndFace: A^-1 BCC of every boundary face (BCC from the owner
+// cell's block, A^-1 = the cell's slot-0 block) into vrBnd; kVRBndCell adds scale times its faces'
+// terms to every boundary cell in slot order.  (One thread per boundary cell doing both would run,
+// in every wave, each slot that any lane has on the boundary.)
+//
+// The boundary is a few thousand faces, a handful of wavefronts per CU at one thread per face: the
+// pass is bound by its chain of dependent loads and arithmetic, not by bandwidth.  A block is 64
+// faces with one wavefront per face point (two rounds of points above 8): the points' basis values
+// and increments go through LDS, then wavefront w forms the column v = w, w + NW, ... of BCC in point
+// order and applies A^-1.
 template <int DIM, int NDOF, int NV, int MODE>
-__global__ void __launch_bounds__(64) kVRBndFace(DevMesh m, const real *__restrict__ uRec, const real *__restrict__ u,
-                                                 const real *__restrict__ x, real *__restrict__ out)
+__global__ void __launch_bounds__(512) kVRBndFace(DevMesh m, const real *__restrict__ uRec, const real *__restrict__ u,
+                                                  const real *__restrict__ x, real *__restrict__ out)
 {
-    constexpr int M = NDOF - 1;
-    const idx t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= m.nBnd)
-        return;
-    const idx f = m.bndFace[t];
+    constexpr int M = NDOF - 1, ROWS = M + NV;
+    extern __shared__ real sPt[]; // [NW][M + NV][64]
+    const int lane = threadIdx.x % 64, w = waveIndex(64), NW = blockDim.x / 64;
+    const idx t = blockIdx.x * 64 + lane;
+    const bool valid = t < m.nBnd;
+    const idx f = m.bndFace[valid ? t : m.nBnd - 1];
     const idx i = m.f2c[f];
     const size_t N = m.N, NB = m.nBnd;
-    real mom[M], cen[3], um[NV];
+    {
+        real mom[M], cen[3], um[NV], own[NV][M];
 #pragma unroll
-    for (int j = 0; j < M; j++)
-        mom[j] = m.moment[(size_t)j * N + i];
+        for (int j = 0; j < M; j++)
+            mom[j] = m.moment[(size_t)j * N + i];
 #pragma unroll
-    for (int r = 0; r < 3; r++)
-        cen[r] = m.cent[(size_t)r * N + i];
-    const real isc = m.iscale[i];
+        for (int r = 0; r < 3; r++)
+            cen[r] = m.cent[(size_t)r * N + i];
+        const real isc = m.iscale[i];
+        const real w0 = m.faceW[f];
 #pragma unroll
-    for (int v = 0; v < NV; v++)
-        um[v] = u ? u[(size_t)v * N + i] : 0.0;
-    auto rec = [&](int v, int j) { return uRec[((size_t)v * M + j) * N + i]; };
-    auto dx = [&](int v, int j) { return x[((size_t)v * M + j) * N + i]; };
-    real BCC[M][NV];
-    boundaryFaceBCC<DIM, NDOF, NV, MODE == 2>(m, f, mom, cen, isc, um, rec, dx, BCC);
+        for (int v = 0; v < NV; v++)
+            um[v] = u ? u[(size_t)v * N + i] : 0.0;
+        // a small block stays in registers across the points
+        constexpr bool REG = M <= 3;
+        if constexpr (REG)
+            if (NV == 5 && m.bcType != nullptr)
 #pragma unroll
-    for (int v = 0; v < NV; v++)
+                for (int v = 0; v < NV; v++)
 #pragma unroll
-        for (int r = 0; r < M; r++)
+                    for (int j = 0; j < M; j++)
+                        own[v][j] = uRec[((size_t)v * M + j) * N + i];
+        auto rec = [&](int v, int j) {
+            if constexpr (REG)
+                return own[v][j];
+            else
+                return uRec[((size_t)v * M + j) * N + i];
+        };
+        auto dx = [&](int v, int j) { return x[((size_t)v * M + j) * N + i]; };
+        real B[M]; // with more points than wavefronts: this wavefront's column, summed over the rounds
+#pragma unroll
+        for (int j = 0; j < M; j++)
+            B[j] = 0;
+        auto addPoints = [&](int v, int n) {
+            for (int g = 0; g < n; g++)
+            {
+                const real *row = sPt + (size_t)g * ROWS * 64 + lane;
+                const real q = row[(M + v) * 64];
+#pragma unroll
+                for (int j = 0; j < M; j++)
+                    B[j] += row[j * 64] * q;
+            }
+        };
+        auto finish = [&](int v) {
+            if (valid)
+#pragma unroll
+                for (int r = 0; r < M; r++)
+                {
+                    real acc = 0;
+#pragma unroll
+                    for (int c2 = 0; c2 < M; c2++)
+                        acc += m.AinvB[((size_t)r * M + c2) * N + i] * B[c2];
+                    out[((size_t)v * M + r) * NB + t] = acc;
+                }
+        };
+        for (int base = 0; base < m.G; base += NW)
         {
-            real acc = 0;
+            const int g = base + w;
+            if (g < m.G)
+            {
+                real phi[M], inc[NV];
+                boundaryPointInc<DIM, NDOF, NV, MODE == 2>(m, f, g, mom, cen, isc, um, rec, dx, phi, inc);
+                const real fac = m.fwj[(size_t)g * m.F + f] * (w0 * w0);
+                real *row = sPt + (size_t)w * ROWS * 64 + lane;
 #pragma unroll
-            for (int c2 = 0; c2 < M; c2++)
-                acc += m.AinvB[((size_t)r * M + c2) * N + i] * BCC[c2][v];
-            out[((size_t)v * M + r) * NB + t] = acc;
+                for (int j = 0; j < M; j++)
+                    row[j * 64] = phi[j];
+#pragma unroll
+                for (int v = 0; v < NV; v++)
+                    row[(M + v) * 64] = inc[v] * fac;
+            }
+            __syncthreads();
+            if (m.G > NW) // then NW >= 5 >= NV: one column per wavefront
+            {
+                if (w < NV)
+                    addPoints(w, min(NW, m.G - base));
+                __syncthreads();
+            }
         }
+        if (m.G > NW)
+        {
+            if (w < NV)
+                finish(w);
+        }
+        else
+            for (int v = w; v < NV; v += NW)
+            {
+#pragma unroll
+                for (int j = 0; j < M; j++)
+                    B[j] = 0;
+                addPoints(v, m.G);
+                finish(v);
+            }
+    }
 }
 
+// one thread per boundary cell and variable (blockIdx.y), the cell's row updated once
 template <int M, int NV>
 __global__ void __launch_bounds__(64) kVRBndCell(DevMesh m, const real *__restrict__ bt, real *__restrict__ uRecNew,
                                                  real scale)
 {
     const idx j = blockIdx.x * blockDim.x + threadIdx.x;
+    const int v = blockIdx.y;
     if (j >= m.nBndCell)
         return;
     const idx i = m.bndCell[j];
     const size_t N = m.N, NB = m.nBnd, NC = m.nBndCell;
-    for (int k = 0; k < m.K; k++)
-    {
-        const int t = m.bndSlot[(size_t)k * NC + j];
-        if (t < 0)
-            continue;
+    real a[M];
 #pragma unroll
-        for (int v = 0; v < NV; v++)
+    for (int r = 0; r < M; r++)
+        a[r] = uRecNew[((size_t)v * M + r) * N + i];
+#pragma unroll
+    for (int k = 0; k < kMaxFC; k++)
+    {
+        const idx t = k < m.K ? m.bndSlot[(size_t)k * NC + j] : idx(-1);
+        if (t >= 0)
 #pragma unroll
             for (int r = 0; r < M; r++)
-                uRecNew[((size_t)v * M + r) * N + i] += scale * bt[((size_t)v * M + r) * NB + t];
+                a[r] += scale * bt[((size_t)v * M + r) * NB + t];
     }
+#pragma unroll
+    for (int r = 0; r < M; r++)
+        uRecNew[((size_t)v * M + r) * N + i] = a[r];
 }
 
 // ---------------------------------------------------------------------------
@@ -458,7 +548,7 @@ __global__ void __launch_bounds__(64) kVRSOR(DevMesh m, const idx *__restrict__ 
             cen[r] = m.cent[(size_t)r * N + i];
         real BCC[M][NV];
         auto rec = [&](int v, int j) { return acc[v][j]; };
-        boundaryFaceBCC<DIM, NDOF, NV, false>(m, f, mom, cen, m.iscale[i], um, rec, rec, BCC);
+        boundaryFaceBCC<DIM, NDOF, NV>(m, f, mom, cen, m.iscale[i], um, rec, BCC);
         real d[NV][M];
 #pragma unroll
         for (int v = 0; v < NV; v++)
@@ -672,17 +762,20 @@ static void vrBoundaryN(Ctx &c, int nVars, const real *uRec, const real *u, cons
     constexpr int M = NDOF - 1;
     if (c.m.nBnd == 0)
         return;
-    const int gf = gridFor(c.m.nBnd, 64), gc = gridFor(c.m.nBndCell, 64);
+    const int G = c.m.G, gf = gridFor(c.m.nBnd, 64), nw = G <= 8 ? G : (G + 1) / 2, bs = 64 * nw;
+    const dim3 gc(gridFor(c.m.nBndCell, 64), nVars);
+    const size_t smem = (size_t)nw * (M + nVars) * 64 * sizeof(real);
+    auto launch = [&](auto face, auto cell) {
+        if (smem > 65536)
+            DNDSR_HIP_CHECK(hipFuncSetAttribute(reinterpret_cast<const void *>(face),
+                                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem));
+        face<<<gf, bs, smem, c.stream>>>(c.m, uRec, u, x, c.vrBnd);
+        cell<<<gc, 64, 0, c.stream>>>(c.m, c.vrBnd, uRecNew, scale);
+    };
     if (nVars == 5)
-    {
-        kVRBndFace<DIM, NDOF, 5, MODE><<<gf, 64, 0, c.stream>>>(c.m, uRec, u, x, c.vrBnd);
-        kVRBndCell<M, 5><<<gc, 64, 0, c.stream>>>(c.m, c.vrBnd, uRecNew, scale);
-    }
+        launch(kVRBndFace<DIM, NDOF, 5, MODE>, kVRBndCell<M, 5>);
     else
-    {
-        kVRBndFace<DIM, NDOF, 1, MODE><<<gf, 64, 0, c.stream>>>(c.m, uRec, u, x, c.vrBnd);
-        kVRBndCell<M, 1><<<gc, 64, 0, c.stream>>>(c.m, c.vrBnd, uRecNew, scale);
-    }
+        launch(kVRBndFace<DIM, NDOF, 1, MODE>, kVRBndCell<M, 1>);
     DNDSR_HIP_CHECK(hipGetLastError());
 }
 static void requireBoundaryValues(const DevMesh &m, int nVars)
