@@ -36,10 +36,9 @@ struct dndsr_ctx
     real *iXLast = nullptr, *iRhsF = nullptr, *iRhs = nullptr, *iDTau = nullptr, *iJd = nullptr, *iInc = nullptr,
          *iTmp = nullptr, *iRes = nullptr;
     float *fRhs = nullptr, *fU = nullptr, *fJd = nullptr, *fLam = nullptr, *fInc = nullptr, *fTmp = nullptr;
-    // cell-major sweep state and per-cell-slot face data of the packed sweeps
-    real *iSlot = nullptr, *iUA = nullptr; // packed sweep: slot data; two [N][16] state + increment arrays
-    float *fSlot = nullptr, *fUA = nullptr;
-    idx *iNbr = nullptr, *fNbr = nullptr; // packed sweep: the neighbours' colour-major positions, [K][N]
+    SGSWork<real> sgs64; // the scalar LU-SGS solve's workspaces (sgs.hip)
+    SGSWork<float> sgs32;
+    real *sgsHalf = nullptr;
     PPStat *iStat = nullptr;   // positivity statistics of the current iteration
     real *iURecSave = nullptr; // uRec at entry, restored when a step fails
     int64_t ppLimited = 0;     // limited cell increments of the last implicit step
@@ -1413,20 +1412,27 @@ static void implicitStep(dndsr_ctx *ctx, const dndsr_euler_settings *es, const d
         launchEvalRHS(c, gp, u, rec, ctx->wDlc, ctx->iRhsF);
         if (roeJ) // the face eigenvalues EvaluateRHS keeps for the Roe Jacobian
             launchFaceRoeLambda(c, gp, u, rec, ctx->wDlc, ctx->bLamRoe);
-        if (kCur)
+        // the unsteady residual: sum_j c_j / dt x_j - u / dt + alphaDiag rhsF, c = 1 for Euler
+        BDFTerms bt{};
+        bt.n = kCur ? kCur : 1;
+        bt.x[0] = xs[0] = ctx->iXLast, coefs[0] = kCur ? kBDFCoef[kCur - 1][1] : 1.0;
+        for (int j = 0; j < kCur - 1; j++)
+            bt.x[1 + j] = xs[1 + j] = xPrevs[j], coefs[1 + j] = kBDFCoef[kCur - 1][2 + j];
+        for (int j = 0; j < bt.n; j++)
+            bt.a[j] = coefs[j] / is->dt;
+        const bool packed = !roeJ && is->gmresCode == 0; // that solve forms its residual and diagonal itself
+        if (!packed)
         {
-            xs[0] = ctx->iXLast, coefs[0] = kBDFCoef[kCur - 1][1];
-            for (int j = 0; j < kCur - 1; j++)
-                xs[1 + j] = xPrevs[j], coefs[1 + j] = kBDFCoef[kCur - 1][2 + j];
-            launchDualResidualBDF(c, is->dt, xs, coefs, kCur, alphaDiag, u, ctx->iRhsF, ctx->iRhs, ctx->iRes);
+            if (kCur)
+                launchDualResidualBDF(c, is->dt, xs, coefs, kCur, alphaDiag, u, ctx->iRhsF, ctx->iRhs, ctx->iRes);
+            else
+                launchDualResidual(c, is->dt, ctx->iXLast, u, ctx->iRhsF, ctx->iRhs, ctx->iRes);
         }
-        else
-            launchDualResidual(c, is->dt, ctx->iXLast, u, ctx->iRhsF, ctx->iRhs, ctx->iRes);
         // fsolve: LUSGSMatrixInit + (1 + sgsIter) symmetric sweeps from a zero increment
         if (roeJ)
             launchLUSGSInitBlock(c, gp, ctx->iDTau, is->dt, alphaDiag, u, ctx->wLam, ctx->bLamRoe, nullptr,
                                  ctx->bJinv, bBad);
-        else
+        else if (!packed)
             launchLUSGSInit(c, ctx->iDTau, is->dt, alphaDiag, ctx->wLam, ctx->iJd);
         if (roeJ)
         {
@@ -1481,28 +1487,16 @@ static void implicitStep(dndsr_ctx *ctx, const dndsr_euler_settings *es, const d
         }
         else if (is->fp32Sweeps)
         {
-            // sweeps with the neighbour state cell-major (the sweep's gathers), FP32
-            const bool fresh = !ctx->fSlot;
-            if (!ctx->fSlot)
-                ctx->fSlot = devAlloc<float>(c, ((size_t)m.K * 5 + 7) * N), ctx->fUA = devAlloc<float>(c, 32 * N),
-                ctx->fNbr = devAlloc<idx>(c, (size_t)m.K * N);
-            launchToF32(c, nU, ctx->iRhs, ctx->fRhs);
-            launchToF32(c, N, ctx->iJd, ctx->fJd);
-            launchToF32(c, F, ctx->wLam, ctx->fLam); // lambdaFace row only
             float *inc = nullptr;
-            launchSGSPacked32(c, gp, (float)alphaDiag, ctx->fRhs, u, ctx->fLam, ctx->fJd, ctx->fUA, ctx->fSlot, ctx->fNbr,
-                              fresh, is->sgsIter, is->gsUpdate, &inc);
+            launchSGSSolve32(c, gp, alphaDiag, bt, is->dt, u, ctx->iRhsF, ctx->iDTau, ctx->wLam, ctx->sgs32,
+                             ctx->sgsHalf, is->sgsIter, is->gsUpdate, ctx->iRes, &inc);
             launchAddIncrementCellMajor(c, gamma, is->incrementRelax, rhoEps, pEps, u, nullptr, inc, ctx->iStat);
         }
         else
         {
-            const bool fresh = !ctx->iSlot;
-            if (!ctx->iSlot)
-                ctx->iSlot = devAlloc<real>(c, ((size_t)m.K * 5 + 7) * N), ctx->iUA = devAlloc<real>(c, 32 * N),
-                ctx->iNbr = devAlloc<idx>(c, (size_t)m.K * N);
             real *inc = nullptr;
-            launchSGSPacked64(c, gp, alphaDiag, ctx->iRhs, u, ctx->wLam, ctx->iJd, ctx->iUA, ctx->iSlot, ctx->iNbr,
-                              fresh, is->sgsIter, is->gsUpdate, &inc);
+            launchSGSSolve64(c, gp, alphaDiag, bt, is->dt, u, ctx->iRhsF, ctx->iDTau, ctx->wLam, ctx->sgs64,
+                             ctx->sgsHalf, is->sgsIter, is->gsUpdate, ctx->iRes, &inc);
             launchAddIncrementCellMajor(c, gamma, is->incrementRelax, rhoEps, pEps, u, inc, nullptr, ctx->iStat);
         }
         // fstop: residual of this iteration relative to its running maximum (density component)

@@ -1853,12 +1853,6 @@ __global__ void __launch_bounds__(256) kDualResidual(idx N, real rdt, const real
 // The BDF unsteady residual (ImplicitBDFDualTimeStep::Step, src/Solver/ODE.hpp:440-451):
 // rhs = sum_j a_j x_j - x / dt + alpha rhsF with a_j = c_j / dt over xLast and up to three
 // earlier states, summed in that order; L1 partial sums as kDualResidual.
-struct BDFTerms
-{
-    const real *x[4];
-    real a[4];
-    int n;
-};
 __global__ void __launch_bounds__(256) kDualResidualBDF(idx N, BDFTerms bt, real rdt, real alpha,
                                                         const real *__restrict__ x, const real *__restrict__ rhsF,
                                                         real *__restrict__ rhs, real *__restrict__ part)
@@ -1935,333 +1929,6 @@ void launchDualResidual(Ctx &c, real dt, const real *xLast, const real *x, const
     DNDSR_HIP_CHECK(hipGetLastError());
     kReduceSum5<<<1, 256, 0, c.stream>>>(c.red, nb, resDev);
     DNDSR_HIP_CHECK(hipGetLastError());
-}
-
-// u += du after the positivity tests of the increment (EvaluateCellRHSAlpha,
-// EulerEvaluator.hxx:1964-2020, with relax = incrementPPRelax) and AddFixedIncrement /
-// ---------------------------------------------------------------------------
-// Packed Gauss-Seidel sweep of the device implicit loop.  Same arithmetic as
-// kSGSColour, other layout: everything the sweep touches is stored in colour-major
-// position order (position p holds cell colorCells[p]), so a colour pass reads and writes
-// one contiguous range whatever the caller's cell order (a locality order for the face
-// and cell kernels need not group cells by colour).  The state the sweep gathers from
-// neighbours (u, uInc, uIncNew) is cell-major, [N][5], so one neighbour costs one or two
-// cache lines instead of ten; the face data a cell needs per slot (signed mean normal,
-// area, lambdaFace) and the neighbour's position are laid out per position and slot,
-// [K][5][N] and [K][N], and the cell's rhs, JDiag and volume per position, all by
-// kSGSSlots once per iteration.  A neighbour precedes in the sweep exactly when its
-// position is lower (the colouring has no neighbours of one colour).
-// ---------------------------------------------------------------------------
-// the mesh-only part of the packed layout (slot normals and areas, neighbour positions, volume):
-// written once per context and precision
-template <typename T>
-__global__ void __launch_bounds__(256) kSGSSlotsStatic(DevMesh m, T *__restrict__ slot, idx *__restrict__ nbr)
-{
-    const idx p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= m.N)
-        return;
-    const size_t N = m.N, F = m.F;
-    const idx i = m.colorCells[p];
-    const T *__restrict__ farea = SGSGeom<T>::area(m);
-    const T *__restrict__ fnorm = SGSGeom<T>::norm(m);
-    for (int k = 0; k < m.K; k++)
-    {
-        const idx f = m.c2f[(size_t)k * N + i];
-        const idx o = m.c2c[(size_t)k * N + i];
-        T q[4] = {0, 0, 0, 0};
-        if (f >= 0)
-        {
-            const T sgn = (m.c2flag[(size_t)k * N + i] & 1) ? T(-1) : T(1);
-#pragma unroll
-            for (int r = 0; r < 3; r++)
-                q[r] = fnorm[r * F + f] * sgn;
-            q[3] = farea[f];
-        }
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-            slot[((size_t)k * 5 + v) * N + p] = q[v];
-        nbr[(size_t)k * N + p] = (f < 0 || o < 0 || o == i) ? idx(-1) : m.cellPos[o];
-    }
-    slot[((size_t)m.K * 5 + 6) * N + p] = SGSGeom<T>::vol(m)[i];
-}
-
-// the per-iteration part: lambdaFace per slot, the cell's rhs and JDiag
-template <typename T>
-__global__ void __launch_bounds__(256) kSGSSlots(DevMesh m, const T *__restrict__ lam, const T *__restrict__ rhs,
-                                                 const T *__restrict__ jd, T *__restrict__ slot)
-{
-    const idx p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= m.N)
-        return;
-    const size_t N = m.N;
-    const idx i = m.colorCells[p];
-    for (int k = 0; k < m.K; k++)
-    {
-        const idx f = m.c2f[(size_t)k * N + i];
-        slot[((size_t)k * 5 + 4) * N + p] = f >= 0 ? lam[f] : T(0);
-    }
-    T *cellRows = slot + (size_t)m.K * 5 * N;
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-        cellRows[(size_t)v * N + p] = rhs[(size_t)v * N + i];
-    cellRows[5 * N + p] = jd[i];
-}
-
-// the packed state: per position a 128-byte row (FP64; 64 bytes FP32) holding the increment
-// (5, at kPackInc) and the state U (5, at kPackU), so that a neighbour costs one cache line;
-// two such arrays, read and written alternately by the sweeps.  Each half of a row is written
-// whole (the increment or the state and three zeros), so no write covers part of a 32-byte
-// sector.
-constexpr int kPackStride = 16, kPackInc = 0, kPackU = 8;
-
-// Skipped colour passes (Gauss-Seidel updates only).  A symmetric sweep after the first
-// begins with the colour the previous sweep ended with; that pass would read the same
-// neighbour increments as the previous one and write the same values, so it is skipped,
-// and the positions [fLo, fHi) of that colour keep their current increments in the array
-// the sweep reads (xr) instead of the one it writes (xw).  The colour the previous sweep
-// skipped is this sweep's last: until its own pass, its current increments are in xw,
-// positions [lLo, lHi).  A neighbour in the first range is read from xr, in the second
-// from xw, any other as usual (xw when already updated in this sweep, else xr).
-struct SweepSkip
-{
-    idx fLo = 0, fHi = 0, lLo = 0, lHi = 0;
-};
-__device__ __forceinline__ bool sgsReadNew(const SweepSkip &sk, idx po, bool useNew)
-{
-    if (po >= sk.fLo && po < sk.fHi)
-        return false;
-    if (po >= sk.lLo && po < sk.lHi)
-        return true;
-    return useNew;
-}
-
-template <typename T>
-__global__ void __launch_bounds__(256) kSGSColourPacked(DevMesh m, real gammaD, T alphaDiag, const T *__restrict__ xr,
-                                                        T *__restrict__ xw, const T *__restrict__ slot,
-                                                        const idx *__restrict__ nbr, int forward, int gsUpdate,
-                                                        int incZero, idx begin, idx end, SweepSkip sk)
-{
-    constexpr int S = kPackStride;
-    const idx p = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= end)
-        return;
-    const size_t N = m.N;
-    const T gamma = (T)gammaD;
-    const T *__restrict__ cellRows = slot + (size_t)m.K * 5 * N;
-    T buf[5];
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-        buf[v] = cellRows[(size_t)v * N + p];
-    const T voli = cellRows[6 * N + p];
-    for (int k = 0; k < m.K; k++)
-    {
-        const idx po = nbr[(size_t)k * N + p];
-        if (po < 0)
-            continue;
-        const bool earlier = forward ? po < p : po > p;
-        const bool useNew = gsUpdate && earlier;
-        if (incZero && !useNew) // the first sweep starts from a zero increment
-            continue;
-        const T *x = (sgsReadNew(sk, po, useNew) ? xw : xr) + (size_t)po * S;
-        T U[5], dU[5], n[3], dF[5];
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            U[v] = x[kPackU + v], dU[v] = x[kPackInc + v];
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-            n[r] = slot[((size_t)k * 5 + r) * N + p];
-        const T area = slot[((size_t)k * 5 + 3) * N + p], lamf = slot[((size_t)k * 5 + 4) * N + p];
-        fluxJacDu<T>(U, n, dU, lamf, gamma, dF);
-        T coef = (T(0.5) * alphaDiag) * area / voli;
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            buf[v] -= coef * dF[v];
-    }
-    const T d = cellRows[5 * N + p];
-#pragma unroll
-    for (int v = 0; v < 8; v++)
-        xw[(size_t)p * S + kPackInc + v] = v < 5 ? buf[v] / d : T(0);
-}
-
-// The same pass with the slot count K fixed at compile time: all K neighbour positions are
-// loaded first and then all K neighbour rows, so a thread waits for two memory round trips
-// instead of two per slot (a colour pass is about one round of waves on the device, so the
-// chain of dependent loads per thread is its run time).  Same arithmetic in the same slot
-// order as kSGSColourPacked: bit-identical results.
-template <typename T, int K>
-constexpr int sgsPackedWaves()
-{
-    return sizeof(T) == 8 ? (K <= 4 ? 4 : 3) : 1; // FP64: the rows of 4 (6) slots in 128 (168) VGPRs
-}
-template <typename T, int K>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(sgsPackedWaves<T, K>())))
-kSGSColourPackedK(DevMesh m, real gammaD, T alphaDiag,
-                                                         const T *__restrict__ xr, T *__restrict__ xw,
-                                                         const T *__restrict__ slot, const idx *__restrict__ nbr,
-                                                         int forward, int gsUpdate, int incZero, idx begin, idx end,
-                                                         SweepSkip sk)
-{
-    constexpr int S = kPackStride;
-    const idx p = begin + blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= end)
-        return;
-    const size_t N = m.N;
-    const T gamma = (T)gammaD;
-    const T *__restrict__ cellRows = slot + (size_t)K * 5 * N;
-    idx po[K];
-#pragma unroll
-    for (int k = 0; k < K; k++)
-        po[k] = nbr[(size_t)k * N + p];
-    // the gathers are unconditional (a slot that is not used reads the cell's own row, a valid
-    // address): a load under a branch makes the compiler wait for every earlier load at the join
-    bool use[K];
-    T U[K][5], dU[K][5];
-#pragma unroll
-    for (int k = 0; k < K; k++)
-    {
-        const bool earlier = forward ? po[k] < p : po[k] > p;
-        const bool useNew = gsUpdate && earlier;
-        use[k] = po[k] >= 0 && !(incZero && !useNew); // the first sweep starts from a zero increment
-        const T *x = use[k] ? (sgsReadNew(sk, po[k], useNew) ? xw : xr) + (size_t)po[k] * S : xr + (size_t)p * S;
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            U[k][v] = x[kPackU + v], dU[k][v] = x[kPackInc + v];
-    }
-    T buf[5];
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-        buf[v] = cellRows[(size_t)v * N + p];
-    const T voli = cellRows[6 * N + p];
-#pragma unroll
-    for (int k = 0; k < K; k++)
-    {
-        if (!use[k])
-            continue;
-        T n[3], dF[5];
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-            n[r] = slot[((size_t)k * 5 + r) * N + p];
-        const T area = slot[((size_t)k * 5 + 3) * N + p], lamf = slot[((size_t)k * 5 + 4) * N + p];
-        fluxJacDu<T>(U[k], n, dU[k], lamf, gamma, dF);
-        T coef = (T(0.5) * alphaDiag) * area / voli;
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            buf[v] -= coef * dF[v];
-    }
-    const T d = cellRows[5 * N + p];
-#pragma unroll
-    for (int v = 0; v < 8; v++)
-        xw[(size_t)p * S + kPackInc + v] = v < 5 ? buf[v] / d : T(0);
-}
-
-// the state into both packed arrays in colour-major position order (the increments need no
-// clearing: the first sweep reads none it has not written, see incZero)
-template <typename T>
-__global__ void __launch_bounds__(256) kToCellMajor(idx N, const idx *__restrict__ cellAt,
-                                                    const real *__restrict__ soa, T *__restrict__ x0,
-                                                    T *__restrict__ x1)
-{
-    constexpr int S = kPackStride;
-    const idx p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= N)
-        return;
-    const idx i = cellAt[p];
-#pragma unroll
-    for (int v = 0; v < 8; v++)
-    {
-        const T a = v < 5 ? (T)soa[(size_t)v * N + i] : T(0);
-        x0[(size_t)p * S + kPackU + v] = a, x1[(size_t)p * S + kPackU + v] = a;
-    }
-}
-
-// the increments of positions [lo, hi) from one packed array into the other
-template <typename T>
-__global__ void __launch_bounds__(256) kCopyIncRows(idx lo, idx hi, const T *__restrict__ from, T *__restrict__ to)
-{
-    constexpr int S = kPackStride;
-    const idx p = lo + blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= hi)
-        return;
-#pragma unroll
-    for (int v = 0; v < 8; v++)
-        to[(size_t)p * S + kPackInc + v] = from[(size_t)p * S + kPackInc + v];
-}
-
-template <typename T>
-void launchSGSPackedT(Ctx &c, const GasParams &gp, T alphaDiag, const T *rhs, const real *u, const T *lam,
-                      const T *jd, T *xbuf, T *slot, idx *nbr, bool fresh, int sgsIter, int gsUpdate, T **result)
-{
-    DevMesh &m = c.m;
-    const int nb = gridFor(m.N, 256);
-    if (fresh)
-        kSGSSlotsStatic<T><<<nb, 256, 0, c.stream>>>(m, slot, nbr);
-    T *x0 = xbuf, *x1 = xbuf + (size_t)kPackStride * m.N;
-    kToCellMajor<T><<<nb, 256, 0, c.stream>>>(m.N, m.colorCells, u, x0, x1);
-    kSGSSlots<T><<<nb, 256, 0, c.stream>>>(m, lam, rhs, jd, slot);
-    DNDSR_HIP_CHECK(hipGetLastError());
-    const int nC = m.nColor;
-    const bool canSkip = gsUpdate && nC >= 2;
-    int prevSkip = -1; // the colour whose pass the previous sweep skipped
-    for (int s = 0; s <= sgsIter; s++)
-        for (int dir = 1; dir >= 0; dir--)
-        {
-            const int first = dir ? 0 : nC - 1, last = dir ? nC - 1 : 0;
-            const bool skipFirst = canSkip && !(s == 0 && dir == 1);
-            SweepSkip sk;
-            if (skipFirst)
-                sk.fLo = m.colorPtrHost[first], sk.fHi = m.colorPtrHost[first + 1];
-            if (prevSkip == last)
-                sk.lLo = m.colorPtrHost[last], sk.lHi = m.colorPtrHost[last + 1];
-            for (int q = skipFirst ? 1 : 0; q < nC; q++)
-            {
-                const int col = dir ? q : nC - 1 - q;
-                const idx b = m.colorPtrHost[col], e = m.colorPtrHost[col + 1];
-                if (e <= b)
-                    continue;
-                KernelTimer kt(c, K_SGS);
-                const int g = gridFor(e - b, 256), z = (s == 0 && dir == 1) ? 1 : 0;
-                if (m.K == 3)
-                    kSGSColourPackedK<T, 3><<<g, 256, 0, c.stream>>>(m, gp.gamma, alphaDiag, x0, x1, slot, nbr, dir,
-                                                                     gsUpdate, z, b, e, sk);
-                else if (m.K == 4)
-                    kSGSColourPackedK<T, 4><<<g, 256, 0, c.stream>>>(m, gp.gamma, alphaDiag, x0, x1, slot, nbr, dir,
-                                                                     gsUpdate, z, b, e, sk);
-                else if (m.K == 6)
-                    kSGSColourPackedK<T, 6><<<g, 256, 0, c.stream>>>(m, gp.gamma, alphaDiag, x0, x1, slot, nbr, dir,
-                                                                     gsUpdate, z, b, e, sk);
-                else
-                    kSGSColourPacked<T><<<g, 256, 0, c.stream>>>(m, gp.gamma, alphaDiag, x0, x1, slot, nbr, dir,
-                                                                 gsUpdate, z, b, e, sk);
-                DNDSR_HIP_CHECK(hipGetLastError());
-            }
-            prevSkip = skipFirst ? first : -1;
-            std::swap(x0, x1);
-        }
-    if (prevSkip >= 0)
-    {
-        // the last sweep skipped its first colour: its increments are still in the array that
-        // sweep read (now x1)
-        const idx b = m.colorPtrHost[prevSkip], e = m.colorPtrHost[prevSkip + 1];
-        if (e > b)
-        {
-            KernelTimer kt(c, K_SGS);
-            kCopyIncRows<T><<<gridFor(e - b, 256), 256, 0, c.stream>>>(b, e, x1, x0);
-            DNDSR_HIP_CHECK(hipGetLastError());
-        }
-    }
-    *result = x0 + kPackInc; // the last increment, stride kPackStride
-}
-void launchSGSPacked64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, const real *u, const real *lam,
-                       const real *jd, real *xbuf, real *slot, idx *nbr, bool fresh, int sgsIter, int gsUpdate,
-                       real **result)
-{
-    launchSGSPackedT<real>(c, gp, alphaDiag, rhs, u, lam, jd, xbuf, slot, nbr, fresh, sgsIter, gsUpdate, result);
-}
-void launchSGSPacked32(Ctx &c, const GasParams &gp, float alphaDiag, const float *rhs, const real *u,
-                       const float *lam, const float *jd, float *xbuf, float *slot, idx *nbr, bool fresh, int sgsIter,
-                       int gsUpdate, float **result)
-{
-    launchSGSPackedT<float>(c, gp, alphaDiag, rhs, u, lam, jd, xbuf, slot, nbr, fresh, sgsIter, gsUpdate, result);
 }
 
 // ---------------------------------------------------------------------------
@@ -2462,8 +2129,8 @@ __device__ void ppCompressInc(const real *u, real *ret, real gamma, real rhoEps,
     }
 }
 
-// CELLMAJOR: du is the packed sweep's increment, rows of kPackStride in colour-major position
-// order (pos = the cell's position)
+// CELLMAJOR: du is the LU-SGS solve's increment (sgs.hip), rows of 8 in colour-major position order
+// (pos = the cell's position)
 template <typename T, bool CELLMAJOR = false>
 __global__ void __launch_bounds__(256) kAddIncrement(idx N, real gamma, real relax, real rhoEps, real pEps,
                                                      real *__restrict__ u, const T *__restrict__ du,
@@ -2476,7 +2143,7 @@ __global__ void __launch_bounds__(256) kAddIncrement(idx N, real gamma, real rel
     const size_t pi = CELLMAJOR ? (size_t)pos[i] : (size_t)i;
 #pragma unroll
     for (int v = 0; v < 5; v++)
-        U[v] = u[(size_t)v * N + i], D[v] = (real)du[CELLMAJOR ? pi * kPackStride + v : (size_t)v * N + i];
+        U[v] = u[(size_t)v * N + i], D[v] = (real)du[CELLMAJOR ? pi * 8 + v : (size_t)v * N + i];
     bool limited = false, bad = false;
     const real a = ppCellAlpha(U, D, gamma, relax, rhoEps, pEps, limited, bad);
 #pragma unroll

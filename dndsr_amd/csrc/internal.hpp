@@ -295,21 +295,32 @@ void launchAddIncrement64(Ctx &c, real gamma, real relax, real rhoEps, real pEps
 void launchAddIncrement32(Ctx &c, real gamma, real relax, real rhoEps, real pEps, real *u, const float *du,
                           PPStat *stat);
 void launchToF32(Ctx &c, size_t n, const real *in, float *out);
-// (1 + sgsIter) forward/backward multicolour sweeps from a zero increment with the state
-// gathered from neighbours stored cell-major: uA <- u as [N][5], slot <- per-cell-slot face
-// data; inc / tmp are [N][5] scratch; *result points at the buffer holding the increment.
-// xbuf: [2][N][16] (two packed arrays of state + increment rows); slot: [(K*5 + 7) N] (per-slot
-// face data, then rhs, JDiag and volume in colour-major position order); nbr: [K N]; fresh: slot
-// and nbr are new (their mesh-only part is written); *result: the increment, rows of 16 in
-// colour-major position order
-void launchSGSPacked64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, const real *u, const real *lam,
-                       const real *jd, real *xbuf, real *slot, idx *nbr, bool fresh, int sgsIter, int gsUpdate,
-                       real **result);
-void launchSGSPacked32(Ctx &c, const GasParams &gp, float alphaDiag, const float *rhs, const real *u,
-                       const float *lam, const float *jd, float *xbuf, float *slot, idx *nbr, bool fresh, int sgsIter,
-                       int gsUpdate, float **result);
-// u += du with du cell-major ([N][5], FP64 or FP32: exactly one of du64 / du32 non-null)
-// du: the packed sweep's increment (rows of 16 in colour-major position order)
+// the sum of a dual-time residual: sum_j a_j x_j over xLast and up to three earlier states
+struct BDFTerms
+{
+    const real *x[4];
+    real a[4];
+    int n;
+};
+// the implicit loop's LU-SGS solve (sgs.hip): workspace per precision, allocated at its first use
+template <typename T>
+struct SGSWork
+{
+    T *x[2] = {nullptr, nullptr}; // increments [N][8] in colour-major position order (the second: Jacobi)
+    T *rec = nullptr, *nq = nullptr, *st = nullptr;
+    idx *nbr = nullptr;
+};
+// rhs = bt - u / dt + alpha rhsF with its L1 norm into resDev, LUSGSMatrixInit's scalar diagonal, and
+// (1 + sgsIter) forward/backward sweeps from a zero increment; *result: the increment, rows of 8 in
+// colour-major position order.  half: [K][N] mesh constants shared by the precisions
+void launchSGSSolve64(Ctx &c, const GasParams &gp, real alpha, const BDFTerms &bt, real dt, const real *u,
+                      const real *rhsF, const real *dTau, const real *lam, SGSWork<real> &w, real *&half, int sgsIter,
+                      int gsUpdate, real *resDev, real **result);
+void launchSGSSolve32(Ctx &c, const GasParams &gp, real alpha, const BDFTerms &bt, real dt, const real *u,
+                      const real *rhsF, const real *dTau, const real *lam, SGSWork<float> &w, real *&half,
+                      int sgsIter, int gsUpdate, real *resDev, float **result);
+// u += du with du the LU-SGS solve's increment, rows of 8 in colour-major position order (exactly one
+// of du64 / du32 non-null)
 void launchAddIncrementCellMajor(Ctx &c, real gamma, real relax, real rhoEps, real pEps, real *u, const real *du64,
                                  const float *du32, PPStat *stat);
 // ---- launchers (model.hip): ModelEvaluator::EvaluateRHS, scalar advection-diffusion (2-D)

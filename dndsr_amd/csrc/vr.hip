@@ -386,7 +386,7 @@ __global__ void __launch_bounds__(512) kVRBndFace(DevMesh m, const real *__restr
         };
         auto finish = [&](int v) {
             if (valid)
-#pragma unroll
+#pragma unroll(M <= 5 ? M : 1) // all rows of a large block in flight would spill
                 for (int r = 0; r < M; r++)
                 {
                     real acc = 0;
