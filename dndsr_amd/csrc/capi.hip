@@ -723,6 +723,7 @@ int dndsr_set_vr_coeffs(dndsr_ctx *ctx, const double *AinvB, const double *Ainvb
     }
     upload(c, m.AinvB, B);
     upload(c, m.Ainvb, b);
+    c.sorFresh = false; // the copy in the order of the SOR lists is rebuilt
     DNDSR_HIP_CHECK(hipStreamSynchronize(c.stream));
     CAPI_END
 }

@@ -123,6 +123,11 @@ struct Ctx
     // scratch owned by the context (grown on demand, freed at destroy)
     real *faceFlux = nullptr;   // [5][F]
     real *vrBnd = nullptr;      // [nVars][M][nBnd] A^-1 BCC of each boundary face (VR sweep boundary term)
+    // the SOR sweep's matrices in list order (vr.hip, sorMatrix): sweeps so far (up to 2), the copy,
+    // whether it matches the coefficients, and whether there was no memory for it
+    int sorUse = 0;
+    real *sorB = nullptr;
+    bool sorFresh = false, sorNoRoom = false;
     size_t faceFluxCap = 0;
     real *red = nullptr;        // reduction partials
     size_t redCap = 0;

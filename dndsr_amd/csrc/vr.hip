@@ -33,12 +33,21 @@ struct VRRows
 
 // KIND: 0 = Jacobi iteration (mode 0), 3 = recordInc (mode 1), 1 = recordInc with
 // uRecIsZero (mode 2), 2 = IterDiff.  The staged mean rows hold u_j - u_i.
+// KIND 4 = the SOR sweep's cells without a boundary face, one colour per launch: the Jacobi
+// formula on the cells list.cells[0 .. n), updated in place (uRecNew = uRec: a colour's cells are
+// no one's neighbours within its launch), with the matrix rows of list position t or of cell i.
+struct CellList
+{
+    const idx *cells = nullptr;
+    idx n = 0;
+    const real *B = nullptr, *b = nullptr; // A^-1 B_f and A^-1 b_f of the list's cells ([K M M][N], [K M][N])
+    bool byPos = false;                    // their entity index: the list position, or the cell
+};
 template <int M, int NV, int KIND>
 __global__ void __launch_bounds__(kTileC *VRRows<M>::RW) __attribute__((amdgpu_waves_per_eu(5)))
-kVRIter(DevMesh m, const real *__restrict__ uRec, real *__restrict__ uRecNew, const real *__restrict__ u, int mode,
-        real relax)
+kVRIter(DevMesh m, const real *uRec, real *uRecNew, const real *__restrict__ u, int mode, real relax, CellList list)
 {
-    constexpr bool DIFF = KIND == 2, REC = KIND != 1, RELAX = KIND == 0;
+    constexpr bool DIFF = KIND == 2, REC = KIND != 1, SOR = KIND == 4, RELAX = KIND == 0 || SOR;
     constexpr int RW = VRRows<M>::RW, RPT = VRRows<M>::RPT;
     constexpr int NROW = (REC ? NV * M : 0) + (DIFF ? 0 : NV); // staged neighbour rows
     constexpr int R0 = REC ? NV * M : 0;                       // first mean row
@@ -48,9 +57,11 @@ kVRIter(DevMesh m, const real *__restrict__ uRec, real *__restrict__ uRecNew, co
     const int tile = xcdTile(blockIdx.x, gridDim.x);
     const size_t N = m.N;
     const int K = m.K;
-    const idx i = tile * kTileC + lane;
-    const bool valid = i < m.N;
+    const idx t0 = tile * kTileC + lane;
+    const bool valid = t0 < (SOR ? list.n : m.N);
+    const idx i = SOR ? list.cells[valid ? t0 : list.n - 1] : t0;
     const uint32_t ioff = (uint32_t)i * 8u; // reads past the row (tail lanes) return 0
+    const uint32_t boff = SOR && list.byPos ? (valid ? (uint32_t)t0 * 8u : kNoRow) : ioff;
     const uint64_t rowB = (uint64_t)N * 8;
     auto row = [&](const real *base) { return rowRsrc(base, rowB); };
     real acc[RPT][NV];
@@ -93,8 +104,8 @@ kVRIter(DevMesh m, const real *__restrict__ uRec, real *__restrict__ uRecNew, co
     // matrix rows of slot k (AinvB / Ainvb hold K slots for every cell), streamed once
     // with the non-temporal hint so that they do not evict the neighbours' rows from L2
     auto loadB = [&](int k, real (*br)[M], real *bb) {
-        const real *B = m.AinvB + ((size_t)(1 + k) * M * M) * N;
-        const real *bv = m.Ainvb + ((size_t)k * M) * N;
+        const real *B = SOR ? list.B + ((size_t)k * M * M) * N : m.AinvB + ((size_t)(1 + k) * M * M) * N;
+        const real *bv = (SOR ? list.b : m.Ainvb) + ((size_t)k * M) * N;
 #pragma unroll
         for (int t = 0; t < RPT; t++)
         {
@@ -102,8 +113,8 @@ kVRIter(DevMesh m, const real *__restrict__ uRec, real *__restrict__ uRecNew, co
             if constexpr (REC)
 #pragma unroll
                 for (int q = 0; q < M; q++)
-                    br[t][q] = bldnt(row(B + ((size_t)r * M + q) * N), ioff);
-            bb[t] = DIFF ? 0.0 : bldnt(row(bv + (size_t)r * N), ioff);
+                    br[t][q] = bldnt(row(B + ((size_t)r * M + q) * N), boff);
+            bb[t] = DIFF ? 0.0 : bldnt(row(bv + (size_t)r * N), boff);
         }
     };
     auto nbIndex = [&](int k) -> idx {
@@ -186,13 +197,14 @@ kVRIter(DevMesh m, const real *__restrict__ uRec, real *__restrict__ uRecNew, co
 }
 
 template <int M, int KIND>
-static void vrLaunch(Ctx &c, int nVars, const real *uRec, real *uRecNew, const real *u, int mode, real relax)
+static void vrLaunch(Ctx &c, int nVars, const real *uRec, real *uRecNew, const real *u, int mode, real relax,
+                     const CellList &list = CellList{})
 {
-    int g = gridFor(c.m.N, kTileC), bs = kTileC * VRRows<M>::RW;
+    int g = gridFor(KIND == 4 ? list.n : c.m.N, kTileC), bs = kTileC * VRRows<M>::RW;
     if (nVars == 5)
-        kVRIter<M, 5, KIND><<<g, bs, 0, c.stream>>>(c.m, uRec, uRecNew, u, mode, relax);
+        kVRIter<M, 5, KIND><<<g, bs, 0, c.stream>>>(c.m, uRec, uRecNew, u, mode, relax, list);
     else if (nVars == 1)
-        kVRIter<M, 1, KIND><<<g, bs, 0, c.stream>>>(c.m, uRec, uRecNew, u, mode, relax);
+        kVRIter<M, 1, KIND><<<g, bs, 0, c.stream>>>(c.m, uRec, uRecNew, u, mode, relax, list);
     else
         throw std::runtime_error("nVars must be 1 or 5");
     DNDSR_HIP_CHECK(hipGetLastError());
@@ -386,7 +398,7 @@ __global__ void __launch_bounds__(512) kVRBndFace(DevMesh m, const real *__restr
         };
         auto finish = [&](int v) {
             if (valid)
-#pragma unroll(M <= 5 ? M : 1) // all rows of a large block in flight would spill
+#pragma unroll M <= 5 ? M : 1 // all rows of a large block in flight would spill
                 for (int r = 0; r < M; r++)
                 {
                     real acc = 0;
@@ -468,16 +480,20 @@ __global__ void __launch_bounds__(64) kVRBndCell(DevMesh m, const real *__restri
 
 // ---------------------------------------------------------------------------
 // SOR form of the sweep (SORInstead = true, recordInc = false,
-// VariationalReconstruction_Reconstruction.hxx:534-589), multicolour: one launch per
-// colour, one thread per cell of the colour, the cell's block kept in registers and
-// updated in place.  Cells of one colour share no face, so a colour's neighbours are
-// not written during its launch and the sweep equals the serial SOR in colour order.
+// VariationalReconstruction_Reconstruction.hxx:534-589), multicolour and in place.  Cells of one
+// colour share no face, so a colour's neighbours are not written during its launches and the sweep
+// equals the serial SOR in colour order.
 // Per cell: uRec_i *= (1 - relax); per face in cell-face order
 //   interior: uRec_i += relax (A^-1 B_f uRec_j + A^-1 b_f (u_j - u_i))
 //   boundary: uRec_i += relax A^-1 BCC(uRec_i as accumulated so far), as the reference
 //             hands GetBoundaryRHS the array being updated (:584).
+// Per colour the cells without a boundary face go through the tile kernel (kVRIter, KIND 4), which
+// streams each matrix row once in coalesced lines; the cells with one, whose boundary term depends
+// on the block accumulated so far, take one thread each (kVRSOR).  A colour is every other cell or
+// fewer, so in the caller's order each colour would fetch whole lines of A^-1 B for a part of their
+// cells: from its second sweep on a context keeps a copy of the matrices in list order (sorMatrix).
 // ---------------------------------------------------------------------------
-template <int DIM, int NDOF, int NV, bool BND>
+template <int DIM, int NDOF, int NV>
 __global__ void __launch_bounds__(64) kVRSOR(DevMesh m, const idx *__restrict__ cells, idx nCells,
                                              real *__restrict__ uRec, const real *__restrict__ u, real relax)
 {
@@ -537,8 +553,6 @@ __global__ void __launch_bounds__(64) kVRSOR(DevMesh m, const idx *__restrict__ 
             }
             continue;
         }
-        if constexpr (!BND) // the cell lists without a boundary face
-            continue;
         real mom[M], cen[3];
 #pragma unroll
         for (int j = 0; j < M; j++)
@@ -840,33 +854,80 @@ void launchVRIter(Ctx &c, int nVars, const real *uRec, real *uRecNew, const real
         vrBoundary<1>(c, nVars, uRec, u, nullptr, uRecNew, -1.0);
 }
 
+// rows [0, n) of src in list order: dst[q][t] = src[q][cells[t]]
+__global__ void __launch_bounds__(256) kPermuteRows(size_t N, int n, const idx *__restrict__ cells,
+                                                    const real *__restrict__ src, real *__restrict__ dst)
+{
+    const size_t t = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (t >= N)
+        return;
+    const idx i = cells[t];
+    for (int q = blockIdx.y; q < n; q += gridDim.y)
+        dst[(size_t)q * N + t] = src[(size_t)q * N + i];
+}
+
+// The matrices the SOR sweep streams.  The first sweep of a context reads them in the caller's cell
+// order; a context that sweeps again gets a copy in the order of the SOR lists, which it keeps (and
+// refreshes when the coefficients are replaced).  No copy while the stream is being captured (it would
+// allocate) or where the memory for it is not there.
+static CellList sorMatrix(Ctx &c)
+{
+    const DevMesh &m = c.m;
+    const size_t N = m.N, nB = (size_t)m.K * m.M * m.M, nb = (size_t)m.K * m.M;
+    CellList l;
+    l.B = m.AinvB + (size_t)m.M * m.M * N, l.b = m.Ainvb;
+    if (m.nColor < 2 || (c.sorUse < 2 && ++c.sorUse < 2))
+        return l;
+    if (!c.sorFresh)
+    {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        DNDSR_HIP_CHECK(hipStreamIsCapturing(c.stream, &cap));
+        if (cap != hipStreamCaptureStatusNone || c.sorNoRoom)
+            return l;
+        if (!c.sorB)
+        {
+            void *p = nullptr;
+            if (hipMalloc(&p, (nB + nb) * N * sizeof(real)) != hipSuccess)
+            {
+                (void)hipGetLastError();
+                c.sorNoRoom = true;
+                return l;
+            }
+            c.owned.push_back(p);
+            c.sorB = static_cast<real *>(p);
+        }
+        const dim3 g(gridFor(m.N, 256), 8);
+        kPermuteRows<<<g, 256, 0, c.stream>>>(N, (int)nB, m.sorCells, m.AinvB + (size_t)m.M * m.M * N, c.sorB);
+        kPermuteRows<<<g, 256, 0, c.stream>>>(N, (int)nb, m.sorCells, m.Ainvb, c.sorB + nB * N);
+        DNDSR_HIP_CHECK(hipGetLastError());
+        c.sorFresh = true;
+    }
+    l.B = c.sorB, l.b = c.sorB + nB * N, l.byPos = true;
+    return l;
+}
+
 template <int DIM, int NDOF>
 static void vrSORN(Ctx &c, int nVars, real *uRec, const real *u, real relax)
 {
     const DevMesh &m = c.m;
-    // per colour two launches: the cells without a boundary face (no boundary branch, fewer
-    // registers), then those with one; cells of one colour are independent
+    CellList l = sorMatrix(c);
+    const real *B = l.B, *b0 = l.b;
     for (int col = 0; col < m.nColor; col++)
     {
         const idx b = m.colorPtrHost[col], s = m.sorSplitHost[col], e = m.colorPtrHost[col + 1];
         if (s > b)
         {
-            if (nVars == 5)
-                kVRSOR<DIM, NDOF, 5, false><<<gridFor(s - b, 64), 64, 0, c.stream>>>(m, m.sorCells + b, s - b, uRec, u,
-                                                                                     relax);
-            else
-                kVRSOR<DIM, NDOF, 1, false><<<gridFor(s - b, 64), 64, 0, c.stream>>>(m, m.sorCells + b, s - b, uRec, u,
-                                                                                     relax);
-            DNDSR_HIP_CHECK(hipGetLastError());
+            l.cells = m.sorCells + b, l.n = s - b;
+            if (l.byPos) // list position 0 is the colour's first cell
+                l.B = B + b, l.b = b0 + b;
+            vrLaunch<NDOF - 1, 4>(c, nVars, uRec, uRec, u, 4, relax, l);
         }
         if (e > s)
         {
             if (nVars == 5)
-                kVRSOR<DIM, NDOF, 5, true><<<gridFor(e - s, 64), 64, 0, c.stream>>>(m, m.sorCells + s, e - s, uRec, u,
-                                                                                    relax);
+                kVRSOR<DIM, NDOF, 5><<<gridFor(e - s, 64), 64, 0, c.stream>>>(m, m.sorCells + s, e - s, uRec, u, relax);
             else
-                kVRSOR<DIM, NDOF, 1, true><<<gridFor(e - s, 64), 64, 0, c.stream>>>(m, m.sorCells + s, e - s, uRec, u,
-                                                                                    relax);
+                kVRSOR<DIM, NDOF, 1><<<gridFor(e - s, 64), 64, 0, c.stream>>>(m, m.sorCells + s, e - s, uRec, u, relax);
             DNDSR_HIP_CHECK(hipGetLastError());
         }
     }
