@@ -34,8 +34,8 @@ struct dndsr_ctx
     bool haveWork = false;
     // implicit dual-time workspace
     real *iXLast = nullptr, *iRhsF = nullptr, *iRhs = nullptr, *iDTau = nullptr, *iJd = nullptr, *iInc = nullptr,
-         *iTmp = nullptr, *iRes = nullptr;
-    float *fRhs = nullptr, *fU = nullptr, *fJd = nullptr, *fLam = nullptr, *fInc = nullptr, *fTmp = nullptr;
+         *iRes = nullptr;
+    float *fU = nullptr, *fJd = nullptr, *fLam = nullptr; // FP32 copies for the GMRES preconditioner
     SGSWork<real> sgs64; // the scalar LU-SGS solve's workspaces (sgs.hip)
     SGSWork<float> sgs32;
     real *sgsHalf = nullptr;
@@ -44,10 +44,11 @@ struct dndsr_ctx
     int64_t ppLimited = 0;     // limited cell increments of the last implicit step
     double ppAlphaMin = 1.0;   // and their smallest alpha
     bool haveImplicit = false;
-    // Roe-Jacobian block LU-SGS workspace: face eigenvalues [3][F], inverse blocks [25][N]
-    // (FP64 and FP32), the singular-block flag
-    real *bLamRoe = nullptr, *bJinv = nullptr;
-    float *bJinvF = nullptr, *bLamRoeF = nullptr;
+    // Roe-Jacobian block LU-SGS workspace: face eigenvalues [3][F], the solves' workspaces
+    // (roejac.hip), the singular-block flag
+    real *bLamRoe = nullptr;
+    SGSBlockWork<real> blk64;
+    SGSBlockWork<float> blk32;
     int *bBad = nullptr;
     // linear-solver workspace (GMRES Krylov basis for up to linK vectors + temporaries)
     LinWork lin;
@@ -102,6 +103,18 @@ static LinWork &linWork(dndsr_ctx *ctx, int k, bool fp32)
         ctx->linF32 = true;
     }
     return w;
+}
+
+// FP32 copies of the state, diagonal and face eigenvalues for an FP32 preconditioner
+static void fp32State(dndsr_ctx *ctx)
+{
+    Ctx &c = ctx->c;
+    if (!ctx->fU)
+        ctx->fU = devAlloc<float>(c, 5 * (size_t)c.m.N);
+    if (!ctx->fJd)
+        ctx->fJd = devAlloc<float>(c, c.m.N);
+    if (!ctx->fLam)
+        ctx->fLam = devAlloc<float>(c, 4 * (size_t)c.m.F);
 }
 
 static thread_local std::string g_err;
@@ -1347,16 +1360,8 @@ static void implicitStep(dndsr_ctx *ctx, const dndsr_euler_settings *es, const d
     const size_t N = m.N, F = m.F;
     const size_t nU = 5 * N, nR = 5 * (size_t)m.M * N;
     timeLoopWork(ctx);
-    if (roeJ && !ctx->bJinv)
-    {
+    if (roeJ && !ctx->bLamRoe)
         ctx->bLamRoe = devAlloc<real>(c, 3 * F);
-        ctx->bJinv = devAlloc<real>(c, 25 * N);
-    }
-    if (roeJ && is->fp32Sweeps && !ctx->bJinvF)
-    {
-        ctx->bJinvF = devAlloc<float>(c, 25 * N);
-        ctx->bLamRoeF = devAlloc<float>(c, 3 * F);
-    }
     int *bBad = roeJ ? blockFlag(ctx) : nullptr;
     if (!ctx->haveImplicit)
     {
@@ -1366,17 +1371,7 @@ static void implicitStep(dndsr_ctx *ctx, const dndsr_euler_settings *es, const d
         ctx->iDTau = devAlloc<real>(c, N);
         ctx->iJd = devAlloc<real>(c, N);
         ctx->iInc = devAlloc<real>(c, nU);
-        ctx->iTmp = devAlloc<real>(c, nU);
         ctx->iRes = devAlloc<real>(c, 8);
-        ctx->fRhs = devAlloc<float>(c, nU);
-        if (!ctx->fU)
-            ctx->fU = devAlloc<float>(c, nU);
-        if (!ctx->fJd)
-            ctx->fJd = devAlloc<float>(c, N);
-        if (!ctx->fLam)
-            ctx->fLam = devAlloc<float>(c, 4 * F);
-        ctx->fInc = devAlloc<float>(c, nU);
-        ctx->fTmp = devAlloc<float>(c, nU);
         ctx->iStat = devAlloc<PPStat>(c, 1);
         ctx->iURecSave = devAlloc<real>(c, nR);
         ctx->haveImplicit = true;
@@ -1430,40 +1425,19 @@ static void implicitStep(dndsr_ctx *ctx, const dndsr_euler_settings *es, const d
                 launchDualResidual(c, is->dt, ctx->iXLast, u, ctx->iRhsF, ctx->iRhs, ctx->iRes);
         }
         // fsolve: LUSGSMatrixInit + (1 + sgsIter) symmetric sweeps from a zero increment
-        if (roeJ)
-            launchLUSGSInitBlock(c, gp, ctx->iDTau, is->dt, alphaDiag, u, ctx->wLam, ctx->bLamRoe, nullptr,
-                                 ctx->bJinv, bBad);
-        else if (!packed)
+        if (!roeJ && !packed)
             launchLUSGSInit(c, ctx->iDTau, is->dt, alphaDiag, ctx->wLam, ctx->iJd);
         if (roeJ)
         {
-            // block sweeps in colour order, ping-ponging the increment from zero
-            real *sumDev = c.red + 5 * ((size_t)gridFor(m.N, 256) + m.nColor + 6);
+            real *inc64 = nullptr;
+            float *inc32 = nullptr;
             if (is->fp32Sweeps)
-            {
-                launchToF32(c, nU, ctx->iRhs, ctx->fRhs);
-                launchToF32(c, nU, u, ctx->fU);
-                launchToF32(c, 25 * N, ctx->bJinv, ctx->bJinvF);
-                launchToF32(c, 4 * F, ctx->wLam, ctx->fLam);
-                launchToF32(c, 3 * F, ctx->bLamRoe, ctx->bLamRoeF);
-                float *a = ctx->fInc, *b = ctx->fTmp;
-                DNDSR_HIP_CHECK(hipMemsetAsync(a, 0, nU * sizeof(float), c.stream));
-                DNDSR_HIP_CHECK(hipMemsetAsync(b, 0, nU * sizeof(float), c.stream));
-                float *res = nullptr;
-                launchSGSBlockSymmetric32(c, gp, (float)alphaDiag, ctx->fRhs, ctx->fU, a, b, ctx->bJinvF, ctx->fLam,
-                                          ctx->bLamRoeF, is->sgsIter, is->gsUpdate, sumDev, &res);
-                launchAddIncrement32(c, gamma, is->incrementRelax, rhoEps, pEps, u, res, ctx->iStat);
-            }
+                launchSGSBlockSolve32(c, gp, alphaDiag, ctx->iRhs, is->dt, u, ctx->iDTau, ctx->wLam, ctx->bLamRoe,
+                                      ctx->blk32, is->sgsIter, is->gsUpdate, bBad, &inc32);
             else
-            {
-                real *a = ctx->iInc, *b = ctx->iTmp;
-                DNDSR_HIP_CHECK(hipMemsetAsync(a, 0, nU * sizeof(real), c.stream));
-                DNDSR_HIP_CHECK(hipMemsetAsync(b, 0, nU * sizeof(real), c.stream));
-                real *res = nullptr;
-                launchSGSBlockSymmetric64(c, gp, alphaDiag, ctx->iRhs, u, a, b, ctx->bJinv, ctx->wLam, ctx->bLamRoe,
-                                          is->sgsIter, is->gsUpdate, sumDev, &res);
-                launchAddIncrement64(c, gamma, is->incrementRelax, rhoEps, pEps, u, res, ctx->iStat);
-            }
+                launchSGSBlockSolve64(c, gp, alphaDiag, ctx->iRhs, is->dt, u, ctx->iDTau, ctx->wLam, ctx->bLamRoe,
+                                      ctx->blk64, is->sgsIter, is->gsUpdate, bBad, &inc64);
+            launchAddIncrementCellMajor(c, gamma, is->incrementRelax, rhoEps, pEps, u, inc64, inc32, ctx->iStat);
         }
         else if (is->gmresCode != 0)
         {
@@ -1474,6 +1448,7 @@ static void implicitStep(dndsr_ctx *ctx, const dndsr_euler_settings *es, const d
             w.sgsIter = is->sgsIter, w.gsUpdate = is->gsUpdate, w.fp32 = is->fp32Sweeps != 0;
             if (w.fp32)
             {
+                fp32State(ctx);
                 launchToF32(c, nU, u, ctx->fU);
                 launchToF32(c, N, ctx->iJd, ctx->fJd);
                 launchToF32(c, F, ctx->wLam, ctx->fLam);
@@ -1592,12 +1567,7 @@ int dndsr_gmres_lusgs(dndsr_ctx *ctx, const dndsr_euler_settings *es, double alp
     w.sgsIter = sgsIter, w.gsUpdate = gsUpdate, w.fp32 = fp32Precond != 0;
     if (w.fp32)
     {
-        if (!ctx->fU)
-            ctx->fU = devAlloc<float>(c, nU);
-        if (!ctx->fJd)
-            ctx->fJd = devAlloc<float>(c, N);
-        if (!ctx->fLam)
-            ctx->fLam = devAlloc<float>(c, 4 * F);
+        fp32State(ctx);
         launchToF32(c, nU, u, ctx->fU);
         launchToF32(c, N, jdiag, ctx->fJd);
         launchToF32(c, F, lambdaFace, ctx->fLam);

@@ -2198,14 +2198,6 @@ void launchAddIncrementCellMajor(Ctx &c, real gamma, real relax, real rhoEps, re
                                                                               du32, stat, c.m.cellPos);
     DNDSR_HIP_CHECK(hipGetLastError());
 }
-void launchAddIncrement32(Ctx &c, real gamma, real relax, real rhoEps, real pEps, real *u, const float *du,
-                          PPStat *stat)
-{
-    KernelTimer kt(c, K_INCREMENT);
-    kAddIncrement<float><<<gridFor(c.m.N, 256), 256, 0, c.stream>>>(c.m.N, gamma, relax, rhoEps, pEps, u, du, stat);
-    DNDSR_HIP_CHECK(hipGetLastError());
-}
-
 __global__ void __launch_bounds__(256) kToF32(size_t n, const real *__restrict__ in, float *__restrict__ out)
 {
     const size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;

@@ -253,12 +253,20 @@ void launchSGSSweep32(Ctx &c, const GasParams &gp, float alphaDiag, const float 
 void launchFaceRoeLambda(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *lamRoe);
 void launchLUSGSInitBlock(Ctx &c, const GasParams &gp, const real *dTau, real dt, real alphaDiag, const real *u,
                           const real *lam, const real *lamRoe, real *jd, real *jinv, int *bad);
-void launchSGSBlockSymmetric64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, const real *u, real *a,
-                               real *b, const real *jinv, const real *lam, const real *lamRoe, int sgsIter,
-                               int gsUpdate, real *sumIncDev, real **result);
-void launchSGSBlockSymmetric32(Ctx &c, const GasParams &gp, float alphaDiag, const float *rhs, const float *u,
-                               float *a, float *b, const float *jinv, const float *lam, const float *lamRoe,
-                               int sgsIter, int gsUpdate, real *sumIncDev, float **result);
+// the implicit loop's block solve (roejac.hip): workspace per precision, allocated at its first use;
+// *result: the increment, rows of 8 in colour-major position order; bad set when a block is singular
+template <typename T>
+struct SGSBlockWork
+{
+    T *x[2] = {nullptr, nullptr}, *C = nullptr, *b = nullptr;
+    idx *nbr = nullptr;
+};
+void launchSGSBlockSolve64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, real dt, const real *u,
+                           const real *dTau, const real *lam, const real *lamRoe, SGSBlockWork<real> &w, int sgsIter,
+                           int gsUpdate, int *bad, real **result);
+void launchSGSBlockSolve32(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, real dt, const real *u,
+                           const real *dTau, const real *lam, const real *lamRoe, SGSBlockWork<float> &w, int sgsIter,
+                           int gsUpdate, int *bad, float **result);
 void launchSGSSweepBlock64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, const real *u,
                            const real *uInc, real *uIncNew, const real *jinv, const real *lam, const real *lamRoe,
                            int forward, int gsUpdate, int uIncIsZero, real *sumIncDev);
@@ -296,8 +304,6 @@ struct PPStat
 void launchPPStatReset(Ctx &c, PPStat *stat);
 // fincrement: u += CompressInc(u, alpha du) with alpha from EvaluateCellRHSAlpha, per cell
 void launchAddIncrement64(Ctx &c, real gamma, real relax, real rhoEps, real pEps, real *u, const real *du,
-                          PPStat *stat);
-void launchAddIncrement32(Ctx &c, real gamma, real relax, real rhoEps, real pEps, real *u, const float *du,
                           PPStat *stat);
 void launchToF32(Ctx &c, size_t n, const real *in, float *out);
 // the sum of a dual-time residual: sum_j a_j x_j over xLast and up to three earlier states

@@ -244,8 +244,10 @@ __device__ inline void faceLambdas(const T *lam, const T *lamRoe, size_t F, idx 
 
 // JacobianDiagBlock::GetInvert (EulerJacobian.hpp:153-190): J^-1 = (D^-1 J)^-1 D^-1 with the
 // scaled block inverted by Gauss-Jordan elimination with complete pivoting.  Returns false for a
-// zero diagonal or a singular block.
-__device__ inline bool invertBlock5(const real *J, real *Jinv)
+// zero diagonal or a singular block.  Every index is a compile-time constant (the row and column
+// exchanges are selects over the candidates), so both blocks stay in registers: indexed by the pivot
+// they lived in scratch memory, which bound the kernels that call this.
+__device__ inline bool invertBlock5(const real (&J)[25], real (&Jinv)[25])
 {
     real P[5][5], X[5][5], dinv[5];
     int cp[5] = {0, 1, 2, 3, 4};
@@ -261,46 +263,69 @@ __device__ inline bool invertBlock5(const real *J, real *Jinv)
 #pragma unroll
         for (int j = 0; j < 5; j++)
             P[i][j] = dinv[i] * J[i * 5 + j], X[i][j] = i == j ? 1.0 : 0.0;
+#pragma unroll
     for (int k = 0; k < 5; k++)
     {
         int pr = k, pc = k;
         real best = -1;
+#pragma unroll
         for (int i = k; i < 5; i++)
+#pragma unroll
             for (int j = k; j < 5; j++)
                 if (fabs(P[i][j]) > best)
                     best = fabs(P[i][j]), pr = i, pc = j;
         ok = ok && best > 0;
-        for (int j = 0; j < 5; j++)
+#pragma unroll
+        for (int i = k + 1; i < 5; i++)
         {
-            real t = P[k][j];
-            P[k][j] = P[pr][j], P[pr][j] = t;
-            t = X[k][j];
-            X[k][j] = X[pr][j], X[pr][j] = t;
+            const bool row = pr == i;
+#pragma unroll
+            for (int j = 0; j < 5; j++)
+            {
+                const real a = P[k][j], b = P[i][j], c = X[k][j], d = X[i][j];
+                P[k][j] = row ? b : a, P[i][j] = row ? a : b;
+                X[k][j] = row ? d : c, X[i][j] = row ? c : d;
+            }
         }
-        for (int i = 0; i < 5; i++)
+#pragma unroll
+        for (int i = k + 1; i < 5; i++)
         {
-            real t = P[i][k];
-            P[i][k] = P[i][pc], P[i][pc] = t;
+            const bool col = pc == i;
+#pragma unroll
+            for (int j = 0; j < 5; j++)
+            {
+                const real a = P[j][k], b = P[j][i];
+                P[j][k] = col ? b : a, P[j][i] = col ? a : b;
+            }
+            const int a = cp[k], b = cp[i];
+            cp[k] = col ? b : a, cp[i] = col ? a : b;
         }
-        int t = cp[k];
-        cp[k] = cp[pc], cp[pc] = t;
         const real piv = 1.0 / P[k][k];
+#pragma unroll
         for (int j = 0; j < 5; j++)
             P[k][j] *= piv, X[k][j] *= piv;
+#pragma unroll
         for (int i = 0; i < 5; i++)
         {
             if (i == k)
                 continue;
             const real fct = P[i][k];
-            if (fct == 0)
-                continue;
+#pragma unroll
             for (int j = 0; j < 5; j++)
                 P[i][j] -= fct * P[k][j], X[i][j] -= fct * X[k][j];
         }
     }
-    for (int k = 0; k < 5; k++)
+#pragma unroll
+    for (int r = 0; r < 5; r++)
+#pragma unroll
         for (int j = 0; j < 5; j++)
-            Jinv[cp[k] * 5 + j] = X[k][j] * dinv[j];
+        {
+            real v = X[0][j];
+#pragma unroll
+            for (int k = 1; k < 5; k++)
+                v = cp[k] == r ? X[k][j] : v;
+            Jinv[r * 5 + j] = v * dinv[j];
+        }
     return ok;
 }
 
@@ -313,16 +338,111 @@ __device__ inline bool invertBlock5(const real *J, real *Jinv)
 // with linMode 1, EulerEvaluator_EvaluateDt.hxx:1762-1835); then 1/dTau + 1/dt on the diagonal.
 // jd and jinv are [25][N] (row-major 5x5 per cell, cell index fastest).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(128) kLUSGSInitBlock(DevMesh m, real gamma, const real *__restrict__ dTau, real dt,
-                                                       real alphaDiag, const real *__restrict__ u,
-                                                       const real *__restrict__ lam, const real *__restrict__ lamRoe,
-                                                       real *__restrict__ jd, real *__restrict__ jinv,
-                                                       int *__restrict__ bad)
+// the face's eigenvalues seen from cell i across slot k, its normal out of the cell, the neighbour's (or
+// ghost's) state and the Roe average of the two
+struct BlockFace
+{
+    real n[3], l0, l123, l4, lvis, coef, uj[5];
+    int type; // boundary type, 0 inside
+    RoeAve ra;
+};
+__device__ inline bool blockFace(const DevMesh &m, real gamma, idx i, int k, const real *ui, real voli, real alphaDiag,
+                                 const real *__restrict__ u, const real *__restrict__ lam,
+                                 const real *__restrict__ lamRoe, BlockFace &b)
+{
+    const size_t N = m.N, F = m.F;
+    const idx f = m.c2f[(size_t)k * N + i];
+    if (f < 0)
+        return false;
+    const idx o = m.c2c[(size_t)k * N + i];
+    const bool front = (m.c2flag[(size_t)k * N + i] & 1) != 0;
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+        b.n[r] = m.fmeanN[(size_t)r * F + f] * (front ? -1.0 : 1.0);
+    faceLambdas(lam, lamRoe, F, f, front, b.l0, b.l123, b.l4);
+    b.lvis = lam[2 * F + f];
+    b.coef = (0.5 * alphaDiag) * m.farea[f] / voli;
+    b.type = 0;
+    if (o < 0)
+    {
+        const int zone = m.fzone[f];
+        b.type = m.bcType[zone];
+        bcGhost(b.type, ui, b.n, m.bcVal + (size_t)zone * 5, gamma, b.uj);
+    }
+    else
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            b.uj[v] = u[(size_t)v * N + o];
+    roeAverage(ui, b.uj, gamma, b.ra);
+    return true;
+}
+// adds the slot's part of the diagonal block
+__device__ inline void blockDiagAdd(const DevMesh &m, real gamma, const BlockFace &b, real (&J)[25])
+{
+    // the isothermal wall linearises as the adiabatic one (the linearised ghost of
+    // generateBV_ViscousWall returns before the density reset, EvaluateDt.hxx:2265-2266)
+    const int typeLin = b.type == BC_WALL_ISO ? BC_WALL : b.type;
+    if (typeLin == BC_WALL || typeLin == BC_WALL_INVIS || typeLin == BC_SYM)
+    {
+        // (A(u_g) - |A| - lambdaVis) dU_g/dU_i, column c of dU_g/dU_i being the ghost map of e_c
+        real JBC[25];
+#pragma unroll
+        for (int c = 0; c < 5; c++)
+        {
+            real e[5] = {0, 0, 0, 0, 0}, g[5];
+            e[c] = 1;
+            bcGhost<real, false>(typeLin, e, b.n, m.bcVal, gamma, g);
+#pragma unroll
+            for (int r = 0; r < 5; r++)
+                JBC[r * 5 + c] = g[r];
+        }
+        real IJ[25];
+#pragma unroll
+        for (int c = 0; c < 5; c++)
+        {
+            real e[5] = {0, 0, 0, 0, 0}, dF[5], inc[5];
+            e[c] = 1;
+            fluxJacDu<real>(b.uj, b.n, e, b.lvis, gamma, dF);
+            roeIncT<real>(e, b.n, b.ra, b.l0, b.l123, b.l4, gamma, inc);
+#pragma unroll
+            for (int r = 0; r < 5; r++)
+                IJ[r * 5 + c] = dF[r] - inc[r];
+        }
+#pragma unroll
+        for (int r = 0; r < 5; r++)
+#pragma unroll
+            for (int c = 0; c < 5; c++)
+            {
+                real acc = 0;
+#pragma unroll
+                for (int q = 0; q < 5; q++)
+                    acc += IJ[r * 5 + q] * JBC[q * 5 + c];
+                J[r * 5 + c] += b.coef * acc;
+            }
+    }
+#pragma unroll
+    for (int c = 0; c < 5; c++)
+    {
+        real e[5] = {0, 0, 0, 0, 0}, inc[5];
+        e[c] = 1;
+        roeIncT<real>(e, b.n, b.ra, b.l0, b.l123, b.l4, gamma, inc);
+        inc[c] += b.lvis;
+#pragma unroll
+        for (int r = 0; r < 5; r++)
+            J[r * 5 + c] += b.coef * inc[r];
+    }
+}
+
+__global__ void __launch_bounds__(64) kLUSGSInitBlock(DevMesh m, real gamma, const real *__restrict__ dTau, real dt,
+                                                      real alphaDiag, const real *__restrict__ u,
+                                                      const real *__restrict__ lam, const real *__restrict__ lamRoe,
+                                                      real *__restrict__ jd, real *__restrict__ jinv,
+                                                      int *__restrict__ bad)
 {
     const idx i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= m.N)
         return;
-    const size_t N = m.N, F = m.F;
+    const size_t N = m.N;
     real ui[5], J[25];
 #pragma unroll
     for (int v = 0; v < 5; v++)
@@ -333,80 +453,9 @@ __global__ void __launch_bounds__(128) kLUSGSInitBlock(DevMesh m, real gamma, co
     const real voli = m.vol[i];
     for (int k = 0; k < m.K; k++)
     {
-        const idx f = m.c2f[(size_t)k * N + i];
-        if (f < 0)
-            continue;
-        const idx o = m.c2c[(size_t)k * N + i];
-        const bool front = (m.c2flag[(size_t)k * N + i] & 1) != 0;
-        real n[3], l0, l123, l4;
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-            n[r] = m.fmeanN[(size_t)r * F + f] * (front ? -1.0 : 1.0);
-        faceLambdas(lam, lamRoe, F, f, front, l0, l123, l4);
-        const real lvis = lam[2 * F + f];
-        const real coef = (0.5 * alphaDiag) * m.farea[f] / voli;
-        const bool bnd = o < 0;
-        int type = 0;
-        real uj[5];
-        if (bnd)
-        {
-            const int zone = m.fzone[f];
-            type = m.bcType[zone];
-            bcGhost(type, ui, n, m.bcVal + (size_t)zone * 5, gamma, uj);
-        }
-        else
-#pragma unroll
-            for (int v = 0; v < 5; v++)
-                uj[v] = u[(size_t)v * N + o];
-        RoeAve ra;
-        roeAverage(ui, uj, gamma, ra);
-        // the isothermal wall linearises as the adiabatic one (the linearised ghost of
-        // generateBV_ViscousWall returns before the density reset, EvaluateDt.hxx:2265-2266)
-        const int typeLin = type == BC_WALL_ISO ? BC_WALL : type;
-        if (bnd && (typeLin == BC_WALL || typeLin == BC_WALL_INVIS || typeLin == BC_SYM))
-        {
-            // (A(u_g) - |A| - lambdaVis) dU_g/dU_i, column c of dU_g/dU_i being the ghost map of e_c
-            real JBC[25];
-            for (int c = 0; c < 5; c++)
-            {
-                real e[5] = {0, 0, 0, 0, 0}, g[5];
-                e[c] = 1;
-                bcGhost(typeLin, e, n, m.bcVal, gamma, g);
-#pragma unroll
-                for (int r = 0; r < 5; r++)
-                    JBC[r * 5 + c] = g[r];
-            }
-            real IJ[25];
-            for (int c = 0; c < 5; c++)
-            {
-                real e[5] = {0, 0, 0, 0, 0}, dF[5], inc[5];
-                e[c] = 1;
-                fluxJacDu<real>(uj, n, e, lvis, gamma, dF);
-                roeIncT<real>(e, n, ra, l0, l123, l4, gamma, inc);
-#pragma unroll
-                for (int r = 0; r < 5; r++)
-                    IJ[r * 5 + c] = dF[r] - inc[r];
-            }
-            for (int r = 0; r < 5; r++)
-                for (int c = 0; c < 5; c++)
-                {
-                    real acc = 0;
-#pragma unroll
-                    for (int q = 0; q < 5; q++)
-                        acc += IJ[r * 5 + q] * JBC[q * 5 + c];
-                    J[r * 5 + c] += coef * acc;
-                }
-        }
-        for (int c = 0; c < 5; c++)
-        {
-            real e[5] = {0, 0, 0, 0, 0}, inc[5];
-            e[c] = 1;
-            roeIncT<real>(e, n, ra, l0, l123, l4, gamma, inc);
-            inc[c] += lvis;
-#pragma unroll
-            for (int r = 0; r < 5; r++)
-                J[r * 5 + c] += coef * inc[r];
-        }
+        BlockFace b;
+        if (blockFace(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b))
+            blockDiagAdd(m, gamma, b, J);
     }
     const real dg = 1.0 / dTau[i] + 1.0 / dt;
 #pragma unroll
@@ -428,7 +477,7 @@ void launchLUSGSInitBlock(Ctx &c, const GasParams &gp, const real *dTau, real dt
                           const real *lam, const real *lamRoe, real *jd, real *jinv, int *bad)
 {
     KernelTimer kt(c, K_LUSGS_INIT);
-    kLUSGSInitBlock<<<gridFor(c.m.N, 128), 128, 0, c.stream>>>(c.m, gp.gamma, dTau, dt, alphaDiag, u, lam, lamRoe, jd,
+    kLUSGSInitBlock<<<gridFor(c.m.N, 64), 64, 0, c.stream>>>(c.m, gp.gamma, dTau, dt, alphaDiag, u, lam, lamRoe, jd,
                                                                jinv, bad);
     DNDSR_HIP_CHECK(hipGetLastError());
 }
@@ -701,44 +750,6 @@ __global__ void __launch_bounds__(256) kCopyColourInc(DevMesh m, idx lo, idx hi,
         to[(size_t)v * N + i] = from[(size_t)v * N + i];
 }
 
-// (1 + sgsIter) symmetric block sweeps from the increments in a (b: the other array), the
-// result in *result.  With Gauss-Seidel updates a sweep after the first skips its first
-// colour, whose pass would repeat the previous sweep's last one (same inputs, same values);
-// the sweep reads that colour's increments from the array it reads, and the next sweep the
-// colour from the array it writes until that colour's own pass; one copy after the last
-// sweep puts the skipped colour's increments into the result.
-template <typename T>
-static void sgsBlockSymmetric(Ctx &c, const GasParams &gp, T alphaDiag, const T *rhs, const T *u, T *a, T *b,
-                              const T *jinv, const T *lam, const T *lamRoe, int sgsIter, int gsUpdate,
-                              real *sumIncDev, T **result)
-{
-    DevMesh &m = c.m;
-    const int nC = m.nColor;
-    const bool canSkip = gsUpdate && nC >= 2;
-    int prevSkip = -1;
-    for (int s = 0; s <= sgsIter; s++)
-        for (int dir = 1; dir >= 0; dir--)
-        {
-            const int first = dir ? 0 : nC - 1, last = dir ? nC - 1 : 0;
-            const int fCol = canSkip && !(s == 0 && dir == 1) ? first : -1;
-            const int lCol = prevSkip == last ? last : -1;
-            sgsSweepBlock<T>(c, gp, alphaDiag, rhs, u, a, b, jinv, lam, lamRoe, dir, gsUpdate, 0, sumIncDev, fCol,
-                             lCol);
-            prevSkip = fCol;
-            std::swap(a, b);
-        }
-    if (prevSkip >= 0)
-    {
-        const idx lo = m.colorPtrHost[prevSkip], hi = m.colorPtrHost[prevSkip + 1];
-        if (hi > lo)
-        {
-            KernelTimer kt(c, K_SGS);
-            kCopyColourInc<T><<<gridFor(hi - lo, 256), 256, 0, c.stream>>>(m, lo, hi, b, a);
-            DNDSR_HIP_CHECK(hipGetLastError());
-        }
-    }
-    *result = a;
-}
 void launchCopyColourInc64(Ctx &c, int col, const real *from, real *to)
 {
     const idx lo = c.m.colorPtrHost[col], hi = c.m.colorPtrHost[col + 1];
@@ -747,17 +758,225 @@ void launchCopyColourInc64(Ctx &c, int col, const real *from, real *to)
     kCopyColourInc<real><<<gridFor(hi - lo, 256), 256, 0, c.stream>>>(c.m, lo, hi, from, to);
     DNDSR_HIP_CHECK(hipGetLastError());
 }
-void launchSGSBlockSymmetric64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, const real *u, real *a,
-                               real *b, const real *jinv, const real *lam, const real *lamRoe, int sgsIter,
-                               int gsUpdate, real *sumIncDev, real **result)
+// ---------------------------------------------------------------------------
+// The block LU-SGS solve of the device implicit loop: LUSGSMatrixInit with useRoeJacobian and
+// (1 + sgsIter) symmetric sweeps from a zero increment.  The off-diagonal blocks do not change over the
+// sweeps (2 (1 + sgsIter) passes over every cell), so kSGSBlkPrep forms them once, already multiplied by
+// the cell's inverse:
+//   x_i = b_i - sum_k C_k x_j,  b_i = J_i^-1 rhs_i,
+//   C_k = 0.5 alpha A_f / V_i J_i^-1 (A(u_j) - |A|_Roe(u_j, u_i) - lambdaVis I),
+// and a pass is a stream of 25 K coalesced values per cell with one 64-byte gather per neighbour (a
+// Roe average, two eigenvector products and 21 gathers per slot when each pass forms the block).
+// Positions as in sgs.hip (colour-major, in place for Gauss-Seidel); everything is formed in FP64 and
+// stored in T.  C [K 25][N], b [5][N], x [N][8].
+// ---------------------------------------------------------------------------
+constexpr int kBlkRow = 8;
+template <typename T>
+__global__ void __launch_bounds__(64) kSGSBlkPrep(DevMesh m, real gamma, const real *__restrict__ dTau, real rdt,
+                                                  real alphaDiag, const real *__restrict__ u,
+                                                  const real *__restrict__ rhs, const real *__restrict__ lam,
+                                                  const real *__restrict__ lamRoe, T *__restrict__ C,
+                                                  T *__restrict__ bv, idx *__restrict__ nbr, int *__restrict__ bad)
 {
-    sgsBlockSymmetric<real>(c, gp, alphaDiag, rhs, u, a, b, jinv, lam, lamRoe, sgsIter, gsUpdate, sumIncDev, result);
+    const idx p = xcdTile(blockIdx.x, gridDim.x) * 64 + (idx)threadIdx.x;
+    if (p >= m.N)
+        return;
+    const size_t N = m.N;
+    const idx i = m.colorCells[p];
+    real ui[5], J[25], Ji[25];
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+        ui[v] = u[(size_t)v * N + i];
+#pragma unroll
+    for (int q = 0; q < 25; q++)
+        J[q] = 0;
+    const real voli = m.vol[i];
+    for (int k = 0; k < m.K; k++)
+    {
+        BlockFace b;
+        if (blockFace(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b))
+            blockDiagAdd(m, gamma, b, J);
+    }
+    const real dg = 1.0 / dTau[i] + rdt;
+#pragma unroll
+    for (int k = 0; k < 5; k++)
+        J[k * 5 + k] += dg;
+    if (!invertBlock5(J, Ji))
+        atomicOr(bad, 1);
+    {
+        real r[5];
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            r[v] = rhs[(size_t)v * N + i];
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            real a = 0;
+#pragma unroll
+            for (int q = 0; q < 5; q++)
+                a += Ji[v * 5 + q] * r[q];
+            bv[(size_t)v * N + p] = (T)a;
+        }
+    }
+    for (int k = 0; k < m.K; k++)
+    {
+        const idx o = m.c2c[(size_t)k * N + i];
+        const bool on = m.c2f[(size_t)k * N + i] >= 0 && o >= 0 && o != i;
+        nbr[(size_t)k * N + p] = on ? m.cellPos[o] : idx(-1);
+        if (!on)
+            continue;
+        BlockFace b;
+        blockFace(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b);
+#pragma unroll
+        for (int c = 0; c < 5; c++)
+        {
+            real e[5] = {0, 0, 0, 0, 0}, dF[5], inc[5];
+            e[c] = 1;
+            fluxJacDu<real>(b.uj, b.n, e, b.lvis, gamma, dF);
+            roeIncT<real>(e, b.n, b.ra, b.l0, b.l123, b.l4, gamma, inc);
+#pragma unroll
+            for (int r = 0; r < 5; r++)
+                dF[r] = b.coef * (dF[r] - inc[r]);
+#pragma unroll
+            for (int r = 0; r < 5; r++)
+            {
+                real a = 0;
+#pragma unroll
+                for (int q = 0; q < 5; q++)
+                    a += Ji[r * 5 + q] * dF[q];
+                C[(size_t)(k * 25 + r * 5 + c) * N + p] = (T)a;
+            }
+        }
+    }
 }
-void launchSGSBlockSymmetric32(Ctx &c, const GasParams &gp, float alphaDiag, const float *rhs, const float *u,
-                               float *a, float *b, const float *jinv, const float *lam, const float *lamRoe,
-                               int sgsIter, int gsUpdate, real *sumIncDev, float **result)
+
+template <typename T, int K>
+__global__ void __launch_bounds__(64) kSGSBlkPass(size_t N, const T *x, T *xw, const T *__restrict__ C,
+                                                  const T *__restrict__ bv, const idx *__restrict__ nbr, int gs,
+                                                  int first, idx begin, idx end)
 {
-    sgsBlockSymmetric<float>(c, gp, alphaDiag, rhs, u, a, b, jinv, lam, lamRoe, sgsIter, gsUpdate, sumIncDev, result);
+    const idx p = begin + xcdTile(blockIdx.x, gridDim.x) * 64 + (idx)threadIdx.x;
+    if (p >= end)
+        return;
+    idx po[K];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        po[k] = nbr[(size_t)k * N + p];
+    T acc[kBlkRow];
+#pragma unroll
+    for (int v = 0; v < kBlkRow; v++)
+        acc[v] = v < 5 ? bv[(size_t)v * N + p] : T(0);
+    T d[K][5];
+    bool use[K];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+    {
+        // unconditional (an unused slot reads the cell's own row): see sgs.hip
+        use[k] = po[k] >= 0 && !(first && !(gs && po[k] < p));
+        const T *row = x + (size_t)(use[k] ? po[k] : p) * kBlkRow;
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            d[k][v] = row[v];
+    }
+#pragma unroll
+    for (int k = 0; k < K; k++)
+    {
+        if (!use[k])
+            continue;
+#pragma unroll
+        for (int r = 0; r < 5; r++)
+        {
+            T a = 0;
+#pragma unroll
+            for (int q = 0; q < 5; q++)
+                a += C[(size_t)(k * 25 + r * 5 + q) * N + p] * d[k][q];
+            acc[r] -= a;
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < kBlkRow; v++)
+        xw[(size_t)p * kBlkRow + v] = acc[v];
+}
+
+template <typename T>
+static void sgsBlkPass(Ctx &c, const SGSBlockWork<T> &w, const T *x, T *xw, int gs, int first, idx b, idx e)
+{
+    DevMesh &m = c.m;
+    if (e <= b)
+        return;
+    KernelTimer kt(c, K_SGS);
+    auto go = [&](auto kern) {
+        kern<<<gridFor(e - b, 64), 64, 0, c.stream>>>((size_t)m.N, x, xw, w.C, w.b, w.nbr, gs, first, b, e);
+    };
+    switch (m.K)
+    {
+    case 2: go(kSGSBlkPass<T, 2>); break;
+    case 3: go(kSGSBlkPass<T, 3>); break;
+    case 4: go(kSGSBlkPass<T, 4>); break;
+    case 5: go(kSGSBlkPass<T, 5>); break;
+    case 6: go(kSGSBlkPass<T, 6>); break;
+    default: throw std::runtime_error("unsupported number of faces per cell");
+    }
+    DNDSR_HIP_CHECK(hipGetLastError());
+}
+
+template <typename T>
+static void sgsBlockSolve(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, real dt, const real *u,
+                          const real *dTau, const real *lam, const real *lamRoe, SGSBlockWork<T> &w, int sgsIter,
+                          int gsUpdate, int *bad, T **result)
+{
+    DevMesh &m = c.m;
+    const size_t N = m.N;
+    if (!w.C)
+    {
+        w.x[0] = devAlloc<T>(c, kBlkRow * N);
+        w.b = devAlloc<T>(c, 5 * N);
+        w.nbr = devAlloc<idx>(c, (size_t)m.K * N);
+        w.C = devAlloc<T>(c, (size_t)m.K * 25 * N);
+    }
+    if (!gsUpdate && !w.x[1])
+        w.x[1] = devAlloc<T>(c, kBlkRow * N);
+    {
+        KernelTimer kt(c, K_LUSGS_INIT);
+        kSGSBlkPrep<T><<<gridFor(m.N, 64), 64, 0, c.stream>>>(m, gp.gamma, dTau, 1.0 / dt, alphaDiag, u, rhs, lam,
+                                                              lamRoe, w.C, w.b, w.nbr, bad);
+        DNDSR_HIP_CHECK(hipGetLastError());
+    }
+    T *x = w.x[0];
+    if (!gsUpdate)
+    {
+        T *y = w.x[1];
+        for (int s = 0; s < 2 * (1 + sgsIter); s++)
+        {
+            sgsBlkPass<T>(c, w, x, y, 0, s == 0, 0, m.N);
+            std::swap(x, y);
+        }
+    }
+    else
+        for (int s = 0; s <= sgsIter; s++)
+            for (int dir = 1; dir >= 0; dir--)
+            {
+                // a sweep after the first skips its first colour, whose pass would repeat the last one
+                const bool first = s == 0 && dir == 1;
+                for (int q = first || m.nColor < 2 ? 0 : 1; q < m.nColor; q++)
+                {
+                    const int col = dir ? q : m.nColor - 1 - q;
+                    sgsBlkPass<T>(c, w, x, x, 1, first, m.colorPtrHost[col], m.colorPtrHost[col + 1]);
+                }
+            }
+    *result = x;
+}
+void launchSGSBlockSolve64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, real dt, const real *u,
+                           const real *dTau, const real *lam, const real *lamRoe, SGSBlockWork<real> &w, int sgsIter,
+                           int gsUpdate, int *bad, real **result)
+{
+    sgsBlockSolve<real>(c, gp, alphaDiag, rhs, dt, u, dTau, lam, lamRoe, w, sgsIter, gsUpdate, bad, result);
+}
+void launchSGSBlockSolve32(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, real dt, const real *u,
+                           const real *dTau, const real *lam, const real *lamRoe, SGSBlockWork<float> &w, int sgsIter,
+                           int gsUpdate, int *bad, float **result)
+{
+    sgsBlockSolve<float>(c, gp, alphaDiag, rhs, dt, u, dTau, lam, lamRoe, w, sgsIter, gsUpdate, bad, result);
 }
 
 void launchSGSSweepBlock64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, const real *u,
