@@ -346,6 +346,7 @@ struct BlockFace
     int type; // boundary type, 0 inside
     RoeAve ra;
 };
+template <bool GAS>
 __device__ inline bool blockFace(const DevMesh &m, real gamma, idx i, int k, const real *ui, real voli, real alphaDiag,
                                  const real *__restrict__ u, const real *__restrict__ lam,
                                  const real *__restrict__ lamRoe, BlockFace &b)
@@ -367,7 +368,7 @@ __device__ inline bool blockFace(const DevMesh &m, real gamma, idx i, int k, con
     {
         const int zone = m.fzone[f];
         b.type = m.bcType[zone];
-        bcGhost(b.type, ui, b.n, m.bcVal + (size_t)zone * 5, gamma, b.uj);
+        bcGhost<real, GAS>(b.type, ui, b.n, m.bcVal + (size_t)zone * 5, gamma, b.uj);
     }
     else
 #pragma unroll
@@ -384,41 +385,19 @@ __device__ inline void blockDiagAdd(const DevMesh &m, real gamma, const BlockFac
     const int typeLin = b.type == BC_WALL_ISO ? BC_WALL : b.type;
     if (typeLin == BC_WALL || typeLin == BC_WALL_INVIS || typeLin == BC_SYM)
     {
-        // (A(u_g) - |A| - lambdaVis) dU_g/dU_i, column c of dU_g/dU_i being the ghost map of e_c
-        real JBC[25];
+        // (A(u_g) - |A| - lambdaVis) dU_g/dU_i column by column: the ghost map of e_c
 #pragma unroll
         for (int c = 0; c < 5; c++)
         {
-            real e[5] = {0, 0, 0, 0, 0}, g[5];
+            real e[5] = {0, 0, 0, 0, 0}, g[5], dF[5], inc[5];
             e[c] = 1;
             bcGhost<real, false>(typeLin, e, b.n, m.bcVal, gamma, g);
+            fluxJacDu<real>(b.uj, b.n, g, b.lvis, gamma, dF);
+            roeIncT<real>(g, b.n, b.ra, b.l0, b.l123, b.l4, gamma, inc);
 #pragma unroll
             for (int r = 0; r < 5; r++)
-                JBC[r * 5 + c] = g[r];
+                J[r * 5 + c] += b.coef * (dF[r] - inc[r]);
         }
-        real IJ[25];
-#pragma unroll
-        for (int c = 0; c < 5; c++)
-        {
-            real e[5] = {0, 0, 0, 0, 0}, dF[5], inc[5];
-            e[c] = 1;
-            fluxJacDu<real>(b.uj, b.n, e, b.lvis, gamma, dF);
-            roeIncT<real>(e, b.n, b.ra, b.l0, b.l123, b.l4, gamma, inc);
-#pragma unroll
-            for (int r = 0; r < 5; r++)
-                IJ[r * 5 + c] = dF[r] - inc[r];
-        }
-#pragma unroll
-        for (int r = 0; r < 5; r++)
-#pragma unroll
-            for (int c = 0; c < 5; c++)
-            {
-                real acc = 0;
-#pragma unroll
-                for (int q = 0; q < 5; q++)
-                    acc += IJ[r * 5 + q] * JBC[q * 5 + c];
-                J[r * 5 + c] += b.coef * acc;
-            }
     }
 #pragma unroll
     for (int c = 0; c < 5; c++)
@@ -454,7 +433,7 @@ __global__ void __launch_bounds__(64) kLUSGSInitBlock(DevMesh m, real gamma, con
     for (int k = 0; k < m.K; k++)
     {
         BlockFace b;
-        if (blockFace(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b))
+        if (blockFace<true>(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b))
             blockDiagAdd(m, gamma, b, J);
     }
     const real dg = 1.0 / dTau[i] + 1.0 / dt;
@@ -771,8 +750,8 @@ void launchCopyColourInc64(Ctx &c, int col, const real *from, real *to)
 // stored in T.  C [K 25][N], b [5][N], x [N][8].
 // ---------------------------------------------------------------------------
 constexpr int kBlkRow = 8;
-template <typename T>
-__global__ void __launch_bounds__(64) kSGSBlkPrep(DevMesh m, real gamma, const real *__restrict__ dTau, real rdt,
+template <typename T, bool GAS>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2))) kSGSBlkPrep(DevMesh m, real gamma, const real *__restrict__ dTau, real rdt,
                                                   real alphaDiag, const real *__restrict__ u,
                                                   const real *__restrict__ rhs, const real *__restrict__ lam,
                                                   const real *__restrict__ lamRoe, T *__restrict__ C,
@@ -794,7 +773,7 @@ __global__ void __launch_bounds__(64) kSGSBlkPrep(DevMesh m, real gamma, const r
     for (int k = 0; k < m.K; k++)
     {
         BlockFace b;
-        if (blockFace(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b))
+        if (blockFace<GAS>(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b))
             blockDiagAdd(m, gamma, b, J);
     }
     const real dg = 1.0 / dTau[i] + rdt;
@@ -826,7 +805,7 @@ __global__ void __launch_bounds__(64) kSGSBlkPrep(DevMesh m, real gamma, const r
         if (!on)
             continue;
         BlockFace b;
-        blockFace(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b);
+        blockFace<GAS>(m, gamma, i, k, ui, voli, alphaDiag, u, lam, lamRoe, b);
 #pragma unroll
         for (int c = 0; c < 5; c++)
         {
@@ -938,8 +917,10 @@ static void sgsBlockSolve(Ctx &c, const GasParams &gp, real alphaDiag, const rea
         w.x[1] = devAlloc<T>(c, kBlkRow * N);
     {
         KernelTimer kt(c, K_LUSGS_INIT);
-        kSGSBlkPrep<T><<<gridFor(m.N, 64), 64, 0, c.stream>>>(m, gp.gamma, dTau, 1.0 / dt, alphaDiag, u, rhs, lam,
-                                                              lamRoe, w.C, w.b, w.nbr, bad);
+        // the gas-dependent ghosts are an out-of-line call: compiled in only where the table has such a zone
+        auto prep = m.gasBC ? kSGSBlkPrep<T, true> : kSGSBlkPrep<T, false>;
+        prep<<<gridFor(m.N, 64), 64, 0, c.stream>>>(m, gp.gamma, dTau, 1.0 / dt, alphaDiag, u, rhs, lam, lamRoe, w.C,
+                                                    w.b, w.nbr, bad);
         DNDSR_HIP_CHECK(hipGetLastError());
     }
     T *x = w.x[0];
