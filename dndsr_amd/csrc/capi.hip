@@ -571,6 +571,7 @@ int dndsr_vr_construct(dndsr_ctx *ctx, const dndsr_mesh_desc *md, const dndsr_vr
     DNDSR_HIP_CHECK(hipStreamSynchronize(c.stream));
 
     setupMetricsAndVR(c);
+    setupLinear(c);
     // FP32 copies of the face and cell geometry read by the FP32 Gauss-Seidel sweeps
     m.fareaF = devAlloc<float>(c, F);
     m.fmeanNF = devAlloc<float>(c, 3 * F);

@@ -4,6 +4,7 @@
 #include <type_traits>
 #include "gas.hpp"
 #include "internal.hpp"
+#include "rhsbnd.hpp"
 
 namespace dndsr
 {
@@ -836,102 +837,11 @@ constexpr int rhsPointsPerLane()
     return DIM == 3 && G == 9 ? 3 : 1;
 }
 
-// Boundary faces (EvaluateRHS.hxx:194-207, 336-345), run after the tile kernel and overwriting the
-// tile kernel's flux of that face.  The Roe average takes the cell mean and its ghost at the face
-// centre (mean normal); every point takes the reconstructed state and its ghost at the point normal;
-// dLambda is the owner cell's.  A few thousand faces leave most of the device idle and the pass is
-// one chain of dependent loads and flux arithmetic, so a block is 64 faces with one wavefront per
-// point (the face constants formed by each); the point fluxes meet in LDS and are summed in point
-// order as in the tile kernels.
-template <int DIM, int NDOF, int G, int RS, bool BATCH>
-__global__ void __launch_bounds__(64 * G) kRHSBoundary(DevMesh m, GasParams gp, const real *__restrict__ u,
-                                                       const real *__restrict__ uRec, const real *__restrict__ dlc,
-                                                       real *__restrict__ fflux)
-{
-    constexpr int M = NDOF - 1;
-    __shared__ real sF[G * 5][64];
-    const int lane = threadIdx.x % 64, g = waveIndex(64);
-    const idx t = blockIdx.x * 64 + lane;
-    const bool valid = t < m.nBnd;
-    const idx f = m.bndFace[valid ? t : m.nBnd - 1];
-    const size_t N = m.N, F = m.F;
-    const idx cL = m.f2c[f];
-    const int zone = m.fzone[f];
-    real ULm[5], URm[5], UL[5], UR[5], nm[3], n[3], x[3];
-#pragma unroll
-    for (int r = 0; r < 3; r++)
-    {
-        nm[r] = m.fmeanN[(size_t)r * F + f];
-        n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
-        x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
-    }
-    const real wj = m.fwj[(size_t)g * F + f];
-    const int type = m.bcType[zone];
-    const real *far = m.bcVal + (size_t)zone * 5;
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-        UL[v] = ULm[v] = u[(size_t)v * N + cL];
-    const real dLambda = dlc ? dlc[cL] : 0.0;
-    if (uRec)
-    {
-        real xs[3], mom[M > 0 ? M : 1], phi[M > 0 ? M : 1];
-#pragma unroll
-        for (int j = 0; j < M; j++)
-            mom[j] = m.moment[(size_t)j * N + cL];
-        const real isc = m.iscale[cL];
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-        {
-            xs[r] = x[r] - m.cent[(size_t)r * N + cL];
-            if (DIM == 3 || r < 2)
-                xs[r] *= isc;
-        }
-        basisRow0<DIM, NDOF>(xs, mom, phi);
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-        {
-            real sacc = 0;
-#pragma unroll
-            for (int j = 0; j < M; j++)
-                sacc += phi[j] * uRec[((size_t)v * M + j) * N + cL];
-            UL[v] += sacc;
-        }
-    }
-    bcGhost(type, ULm, nm, far, gp.gamma, URm);
-    bcGhost(type, UL, n, far, gp.gamma, UR);
-    real Fl[5];
-    if constexpr (BATCH)
-    {
-        RoeBatchFace bf;
-        roeBatchSetup<RS>(ULm, URm, nm, gp, dLambda, bf);
-        roeBatchPoint<RS>(UL, UR, n, gp, bf, Fl);
-    }
-    else
-    {
-        RoeAve ra;
-        real l0, l1, l4;
-        roeAverage(ULm, URm, gp.gamma, ra);
-        riemannFluxR<RS>(UL, UR, ra, n, gp, dLambda, Fl, l0, l1, l4);
-    }
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-        sF[g * 5 + v][lane] = (-Fl[v]) * wj;
-    __syncthreads();
-    for (int v = g; v < 5; v += G)
-    {
-        real acc = 0;
-#pragma unroll
-        for (int q = 0; q < G; q++)
-            acc += sF[q * 5 + v][lane];
-        if (valid)
-            fflux[(size_t)v * F + f] = acc;
-    }
-}
-
 // ---------------------------------------------------------------------------
 // Laminar viscous face fluxes (EvaluateRHS.hxx:257-424 with fluxFace,
-// EvaluateDt.hxx:1163-1215; finc -= visFlux at :1460).  One thread per face, after
-// the inviscid face and boundary passes: at every face point both sides' values and
+// EvaluateDt.hxx:1163-1215; finc -= visFlux at :1460).  One thread per face (all of them, or after the
+// linear face kernel, which includes the interior ones, the boundary list), after the inviscid face and
+// boundary passes: at every face point both sides' values and
 // gradients D1phi uRec, the GRP mean gradient
 //   GradUMean = (GradL + GradR) / 2 + n (UR - UL) / distGRP,
 //   distGRP = max(min(distBaryPerp, 2 d0), d0 / 4), d0 = 2 minVol / area,
@@ -1102,11 +1012,13 @@ using ViscSide = std::conditional_t<NDOF == DIM + 1, SideLin<DIM>, SideRec<DIM, 
 
 template <int DIM, int NDOF, bool GAS>
 __global__ void __launch_bounds__(128) kRHSViscous(DevMesh m, GasParams gp, const real *__restrict__ u,
-                                                   const real *__restrict__ uRec, real *__restrict__ fflux)
+                                                   const real *__restrict__ uRec, real *__restrict__ fflux,
+                                                   const idx *__restrict__ list, idx nList)
 {
-    const idx f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= m.F)
+    const idx t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= nList)
         return;
+    const idx f = list ? list[t] : t;
     const size_t N = m.N, F = m.F;
     const idx cL = m.f2c[f], cR = m.f2c[F + f];
     const bool bnd = cR < 0;
@@ -1203,12 +1115,7 @@ static void rhsLaunch(Ctx &c, const GasParams &gp, const real *u, const real *uR
         kern<<<gridFor(c.m.F, kTileF), kTileF * G, smem, c.stream>>>(c.m, gp, u, uRec, dlc, ff);
     }
     DNDSR_HIP_CHECK(hipGetLastError());
-    if (c.m.nBnd > 0)
-    {
-        kRHSBoundary<DIM, NDOF, G, RS, BATCH><<<gridFor(c.m.nBnd, 64), 64 * G, 0, c.stream>>>(c.m, gp, u, uRec, dlc,
-                                                                                             ff);
-        DNDSR_HIP_CHECK(hipGetLastError());
-    }
+    rhsBoundaryLaunch<DIM, NDOF, G, RS, BATCH>(c, gp, u, uRec, dlc, ff);
 }
 
 template <int DIM, int NDOF, int G>
@@ -1261,19 +1168,27 @@ static void rhsDispatchRS(Ctx &c, const GasParams &gp, const real *u, const real
 // face quadrature sizes: 2-D Line rules of 2 / 3 points (intOrder 2..5), 3-D Quad rules
 // of 4 / 9 points (intOrder 2..5), Tri rules of 6 points (intOrder 3..4); the tile
 // kernel is specialised on the point count.
+static const char *const kBadFaceRule =
+    "EvaluateRHS supports 2/3 face points in 2-D (intOrder 2..5), 4/9 on quadrilateral faces (intOrder 2..5) and 6 on "
+    "triangular faces (intOrder 3..4)";
 template <int DIM, int NDOF>
 static void rhsDispatch(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff)
 {
     constexpr int G1 = DIM == 2 ? 2 : 4, G2 = DIM == 2 ? 3 : 9;
-    if (c.m.G == G1)
-        rhsDispatchRS<DIM, NDOF, G1>(c, gp, u, uRec, dlc, ff);
-    else if (c.m.G == G2)
+    constexpr bool LIN = NDOF == DIM + 1; // linear: all rules but the 9-point one take the kernel of facelin.hip
+    if (c.m.G == G2 && (!LIN || DIM == 3))
         rhsDispatchRS<DIM, NDOF, G2>(c, gp, u, uRec, dlc, ff);
-    else if (DIM == 3 && c.m.G == 6)
-        rhsDispatchRS<DIM, NDOF, 6>(c, gp, u, uRec, dlc, ff);
+    else if constexpr (!LIN)
+    {
+        if (c.m.G == G1)
+            rhsDispatchRS<DIM, NDOF, G1>(c, gp, u, uRec, dlc, ff);
+        else if (DIM == 3 && c.m.G == 6)
+            rhsDispatchRS<DIM, NDOF, 6>(c, gp, u, uRec, dlc, ff);
+        else
+            throw std::runtime_error(kBadFaceRule);
+    }
     else
-        throw std::runtime_error("EvaluateRHS supports 2/3 face points in 2-D (intOrder 2..5), 4/9 on quadrilateral "
-                                 "faces (intOrder 2..5) and 6 on triangular faces (intOrder 3..4)");
+        throw std::runtime_error(kBadFaceRule);
 }
 
 void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *rhs,
@@ -1283,9 +1198,15 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
     if (m.nBnd > 0 && !m.bcType)
         throw std::runtime_error("the mesh has boundary faces: set the boundary conditions first (dndsr_set_bc)");
     real *ff = faceFluxBuf ? faceFluxBuf : c.faceFlux;
+    if (gp.viscous && !(gp.prGas > 0 && gp.Rgas > 0 && gp.muGas >= 0))
+        throw std::runtime_error("viscous residual needs prGas > 0, Rgas > 0 and muGas >= 0");
+    // first-order and linear reconstructions: the interior faces' whole flux in one pass
+    const bool linear = (!uRec || m.P == 1) && rhsLinearRule(m);
     {
         KernelTimer kt(c, K_RHS_FACE); // inviscid interior, periodic and boundary faces
-        if (m.dim == 2)
+        if (linear)
+            launchRHSFaceLinear(c, gp, u, uRec, dlc, ff, faceFluxBuf == nullptr);
+        else if (m.dim == 2)
         {
             if (!uRec || m.P == 1)
                 rhsDispatch<2, 3>(c, gp, u, uRec, dlc, ff);
@@ -1304,21 +1225,22 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
                 rhsDispatch<3, 20>(c, gp, u, uRec, dlc, ff);
         }
     }
-    if (gp.viscous)
+    const bool bndOnly = linear && rhsLinearViscous(m); // the interior faces have theirs
+    if (gp.viscous && (!bndOnly || m.nBnd > 0))
     {
         KernelTimer kt(c, K_RHS_VISCOUS);
-        if (!(gp.prGas > 0 && gp.Rgas > 0 && gp.muGas >= 0))
-            throw std::runtime_error("viscous residual needs prGas > 0, Rgas > 0 and muGas >= 0");
-        const int nb = gridFor(m.F, 128);
+        const idx *list = bndOnly ? m.bndFace : nullptr;
+        const idx nList = bndOnly ? m.nBnd : m.F;
+        const int nb = gridFor(nList, 128);
         const int P = uRec ? m.P : 1;
         // the gas-dependent ghosts only where the table has such a zone (their branch costs
         // the kernel registers)
         auto launchVis = [&](auto dimC, auto ndofC) {
             constexpr int D = decltype(dimC)::value, ND = decltype(ndofC)::value;
             if (m.gasBC)
-                kRHSViscous<D, ND, true><<<nb, 128, 0, c.stream>>>(m, gp, u, uRec, ff);
+                kRHSViscous<D, ND, true><<<nb, 128, 0, c.stream>>>(m, gp, u, uRec, ff, list, nList);
             else
-                kRHSViscous<D, ND, false><<<nb, 128, 0, c.stream>>>(m, gp, u, uRec, ff);
+                kRHSViscous<D, ND, false><<<nb, 128, 0, c.stream>>>(m, gp, u, uRec, ff, list, nList);
         };
         using I2 = std::integral_constant<int, 2>;
         using I3 = std::integral_constant<int, 3>;

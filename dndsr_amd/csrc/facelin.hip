@@ -1,0 +1,498 @@
+// facelin.hip -- face fluxes of EvaluateRHS with a linear (or no) reconstruction, one pass over the
+// interior faces: the Riemann flux and, in a viscous run with one normal per face, the Navier-Stokes flux
+// (EulerEvaluator_EvaluateRHS.hxx:171-662, EvaluateDt.hxx:1163-1215).
+//
+// One thread per face (lane = face), no LDS and no barrier.  A linear reconstruction needs few values
+// per side: the basis row times the coefficients is G (x - cent - scale moment), G = uRec / scale, so a
+// side is its mean u, the gradient G and the offset (26 values in 3-D, 23 on tetrahedra), read once and
+// reduced at once to its states at the face's points (on a triangle, whose points are affine
+// combinations of its vertices, to the state at one vertex and its changes along two sides); of the
+// gradients only the mean of the two sides lives on, for the viscous flux.  The tile kernels of the higher orders, one wavefront per point
+// and the sides staged in LDS, re-read 80 rows of it there and left the viscous flux to a second pass
+// with all its gathers.
+//
+// On a triangle the unit normal is one for the face and the points come from the vertices, so 13
+// values per face (vertices, mean normal, area) replace the 42 of the point tables; neighbours of an
+// unstructured mesh are gathered from cell records of 160 + 32 bytes in 16-byte loads, one or two
+// cache lines each, instead of 27 scattered rows (the address pipeline, one line per lane and load,
+// was the tile kernel's bound there).  The records are written by a pass over the cells (kLinPack).
+// Meshes of quadrilaterals or hexahedra are numbered so that neighbouring faces have neighbouring
+// cells: their rows are coalesced as they stand.
+//
+// Measured: 945k tetrahedra (1.9M faces), viscous Roe: 171 us + 72 us for the records, against 288 us
+// (tile kernel) + 424 us (viscous pass); 333k faces of a mixed 2-D mesh, viscous Roe: 26 us against
+// 33 + 37 us; 744k hexahedral faces, inviscid Roe: 69 us against 84 us.
+#include "geom.hpp"
+#include "rhsbnd.hpp"
+
+namespace dndsr
+{
+constexpr int kLinRow = 20;
+
+struct ViscGas
+{
+    real g1, Cp, kOverMu;
+};
+// Navier-Stokes flux at a point (viscousPointFlux of gas.hpp with the mean gradient given and its
+// quotients by the density taken as products with one reciprocal): Gm + n (UR - UL) idist is the
+// gradient, Gm the mean of the two sides'
+template <int DIM>
+__device__ __forceinline__ void viscousPointLin(const GasParams &gp, const ViscGas &vg, const real *UL, const real *UR,
+                                                const real (&Gm)[DIM][5], const real *n, real idist, real *Fv)
+{
+    real U[5], jump[5];
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+        U[v] = 0.5 * (UL[v] + UR[v]), jump[v] = (UR[v] - UL[v]) * idist;
+    const real ri = rcpN(U[0]);
+    const real vel[3] = {U[1] * ri, U[2] * ri, U[3] * ri};
+    const real vSqr = dot3(vel, vel);
+    const real p = vg.g1 * (U[4] - 0.5 * U[0] * vSqr);
+    // velocity and temperature gradients: dv = (d(rho v) - v d rho) / rho,
+    // dp = (gamma - 1) (dE - v . d(rho v) + |v|^2 d rho / 2), dT = c (rho dp - p d rho)
+    real gv[3][3], gT[3];
+    const real c = gp.gamma * ri * ri / (vg.g1 * vg.Cp);
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+    {
+        real g[5];
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            g[v] = (d < DIM ? Gm[d < DIM ? d : 0][v] : 0.0) + n[d] * jump[v];
+        real vm = 0;
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+        {
+            gv[d][j] = (g[1 + j] - vel[j] * g[0]) * ri;
+            vm += vel[j] * g[1 + j];
+        }
+        const real dp = vg.g1 * (g[4] - vm + 0.5 * vSqr * g[0]);
+        gT[d] = c * (U[0] * dp - p * g[0]);
+    }
+    const real mu = muEff(gp, U, gasTemperature(gp, p, U[0]));
+    const real k = vg.kOverMu * mu;
+    const real tr = (-2. / 3.) * mu * (gv[0][0] + gv[1][1] + gv[2][2]);
+    real e = 0;
+    Fv[0] = 0;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+    {
+        real s = tr * n[i];
+#pragma unroll
+        for (int j = 0; j < 3; j++)
+            s += mu * (gv[i][j] + gv[j][i]) * n[j];
+        Fv[1 + i] = s;
+        e += s * vel[i] + k * gT[i] * n[i];
+    }
+    Fv[4] = e;
+}
+
+// u [5] and G [3][5] of every cell, cell-major
+__global__ void __launch_bounds__(256) kLinPack(DevMesh m, const real *__restrict__ u, const real *__restrict__ uRec,
+                                                real *__restrict__ out)
+{
+    const idx i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m.N)
+        return;
+    const size_t N = m.N;
+    const real isc = m.iscale[i];
+    real r[kLinRow];
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+    {
+        r[v] = u[(size_t)v * N + i];
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+            r[5 + d * 5 + v] = uRec[((size_t)v * 3 + d) * N + i] * isc;
+    }
+    double2 *o = reinterpret_cast<double2 *>(out + (size_t)i * kLinRow);
+#pragma unroll
+    for (int q = 0; q < kLinRow / 2; q++)
+        o[q] = make_double2(r[2 * q], r[2 * q + 1]);
+}
+
+// the cells' constants: rows of 4 (tetrahedra, whose vertex mean is their barycentre: centre, 1 / scale) or
+// of 8 (centre, 1 / scale, scale times moment, 0)
+__global__ void __launch_bounds__(256) kLinCentre(DevMesh m, real *__restrict__ linC, int row)
+{
+    const idx i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= m.N)
+        return;
+    const size_t N = m.N;
+    real *o = linC + (size_t)i * row;
+    for (int r = 0; r < 3; r++)
+        o[r] = m.cent[r * N + i];
+    o[3] = m.iscale[i];
+    for (int r = 4; r < row; r++)
+        o[r] = r < 4 + m.dim ? m.scale[i] * m.moment[(size_t)(r - 4) * N + i] : 0.0;
+}
+// distGRP of an interior face with one normal (EvaluateRHS.hxx:346-424)
+__global__ void __launch_bounds__(256) kLinDist(DevMesh m, real *__restrict__ out)
+{
+    const idx f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= m.F)
+        return;
+    const size_t N = m.N, F = m.F;
+    const idx cL = m.f2c[f], cR = m.f2c[F + f];
+    out[f] = 1;
+    if (cR < 0)
+        return;
+    real dn = 0;
+    for (int r = 0; r < 3; r++)
+        dn += ((m.bary[r * N + cR] - m.fshift[r * F + f]) - m.bary[r * N + cL]) * m.fmeanN[r * F + f];
+    const real d0 = fmin(m.vol[cL], m.vol[cR]) / m.farea[f] * 2;
+    out[f] = 1.0 / fmax(fmin(fabs(dn), d0 * 2), d0 * 0.25);
+}
+
+template <int DIM, bool TRI>
+struct LinSide
+{
+    real u[5], G[DIM][5], c[3], d[DIM];
+    // rec: the cell records (linRec), or null: the rows of u and uRec
+    __device__ __forceinline__ void load(const DevMesh &m, idx i, const real *__restrict__ u_,
+                                         const real *__restrict__ uRec, const real *__restrict__ rec)
+    {
+        const size_t N = m.N;
+#pragma unroll
+        for (int r = 0; r < DIM; r++)
+            d[r] = 0;
+        if (uRec)
+        {
+            const double2 *q = reinterpret_cast<const double2 *>(m.linC + (size_t)i * (TRI ? 4 : 8));
+            const double2 a = q[0], b = q[1];
+            c[0] = a.x, c[1] = a.y, c[2] = b.x;
+            if constexpr (!TRI)
+            {
+                const double2 e = q[2];
+                d[0] = e.x, d[1] = e.y;
+                if constexpr (DIM == 3)
+                    d[DIM - 1] = reinterpret_cast<const real *>(q)[6];
+            }
+            if (TRI && rec)
+            {
+                real r[kLinRow];
+                const double2 *p = reinterpret_cast<const double2 *>(rec + (size_t)i * kLinRow);
+#pragma unroll
+                for (int k = 0; k < kLinRow / 2; k++)
+                {
+                    const double2 t = p[k];
+                    r[2 * k] = t.x, r[2 * k + 1] = t.y;
+                }
+#pragma unroll
+                for (int v = 0; v < 5; v++)
+                {
+                    u[v] = r[v];
+#pragma unroll
+                    for (int k = 0; k < DIM; k++)
+                        G[k][v] = r[5 + k * 5 + v];
+                }
+                return;
+            }
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+            {
+                u[v] = ldu(u_ + (size_t)v * N, (uint32_t)i);
+#pragma unroll
+                for (int k = 0; k < DIM; k++)
+                    G[k][v] = ldu(uRec + ((size_t)v * DIM + k) * N, (uint32_t)i) * b.y;
+            }
+            return;
+        }
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            u[v] = ldu(u_ + (size_t)v * N, (uint32_t)i);
+#pragma unroll
+            for (int k = 0; k < DIM; k++)
+                G[k][v] = 0;
+        }
+        c[0] = c[1] = c[2] = 0;
+    }
+    // the state at x: u + G (x - centre - scale moment), the small offset formed first
+    __device__ __forceinline__ void at(const real *x, real *U) const
+    {
+        real e[DIM];
+#pragma unroll
+        for (int k = 0; k < DIM; k++)
+            e[k] = (x[k] - c[k]) - d[k];
+        along(e, U);
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            U[v] += u[v];
+    }
+    __device__ __forceinline__ void along(const real *e, real *dU) const
+    {
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            real a = 0;
+#pragma unroll
+            for (int k = 0; k < DIM; k++)
+                a += G[k][v] * e[k];
+            dU[v] = a;
+        }
+    }
+};
+
+constexpr real triWeightSum()
+{
+    real s = 0;
+    for (int g = 0; g < 6; g++)
+        s += kTri6[2][g];
+    return s;
+}
+
+// flux forms that read deltaLambdaCell (the H-correction fixes and HLLE+)
+constexpr bool readsDeltaLambda(int rs) { return rs == RS_HLLEP || rs == RS_HLLEP_V1 || rs == RS_Roe_M6 || rs == RS_Roe_M8; }
+
+template <int DIM, int G, int RS, bool BATCH, bool VIS, bool TRI>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
+kRHSFaceLin(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
+            const real *__restrict__ rec, const real *__restrict__ dlc, real *__restrict__ fflux)
+{
+    constexpr bool ONE_N = TRI || DIM == 2; // one normal per face
+    static_assert(ONE_N || !VIS, "quadrilateral faces keep their own viscous pass");
+    constexpr int NS = TRI ? 3 : G;
+    const idx f = xcdTile(blockIdx.x, gridDim.x) * 64 + (idx)threadIdx.x;
+    if (f >= m.F)
+        return;
+    const size_t F = m.F;
+    const uint32_t fu = (uint32_t)f;
+    const idx cL = ldu(m.f2c, fu), cR = ldu(m.f2c + F, fu);
+    // the points (or the vertices of a triangle), the normal and the shift into the right cell's frame
+    real x[NS][3], n[3], sh[3];
+    if constexpr (TRI)
+    {
+        idx nd[3];
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+            nd[k] = ldu(m.face2node + (size_t)k * F, fu);
+#pragma unroll
+        for (int k = 0; k < 3; k++)
+#pragma unroll
+            for (int r = 0; r < 3; r++)
+                x[k][r] = ldu(m.coords + (size_t)r * m.nNode, (uint32_t)nd[k]);
+    }
+    else
+#pragma unroll
+        for (int k = 0; k < NS; k++)
+#pragma unroll
+            for (int r = 0; r < DIM; r++)
+                x[k][r] = ldu(m.fpts + ((size_t)k * 3 + r) * F, fu);
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+    {
+        sh[r] = ldu(m.fshift + (size_t)r * F, fu);
+        if constexpr (ONE_N || BATCH)
+            n[r] = ldu(m.fmeanN + (size_t)r * F, fu);
+    }
+    real wArea = 0, idist = 0;
+    if constexpr (TRI)
+        wArea = ldu(m.farea, fu) * (1.0 / triWeightSum());
+    if constexpr (VIS)
+        idist = ldu(m.linDist, fu);
+    if (cR < 0) // boundary faces: kRHSBoundary and the viscous pass over the boundary list
+        return;
+    real SL[NS][5], SR[NS][5], Gm[DIM][5];
+    RoeBatchFace bf;
+    {
+        LinSide<DIM, TRI> L, R;
+        L.load(m, cL, u, uRec, rec);
+        R.load(m, cR, u, uRec, rec);
+#pragma unroll
+        for (int k = 0; k < NS; k++)
+        {
+            if (TRI && k > 0) // a triangle: the state at its first vertex and its changes along two sides
+            {
+                const real e[3] = {x[k][0] - x[0][0], x[k][1] - x[0][1], x[k][2] - x[0][2]};
+                L.along(e, SL[k]);
+                R.along(e, SR[k]);
+                continue;
+            }
+            real xr[3];
+            L.at(x[k], SL[k]);
+#pragma unroll
+            for (int r = 0; r < DIM; r++)
+                xr[r] = x[k][r] + sh[r];
+            R.at(xr, SR[k]);
+        }
+        if constexpr (VIS)
+#pragma unroll
+            for (int d = 0; d < DIM; d++)
+#pragma unroll
+                for (int v = 0; v < 5; v++)
+                    Gm[d][v] = 0.5 * (L.G[d][v] + R.G[d][v]);
+        if constexpr (BATCH)
+            roeBatchSetup<RS>(L.u, R.u, n, gp,
+                              dlc && readsDeltaLambda(RS) ? fmax(dlc[cL], dlc[cR]) : 0.0, bf);
+        else
+            roeAverage(L.u, R.u, gp.gamma, bf.r);
+    }
+    real dLambda = 0;
+    if constexpr (!BATCH && readsDeltaLambda(RS))
+        if (dlc)
+            dLambda = fmax(dlc[cL], dlc[cR]);
+    const real Cp = cpGas(gp);
+    const ViscGas vg{gp.gamma - 1, Cp, Cp / gp.prGas};
+    // state, weight and (where it varies) normal of point g
+    auto point = [&](int g, real *UL, real *UR, real &wj) {
+        if constexpr (TRI)
+        {
+            const real b1 = kTri6[0][g], b2 = kTri6[1][g];
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+            {
+                UL[v] = SL[0][v] + (b1 * SL[1][v] + b2 * SL[2][v]);
+                UR[v] = SR[0][v] + (b1 * SR[1][v] + b2 * SR[2][v]);
+            }
+            wj = kTri6[2][g] * wArea;
+        }
+        else
+        {
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+                UL[v] = SL[g < NS ? g : 0][v], UR[v] = SR[g < NS ? g : 0][v];
+            wj = ldu(m.fwj + (size_t)g * F, fu);
+            if constexpr (!ONE_N)
+#pragma unroll
+                for (int r = 0; r < 3; r++)
+                    n[r] = ldu(m.fnorm + ((size_t)g * 3 + r) * F, fu);
+        }
+    };
+    real acc[5] = {0, 0, 0, 0, 0};
+    // a triangle's points differ by three constants only: a loop (unrolled, six interleaved fluxes spill)
+#pragma unroll TRI ? 1 : G
+    for (int g = 0; g < G; g++)
+    {
+        real UL[5], UR[5], wj, Fl[5];
+        point(g, UL, UR, wj);
+        if constexpr (BATCH)
+            roeBatchPoint<RS>(UL, UR, n, gp, bf, Fl);
+        else
+        {
+            real l0, l1, l4;
+            riemannFluxR<RS>(UL, UR, bf.r, n, gp, dLambda, Fl, l0, l1, l4);
+        }
+        if constexpr (VIS)
+        {
+            real Fv[5];
+            viscousPointLin<DIM>(gp, vg, UL, UR, Gm, n, idist, Fv);
+#pragma unroll
+            for (int v = 1; v < 5; v++)
+                Fl[v] -= Fv[v];
+        }
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            acc[v] -= Fl[v] * wj;
+    }
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+        stu(fflux + (size_t)v * F, fu, acc[v]);
+}
+
+// with one normal per face the linear pass includes the viscous flux; on a quadrilateral, whose normal
+// and viscous distance vary, the two together need more registers than there are
+bool rhsLinearViscous(const DevMesh &m) { return m.dim == 2 || m.faceType == E_TRI3; }
+bool rhsLinearRule(const DevMesh &m)
+{
+    return m.dim == 2 ? (m.G == 2 || m.G == 3) : (m.faceType == E_TRI3 ? m.G == 6 : m.G == 4);
+}
+
+// mesh constants and the cell records' memory, with the metrics
+void setupLinear(Ctx &c)
+{
+    DevMesh &m = c.m;
+    if (!rhsLinearRule(m))
+        return;
+    if (m.P == 1)
+    {
+        const int row = m.faceType == E_TRI3 ? 4 : 8;
+        m.linC = devAlloc<real>(c, row * (size_t)m.N);
+        kLinCentre<<<gridFor(m.N, 256), 256, 0, c.stream>>>(m, m.linC, row);
+        if (m.faceType == E_TRI3)
+            c.linRec = devAlloc<real>(c, kLinRow * (size_t)m.N);
+    }
+    if (rhsLinearViscous(m))
+    {
+        m.linDist = devAlloc<real>(c, m.F);
+        kLinDist<<<gridFor(m.F, 256), 256, 0, c.stream>>>(m, m.linDist);
+    }
+    DNDSR_HIP_CHECK(hipGetLastError());
+}
+
+struct LinArgs
+{
+    const real *u, *uRec, *rec, *dlc;
+    real *ff;
+};
+template <int DIM, int G, bool TRI, int RS, bool BATCH>
+static void linLaunch(Ctx &c, const GasParams &gp, const LinArgs &a)
+{
+    auto kern = kRHSFaceLin<DIM, G, RS, BATCH, false, TRI>;
+    if constexpr (TRI || DIM == 2)
+        if (gp.viscous)
+            kern = kRHSFaceLin<DIM, G, RS, BATCH, true, TRI>;
+    kern<<<gridFor(c.m.F, 64), 64, 0, c.stream>>>(c.m, gp, a.u, a.uRec, a.rec, a.dlc, a.ff);
+    DNDSR_HIP_CHECK(hipGetLastError());
+    rhsBoundaryLaunch<DIM, DIM + 1, G, RS, BATCH>(c, gp, a.u, a.uRec, a.dlc, a.ff);
+}
+template <int DIM, int G, bool TRI>
+static void linDispatch(Ctx &c, const GasParams &gp, const LinArgs &a)
+{
+    const bool batch = gp.rsMeanValueEig != 0 && gp.rsType >= RS_Roe_M1 && gp.rsType <= RS_Roe_M5;
+#define DNDSR_LIN_CASE(RSV, B)                              \
+    case RSV:                                              \
+        linLaunch<DIM, G, TRI, RSV, B>(c, gp, a);          \
+        break;
+    if (batch)
+        switch (gp.rsType)
+        {
+            DNDSR_LIN_CASE(RS_Roe_M1, true)
+            DNDSR_LIN_CASE(RS_Roe_M2, true)
+            DNDSR_LIN_CASE(RS_Roe_M3, true)
+            DNDSR_LIN_CASE(RS_Roe_M4, true)
+            DNDSR_LIN_CASE(RS_Roe_M5, true)
+        default: throw std::runtime_error("invalid batched Riemann solver");
+        }
+    else
+        switch (gp.rsType)
+        {
+            DNDSR_LIN_CASE(RS_Roe, false)
+            DNDSR_LIN_CASE(RS_HLLC, false)
+            DNDSR_LIN_CASE(RS_HLLEP, false)
+            DNDSR_LIN_CASE(RS_HLLEP_V1, false)
+            DNDSR_LIN_CASE(RS_Roe_M1, false)
+            DNDSR_LIN_CASE(RS_Roe_M2, false)
+            DNDSR_LIN_CASE(RS_Roe_M3, false)
+            DNDSR_LIN_CASE(RS_Roe_M4, false)
+            DNDSR_LIN_CASE(RS_Roe_M5, false)
+            DNDSR_LIN_CASE(RS_Roe_M6, false)
+            DNDSR_LIN_CASE(RS_Roe_M7, false)
+            DNDSR_LIN_CASE(RS_Roe_M8, false)
+        default: throw std::runtime_error("the rs type is invalid");
+        }
+#undef DNDSR_LIN_CASE
+}
+
+void launchRHSFaceLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff,
+                         bool pack)
+{
+    DevMesh &m = c.m;
+    LinArgs a{u, uRec, nullptr, dlc, ff};
+    if (uRec && pack && c.linRec)
+    {
+        kLinPack<<<gridFor(m.N, 256), 256, 0, c.stream>>>(m, u, uRec, c.linRec);
+        DNDSR_HIP_CHECK(hipGetLastError());
+        a.rec = c.linRec;
+    }
+    if (m.dim == 2 && m.G == 2)
+        linDispatch<2, 2, false>(c, gp, a);
+    else if (m.dim == 2)
+        linDispatch<2, 3, false>(c, gp, a);
+    else if (m.faceType == E_TRI3)
+        linDispatch<3, 6, true>(c, gp, a);
+    else
+        linDispatch<3, 4, false>(c, gp, a);
+}
+
+} // namespace dndsr

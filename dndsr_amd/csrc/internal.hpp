@@ -83,6 +83,9 @@ struct DevMesh
     real *moment = nullptr;   // [M][N]
     real *cpts = nullptr;     // [Gc][3][N]
     real *cwj = nullptr;      // [Gc][N]
+    // linear reconstruction (facelin.hip): [N][4] or [N][8] cell constants; [F] the inverse viscous distance
+    // of interior faces with one normal
+    real *linC = nullptr, *linDist = nullptr;
     // VR
     real *AinvB = nullptr;    // [(K+1)*M*M][N]
     real *Ainvb = nullptr;    // [K*M][N]
@@ -123,6 +126,7 @@ struct Ctx
     // scratch owned by the context (grown on demand, freed at destroy)
     real *faceFlux = nullptr;   // [5][F]
     real *vrBnd = nullptr;      // [nVars][M][nBnd] A^-1 BCC of each boundary face (VR sweep boundary term)
+    real *linRec = nullptr;     // [N][20] means and gradients (linear reconstruction on tetrahedra, facelin.hip)
     // the SOR sweep's matrices in list order (vr.hip, sorMatrix): sweeps so far (up to 2), the copy,
     // whether it matches the coefficients, and whether there was no memory for it
     int sorUse = 0;
@@ -232,6 +236,14 @@ struct StageUpdate
 void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *deltaLambdaCell,
                    real *rhs, const StageUpdate *stage = nullptr, real *faceFluxBuf = nullptr,
                    bool flagNonFinite = true);
+// ---- launchers (facelin.hip): fluxes (inviscid and viscous) of the interior faces and inviscid boundary
+// fluxes with a linear or no reconstruction, for the face rules rhsLinearRule names; pack: the
+// context's cell records may be used (else the cell rows are read directly)
+bool rhsLinearRule(const DevMesh &m);
+bool rhsLinearViscous(const DevMesh &m);
+void setupLinear(Ctx &c);
+void launchRHSFaceLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff,
+                         bool pack);
 void launchLUSGSInit(Ctx &c, const real *dTau, real dt, real alphaDiag, const real *lambdaFace, real *jdiag);
 // a sweep of the transposed scalar LU-SGS matrix (the adjoint preconditioner), FP64
 void launchSGSSweepT64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, const real *u, const real *uInc,

@@ -1,0 +1,69 @@
+"""The linear face kernel (maxOrder 1 or no reconstruction) against the oracle on every face rule it
+takes, odd face counts, periodic shifts, boundary faces left to their own passes, viscous or not, and
+flux forms that read deltaLambdaCell or share the face's eigenvalues; on tetrahedra also the entry
+point that reads the cell rows instead of the cell records (bit-identical)."""
+from __future__ import annotations
+
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from helpers import RS, random_rec, random_state, rel_l2
+
+pytestmark = pytest.mark.gpu
+
+GAS = dict(Rgas=1.0, muGas=0.05, prGas=0.72, TRef=1.5, CSutherland=0.4)
+
+
+def _mesh(kind):
+    from dndsr_amd import bc
+    from dndsr_amd import mesh as mm
+    if kind == "tri":
+        return mm.tri_grid(7, 5, 1.0, 1.0, periodic=(True, True), jitter=0.1, seed=3), None
+    if kind == "quad":
+        return mm.periodic_quad_grid(9, 7, 1.0, 0.8, jitter=0.1, seed=3), None
+    if kind == "mixed":
+        return mm.mixed_grid(10, 6, 1.0, 1.0, periodic=(True, False), zones=dict(ymin=0, ymax=1), jitter=0.05,
+                             seed=3), [bc.BC_WALL, bc.BC_SYM]
+    if kind == "hex":
+        return mm.periodic_hex_grid(5, 4, 3, 1.0, 1.0, 1.0, jitter=0.1, seed=3), None
+    return mm.tet_grid(3, 4, 3, 1.0, 1.0, 1.0, periodic=(True, False, True), zones=dict(ymin=0, ymax=1),
+                       jitter=0.05, seed=3), [bc.BC_WALL, bc.BC_WALL_INVIS]
+
+
+@pytest.mark.parametrize("kind,intOrder", [("tri", 3), ("quad", 3), ("quad", 5), ("mixed", 3), ("hex", 3),
+                                           ("tet", 3), ("tet", 4)])
+@pytest.mark.parametrize("rs,batch", [("Roe", 0), ("HLLEP", 0), ("Roe_M1", 1)])
+def test_residual_matches_oracle(require_gpu, kind, intOrder, rs, batch):
+    import pyoracle as po
+    from dndsr_amd import bc
+    from dndsr_amd._lib import check, lib
+    from dndsr_amd.cfv import VariationalReconstruction, _ptr
+    from dndsr_amd.euler import EulerEvaluator
+    print(f"\n[face linear] {kind} intOrder {intOrder} {rs} batch={batch}", flush=True)
+    m, types = _mesh(kind)
+    s = dict(maxOrder=1, intOrder=intOrder)
+    zw = {} if types is None else dict(zoneDirWeight=bc.euler_dir_weights(types, 1))
+    o = po.OracleVR(m, **s, **zw)
+    g = VariationalReconstruction(m, dict(s, **zw)).construct()
+    if types:
+        o.set_bc(types, np.ones((len(types), 5)), 1.4)
+    u, rec = random_state(g.nCell, 5), random_rec(g.nCell, g.M)
+    du, dr, rhs = g.to_device(u), g.to_device(rec), g.BuildUDof(5)
+    for viscous in (False, True):
+        es = po.OracleVR.euler_settings(1.4, RS[rs], batch, 1.0, 1.0, viscous=int(viscous), muModel=1, **GAS)
+        ev = EulerEvaluator(g, dict(riemannSolverType=rs, rsMeanValueEig=batch, viscous=viscous,
+                                    idealGasProperty=dict(GAS, muModel=1),
+                                    **(dict(bcTypes=types, bcValues=np.ones((len(types), 5))) if types else {})))
+        ev.EvaluateDt(g.BuildUDof(1)[0], du, None, CFL=1.0)
+        dlc = o.eval_dt(es, u, 1.0, 1e100, True)[2]
+        for r, d in ((rec, dr), (None, None)):
+            ev.EvaluateRHS(rhs, None, du, d, d)
+            assert rel_l2(g.to_host(rhs), o.eval_rhs(es, u, r, dlc)) <= 1e-12, (viscous, r is None)
+            if kind == "tet":
+                other = g.BuildUDof(5)
+                check(lib().dndsr_eval_rhs_noalloc(ev.ctx.h, C.byref(ev.es), _ptr(du), _ptr(d),
+                                                   _ptr(ev.deltaLambdaCell), _ptr(other)))
+                ev.ctx.sync()
+                assert np.array_equal(g.to_host(rhs), g.to_host(other))
