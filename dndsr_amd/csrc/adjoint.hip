@@ -8,12 +8,12 @@
 //                 deltaLambdaCell frozen; a boundary face takes U_R = ghost(U_L), u_R = ghost(u_L) (at
 //                 the mean normal), G_R = G_L;
 //   VR sweep:     y_i = c0 x_i + c1 sum_k [A^-1B_{i,k} x_j + A^-1b_{i,k} (u_j - u_i)].
-// Flux derivatives come from the templated Riemann solvers evaluated on dual
-// numbers (one pass per input direction), so every branch of the flux is
-// differentiated as executed.  Reconstruction is not stored: the caller passes the
-// same uRec the forward pass used (the Python wrapper recomputes it).
-#include "dual.hpp"
-#include "gas.hpp"
+// Flux derivatives are the reverse passes of gasadj.hpp, ghost states go through dual numbers (five
+// passes of the ghost alone); every branch is differentiated as executed.  Reconstruction is not
+// stored: the caller passes the same uRec the forward pass used (the Python wrapper recomputes it).
+#include <algorithm>
+
+#include "gasadj.hpp"
 #include "internal.hpp"
 
 namespace dndsr
@@ -109,19 +109,172 @@ __device__ inline void cellValGradAt(const DevMesh &m, idx c, const real *x, con
     }
 }
 
-// Point-sensitivity rows (of the buffer pbuf[row][G F]): 0-4 d/dU_L, 5-9 d/dU_R, 10-14
-// d/du_L (cell mean), 15-19 d/du_R, and with viscous fluxes 20-34 d/dG_L[d][v]
-// (row 20 + 5 d + v), 35-49 d/dG_R.
-constexpr int kAdjRowsInv = 20, kAdjRowsVis = 50;
-
-// One thread per (face, point), point-major: t = g F + f.  Writes the 20 sensitivities
-// dF.Fbar / d(UL, UR, uLmean, uRmean) of the point to pbuf[20][G F].
-template <int DIM, int NDOF, int RS, bool BATCH>
-__global__ void __launch_bounds__(128) kRHSPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u,
-                                                    const real *__restrict__ uRec, const real *__restrict__ dlc,
-                                                    const real *__restrict__ fbar, real *__restrict__ pbuf)
+// value, gradient and geometry of an interior face point, shared by the point and face kernels
+template <int DIM, int NDOF>
+struct AdjSide
 {
-    constexpr int M = NDOF - 1;
+    real U[5], phi[NDOF > 1 ? NDOF - 1 : 1], G[3][5];
+    __device__ __forceinline__ void load(const DevMesh &m, idx c, const real *x, const real *shift, const real *um,
+                                         const real *__restrict__ uRec, bool grad)
+    {
+        constexpr int M = NDOF - 1;
+        const size_t N = m.N;
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            U[v] = um[v];
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+                G[d][v] = 0;
+        if (!uRec)
+            return;
+        cellBasisAt<DIM, NDOF>(m, c, x, shift, phi);
+        real dphi[DIM][M > 0 ? M : 1], p2[M > 0 ? M : 1];
+        if (grad)
+        {
+            if constexpr (M == DIM) // linear: d phi_j / d x_d = delta / scale
+            {
+                const real isc = m.iscale[c];
+#pragma unroll
+                for (int d = 0; d < DIM; d++)
+#pragma unroll
+                    for (int j = 0; j < M; j++)
+                        dphi[d][j] = d == j ? isc : 0.0;
+            }
+            else
+                cellBasisGradAt<DIM, NDOF>(m, c, x, shift, p2, dphi);
+        }
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            real s = 0;
+#pragma unroll
+            for (int j = 0; j < M; j++)
+            {
+                const real r = uRec[(size_t)(v * M + j) * N + c];
+                s += phi[j] * r;
+                if (grad)
+                {
+                    if constexpr (M == DIM)
+                        G[j][v] = dphi[j][j] * r;
+                    else
+#pragma unroll
+                        for (int d = 0; d < DIM; d++)
+                            G[d][v] += dphi[d][j] * r;
+                }
+            }
+            U[v] += s;
+        }
+    }
+};
+
+// Sensitivities of an interior face point: s = Fbar . F(U_L, U_R, u_L, u_R) - Fbar . Fv, with respect to the
+// point states (UL, UR), the cell means (mL, mR) and the mean gradient of the two sides (Gb)
+template <int RS, bool BATCH>
+__device__ __forceinline__ void facePointBar(const DevMesh &m, const GasParams &gp, idx f, idx cL, idx cR,
+                                             const real *sh, const real *uL, const real *uR, const real *UL,
+                                             const real *UR, const real (*GL)[5], const real (*GR)[5], const real *n,
+                                             const real *nm, real dLambda, const real *Fbar, bool vis, real *ULb,
+                                             real *URb, real *mLb, real *mRb, real (*Gb)[5])
+{
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+        ULb[v] = URb[v] = mLb[v] = mRb[v] = 0;
+    RoeAve r;
+    RoeBar rb;
+    roeAverage(uL, uR, gp.gamma, r);
+    riemannFluxBar<RS, BATCH>(UL, UR, r, n, nm, gp, dLambda, Fbar, ULb, URb, rb);
+    roeAverageBar(uL, uR, gp.gamma, r, rb, mLb, mRb);
+    if (!vis)
+        return;
+    const size_t N = m.N;
+    real dn = 0, Ga[3][5], Fvb[5];
+#pragma unroll
+    for (int q = 0; q < 3; q++)
+        dn += ((m.bary[(size_t)q * N + cR] - sh[q]) - m.bary[(size_t)q * N + cL]) * n[q];
+    const real d0 = fmin(m.vol[cL], m.vol[cR]) / m.farea[f] * 2;
+    const real idist = 1.0 / fmax(fmin(fabs(dn), d0 * 2), d0 * 0.25);
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+    {
+        Fvb[v] = -Fbar[v];
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+            Ga[d][v] = 0.5 * (GL[d][v] + GR[d][v]);
+    }
+    viscousPointBar(gp, UL, UR, Ga, n, idist, false, Fvb, ULb, URb, Gb);
+}
+
+// The same for a boundary point: the right states are the ghosts of the left ones (the mean's at nm), GR = GL
+template <int RS, bool BATCH>
+__device__ __forceinline__ void bndPointBar(const DevMesh &m, const GasParams &gp, idx f, idx cL, const real *uL,
+                                            const real *UL, const real (*GL)[5], const real *n, const real *nm,
+                                            real dLambda, const real *Fbar, int vis, real *ULb, real *mLb,
+                                            real (*Gb)[5])
+{
+    const int zone = m.fzone[f], type = m.bcType[zone];
+    const real *far = m.bcVal + (size_t)zone * 5;
+    real UR[5], uR[5], URb[5], mRb[5];
+    bcGhost(type, UL, n, far, gp.gamma, UR);
+    bcGhost(type, uL, nm, far, gp.gamma, uR);
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+        ULb[v] = URb[v] = mLb[v] = mRb[v] = 0;
+    RoeAve r;
+    RoeBar rb;
+    roeAverage(uL, uR, gp.gamma, r);
+    riemannFluxBar<RS, BATCH>(UL, UR, r, n, nm, gp, dLambda, Fbar, ULb, URb, rb);
+    roeAverageBar(uL, uR, gp.gamma, r, rb, mLb, mRb);
+#pragma unroll
+    for (int d = 0; d < 3; d++)
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            Gb[d][v] = 0;
+    if (vis && !(type == BC_WALL_INVIS || type == BC_SYM || type == BC_FAR || type == BC_OUT))
+    {
+        const size_t N = m.N, F = m.F;
+        real dn = 0, Fvb[5];
+#pragma unroll
+        for (int q = 0; q < 3; q++)
+            dn += (m.fcent[(size_t)q * F + f] - m.bary[(size_t)q * N + cL]) * n[q];
+        const real d0 = m.vol[cL] / m.farea[f] * 2;
+        const real idist = 1.0 / fmax(fmin(fabs(dn) * 2.0, d0 * 2), d0 * 0.25);
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            Fvb[v] = -Fbar[v];
+        viscousPointBar(gp, UL, UR, GL, n, idist, type == BC_WALL, Fvb, ULb, URb, Gb);
+    }
+    // the ghosts' Jacobians transposed, one column per pass
+#pragma unroll 1
+    for (int c = 0; c < 5; c++)
+    {
+        Dual D[5], E[5], DR[5], ER[5];
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            D[v] = Dual(UL[v], v == c ? 1.0 : 0.0), E[v] = Dual(uL[v], v == c ? 1.0 : 0.0);
+        bcGhost(type, D, n, far, gp.gamma, DR);
+        bcGhost(type, E, nm, far, gp.gamma, ER);
+        real a = 0, b = 0;
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            a += URb[v] * DR[v].d, b += mRb[v] * ER[v].d;
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            if (v == c)
+                ULb[v] += a, mLb[v] += b;
+    }
+}
+
+// Point-sensitivity rows (of the buffer pbuf[row][G F]): 0-4 d/dU_L, 5-9 d/dU_R, 10-14 d/du_L (cell mean),
+// 15-19 d/du_R, and with viscous fluxes 20-34 d/dG[d][v] of the two sides' mean gradient (row 20 + 5 d + v;
+// each side takes half, and a boundary face, whose sides share one gradient, stores twice its value).
+// One thread per (face, point), point-major: t = g F + f.
+template <int DIM, int NDOF, int RS, bool BATCH>
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+kRHSPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
+             const real *__restrict__ dlc, const real *__restrict__ fbar, real *__restrict__ pbuf, int vis)
+{
     const size_t N = m.N, F = m.F, GF = (size_t)m.G * F;
     const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= GF)
@@ -131,151 +284,48 @@ __global__ void __launch_bounds__(128) kRHSPointAdj(DevMesh m, GasParams gp, con
     const idx cL = m.f2c[f], cR = m.f2c[F + f];
     if (cR < 0) // boundary faces: kRHSBndPointAdj
         return;
-    real x[3], n[3], sh[3];
+    real x[3], n[3], nm[3], sh[3], uL[5], uR[5], Fbar[5];
 #pragma unroll
     for (int r = 0; r < 3; r++)
     {
         x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
         n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
         sh[r] = m.fshift[(size_t)r * F + f];
+        nm[r] = BATCH ? m.fmeanN[(size_t)r * F + f] : 0.0;
     }
     const real wj = m.fwj[(size_t)g * F + f];
-    real UL[5], UR[5], uLm[5], uRm[5], Fbar[5];
 #pragma unroll
     for (int v = 0; v < 5; v++)
     {
-        uLm[v] = UL[v] = u[(size_t)v * N + cL];
-        uRm[v] = UR[v] = u[(size_t)v * N + cR];
+        uL[v] = u[(size_t)v * N + cL], uR[v] = u[(size_t)v * N + cR];
         Fbar[v] = -wj * fbar[(size_t)v * F + f];
     }
-    if (uRec)
-    {
-        real phiL[M > 0 ? M : 1], phiR[M > 0 ? M : 1];
-        cellBasisAt<DIM, NDOF>(m, cL, x, nullptr, phiL);
-        cellBasisAt<DIM, NDOF>(m, cR, x, sh, phiR);
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-        {
-            real sL = 0, sR = 0;
-#pragma unroll
-            for (int j = 0; j < M; j++)
-            {
-                sL += phiL[j] * uRec[(size_t)(v * M + j) * N + cL];
-                sR += phiR[j] * uRec[(size_t)(v * M + j) * N + cR];
-            }
-            UL[v] += sL, UR[v] += sR;
-        }
-    }
     const real dLambda = dlc ? fmax(dlc[cL], dlc[cR]) : 0.0;
-    real nm[3];
-    if constexpr (BATCH)
-    {
-#pragma unroll
-        for (int r = 0; r < 3; r++)
-            nm[r] = m.fmeanN[(size_t)r * F + f];
-    }
-#pragma unroll 1
-    for (int d = 0; d < 20; d++)
-    {
-        const int which = d / 5, comp = d % 5;
-        Dual DL[5], DR[5], DLm[5], DRm[5], DF[5];
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-        {
-            DL[v] = Dual(UL[v], which == 0 && v == comp ? 1.0 : 0.0);
-            DR[v] = Dual(UR[v], which == 1 && v == comp ? 1.0 : 0.0);
-            DLm[v] = Dual(uLm[v], which == 2 && v == comp ? 1.0 : 0.0);
-            DRm[v] = Dual(uRm[v], which == 3 && v == comp ? 1.0 : 0.0);
-        }
-        if constexpr (BATCH)
-        {
-            RoeBatchFaceT<Dual> bf;
-            roeBatchSetup<RS>(DLm, DRm, nm, gp, dLambda, bf);
-            roeBatchPoint<RS>(DL, DR, n, gp, bf, DF);
-        }
-        else
-        {
-            Dual l0, l1, l4;
-            riemannFlux<RS>(DL, DR, DLm, DRm, n, gp, dLambda, DF, l0, l1, l4);
-        }
-        real s = 0;
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            s += Fbar[v] * DF[v].d;
-        pbuf[(size_t)d * GF + t] = s;
-    }
-}
-
-// Viscous part of an interior face point: adds d(Fv . Fvbar)/dU_L,R to rows 0-9 and
-// writes the gradient rows 20-49.  Fvbar = -Fbar (the face flux gains +Fv w).
-template <int DIM, int NDOF>
-__global__ void __launch_bounds__(128) kRHSPointAdjVis(DevMesh m, GasParams gp, const real *__restrict__ u,
-                                                       const real *__restrict__ uRec, const real *__restrict__ fbar,
-                                                       real *__restrict__ pbuf)
-{
-    const size_t N = m.N, F = m.F, GF = (size_t)m.G * F;
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= GF)
-        return;
-    const idx f = (idx)(t % F);
-    const int g = (int)(t / F);
-    const idx cL = m.f2c[f], cR = m.f2c[F + f];
-    if (cR < 0)
-        return;
-    real x[3], n[3], sh[3], dB[3];
-#pragma unroll
-    for (int r = 0; r < 3; r++)
-    {
-        x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
-        n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
-        sh[r] = m.fshift[(size_t)r * F + f];
-        dB[r] = (m.bary[(size_t)r * N + cR] - sh[r]) - m.bary[(size_t)r * N + cL];
-    }
-    const real d0 = fmin(m.vol[cL], m.vol[cR]) / m.farea[f] * 2;
-    const real wj = m.fwj[(size_t)g * F + f];
-    real Fvb[5];
+    AdjSide<DIM, NDOF> L, R;
+    L.load(m, cL, x, nullptr, uL, uRec, vis != 0);
+    R.load(m, cR, x, sh, uR, uRec, vis != 0);
+    real a[5], b[5], c[5], d[5], Gb[3][5];
+    facePointBar<RS, BATCH>(m, gp, f, cL, cR, sh, uL, uR, L.U, R.U, L.G, R.G, n, nm, dLambda, Fbar, vis != 0, a, b, c,
+                            d, Gb);
 #pragma unroll
     for (int v = 0; v < 5; v++)
-        Fvb[v] = wj * fbar[(size_t)v * F + f];
-    real UL[5], UR[5], GL[3][5], GR[3][5];
-    cellValGradAt<DIM, NDOF>(m, cL, x, nullptr, u, uRec, UL, GL);
-    cellValGradAt<DIM, NDOF>(m, cR, x, sh, u, uRec, UR, GR);
-#pragma unroll 1
-    for (int d = 0; d < 40; d++)
     {
-        Dual DL[5], DR[5], DGL[3][5], DGR[3][5], DF[5];
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-        {
-            DL[v] = Dual(UL[v], d == v ? 1.0 : 0.0);
-            DR[v] = Dual(UR[v], d == 5 + v ? 1.0 : 0.0);
-#pragma unroll
-            for (int q = 0; q < 3; q++)
-            {
-                DGL[q][v] = Dual(GL[q][v], d == 10 + 5 * q + v ? 1.0 : 0.0);
-                DGR[q][v] = Dual(GR[q][v], d == 25 + 5 * q + v ? 1.0 : 0.0);
-            }
-        }
-        viscousPointFlux(gp, DL, DR, DGL, DGR, n, dB, d0, false, false, DF);
-        real sv = 0;
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            sv += Fvb[v] * DF[v].d;
-        const int row = d < 10 ? d : 20 + (d - 10);
-        if (d < 10)
-            pbuf[(size_t)row * GF + t] += sv;
-        else
-            pbuf[(size_t)row * GF + t] = sv;
+        pbuf[(size_t)v * GF + t] = a[v], pbuf[(size_t)(5 + v) * GF + t] = b[v];
+        pbuf[(size_t)(10 + v) * GF + t] = c[v], pbuf[(size_t)(15 + v) * GF + t] = d[v];
     }
+    if (vis)
+#pragma unroll
+        for (int q = 0; q < DIM; q++)
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+                pbuf[(size_t)(20 + 5 * q + v) * GF + t] = Gb[q][v];
 }
 
-// One thread per (boundary face, point): the sensitivities of the inviscid flux against
-// the ghost states (and of the viscous flux, vis) to the interior point value, cell mean
-// and gradient; the front-side rows are zero.
+// One thread per (boundary face, point): the rows of the back side (the front side has no state of its own)
 template <int DIM, int NDOF, int RS, bool BATCH>
-__global__ void __launch_bounds__(128) kRHSBndPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u,
-                                                       const real *__restrict__ uRec, const real *__restrict__ dlc,
-                                                       const real *__restrict__ fbar, real *__restrict__ pbuf, int vis)
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+kRHSBndPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
+                const real *__restrict__ dlc, const real *__restrict__ fbar, real *__restrict__ pbuf, int vis)
 {
     const size_t N = m.N, F = m.F, GF = (size_t)m.G * F;
     const size_t tb = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -285,85 +335,210 @@ __global__ void __launch_bounds__(128) kRHSBndPointAdj(DevMesh m, GasParams gp, 
     const int g = (int)(tb / m.nBnd);
     const size_t t = (size_t)g * F + f;
     const idx cL = m.f2c[f];
-    const int zone = m.fzone[f], type = m.bcType[zone];
-    const real *far = m.bcVal + (size_t)zone * 5;
-    real x[3], n[3], nm[3], dB[3];
+    real x[3], n[3], nm[3], uL[5], Fbar[5];
 #pragma unroll
     for (int r = 0; r < 3; r++)
     {
         x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
         n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
         nm[r] = m.fmeanN[(size_t)r * F + f];
-        dB[r] = m.fcent[(size_t)r * F + f] - m.bary[(size_t)r * N + cL];
     }
-    const real d0 = m.vol[cL] / m.farea[f] * 2;
     const real wj = m.fwj[(size_t)g * F + f];
-    const real dLambda = dlc ? dlc[cL] : 0.0;
-    real Fbar[5], uLm[5];
 #pragma unroll
     for (int v = 0; v < 5; v++)
-    {
-        Fbar[v] = -wj * fbar[(size_t)v * F + f];
-        uLm[v] = u[(size_t)v * N + cL];
-    }
-    real UL[5], GL[3][5];
-    cellValGradAt<DIM, NDOF>(m, cL, x, nullptr, u, uRec, UL, GL);
-    const bool visFace =
-        vis && !(type == BC_WALL_INVIS || type == BC_SYM || type == BC_FAR || type == BC_OUT);
-    const int nDir = vis ? 25 : 10;
-#pragma unroll 1
-    for (int d = 0; d < nDir; d++)
-    {
-        Dual DL[5], DLm[5], DR[5], DRm[5], DF[5];
+        uL[v] = u[(size_t)v * N + cL], Fbar[v] = -wj * fbar[(size_t)v * F + f];
+    AdjSide<DIM, NDOF> L;
+    L.load(m, cL, x, nullptr, uL, uRec, vis != 0);
+    real a[5], c[5], Gb[3][5];
+    bndPointBar<RS, BATCH>(m, gp, f, cL, uL, L.U, L.G, n, nm, dlc ? dlc[cL] : 0.0, Fbar, vis, a, c, Gb);
 #pragma unroll
-        for (int v = 0; v < 5; v++)
-        {
-            DL[v] = Dual(UL[v], d == v ? 1.0 : 0.0);
-            DLm[v] = Dual(uLm[v], d == 5 + v ? 1.0 : 0.0);
-        }
-        bcGhost(type, DLm, nm, far, gp.gamma, DRm);
-        bcGhost(type, DL, n, far, gp.gamma, DR);
-        if constexpr (BATCH)
-        {
-            RoeBatchFaceT<Dual> bf;
-            roeBatchSetup<RS>(DLm, DRm, nm, gp, dLambda, bf);
-            roeBatchPoint<RS>(DL, DR, n, gp, bf, DF);
-        }
-        else
-        {
-            Dual l0, l1, l4;
-            riemannFlux<RS>(DL, DR, DLm, DRm, n, gp, dLambda, DF, l0, l1, l4);
-        }
-        real sv = 0;
+    for (int v = 0; v < 5; v++)
+        pbuf[(size_t)v * GF + t] = a[v], pbuf[(size_t)(10 + v) * GF + t] = c[v];
+    if (vis)
 #pragma unroll
-        for (int v = 0; v < 5; v++)
-            sv += Fbar[v] * DF[v].d;
-        if (visFace)
-        {
-            Dual DGL[3][5], DV[5];
-#pragma unroll
-            for (int q = 0; q < 3; q++)
-#pragma unroll
-                for (int v = 0; v < 5; v++)
-                    DGL[q][v] = Dual(GL[q][v], d == 10 + 5 * q + v ? 1.0 : 0.0);
-            viscousPointFlux(gp, DL, DR, DGL, DGL, n, dB, d0, true, type == BC_WALL, DV);
+        for (int q = 0; q < DIM; q++)
 #pragma unroll
             for (int v = 0; v < 5; v++)
-                sv -= Fbar[v] * DV[v].d;
+                pbuf[(size_t)(20 + 5 * q + v) * GF + t] = 2 * Gb[q][v];
+}
+
+// ---------------------------------------------------------------------------
+// Linear reconstruction: the point sensitivities of a face are contracted with the basis where they are
+// formed, so a face stores 5 + 5 DIM values per side (30 in 2-D, against 2 x 35 per point) and the cells
+// only add their faces' rows.  A block is 64 faces; wavefront w takes the points w, w + NW, ... and sums
+// them in its own LDS rows (the reverse pass leaves no registers for 30 accumulators), which are then added in
+// wavefront order.  fbuf [2][5 + 5 DIM][F].
+// ---------------------------------------------------------------------------
+template <int DIM>
+constexpr int adjFaceWaves() { return DIM == 2 ? 2 : 3; }
+template <int DIM, int RS, bool BATCH, bool VIS>
+__global__ void __launch_bounds__(64 * adjFaceWaves<DIM>()) __attribute__((amdgpu_waves_per_eu(2)))
+kRHSFaceAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
+            const real *__restrict__ dlc, const real *__restrict__ fbar, real *__restrict__ fbuf)
+{
+    constexpr int NW = adjFaceWaves<DIM>(), Q = 5 + 5 * DIM;
+    __shared__ real sm[NW][2 * Q][64];
+    const int lane = threadIdx.x % 64, w = waveIndex(64);
+    const size_t N = m.N, F = m.F;
+    const idx f0 = xcdTile(blockIdx.x, gridDim.x) * 64, f = f0 + lane;
+    const idx cL = f < m.F ? m.f2c[f] : -1, cR = f < m.F ? m.f2c[F + f] : -1;
+    const bool on = cR >= 0; // boundary faces: kRHSBndFaceAdj
+    for (int g = w; g < m.G; g += NW)
+    {
+        if (!on)
+            continue;
+        real x[3], n[3], nm[3], sh[3], uL[5], uR[5], Fbar[5];
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+        {
+            x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
+            n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
+            sh[r] = m.fshift[(size_t)r * F + f];
+            nm[r] = BATCH ? m.fmeanN[(size_t)r * F + f] : 0.0;
         }
-        const int row = d < 5 ? d : (d < 10 ? 10 + (d - 5) : 20 + (d - 10));
-        pbuf[(size_t)row * GF + t] = sv;
+        const real wj = m.fwj[(size_t)g * F + f];
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            uL[v] = u[(size_t)v * N + cL], uR[v] = u[(size_t)v * N + cR];
+            Fbar[v] = -wj * fbar[(size_t)v * F + f];
+        }
+        const real dLambda = dlc ? fmax(dlc[cL], dlc[cR]) : 0.0;
+        AdjSide<DIM, DIM + 1> L, R;
+        L.load(m, cL, x, nullptr, uL, uRec, VIS);
+        R.load(m, cR, x, sh, uR, uRec, VIS);
+        real a[5], b[5], c[5], d[5], Gb[3][5];
+        facePointBar<RS, BATCH>(m, gp, f, cL, cR, sh, uL, uR, L.U, R.U, L.G, R.G, n, nm, dLambda, Fbar, VIS, a, b, c,
+                                d, Gb);
+        const real hL = 0.5 * m.iscale[cL], hR = 0.5 * m.iscale[cR];
+        const bool first = g == w;
+        auto put = [&](int q, real val) { sm[w][q][lane] = first ? val : sm[w][q][lane] + val; };
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            put(v, a[v] + c[v]);
+            put(Q + v, b[v] + d[v]);
+            if (uRec)
+#pragma unroll
+                for (int j = 0; j < DIM; j++)
+                {
+                    put(5 + v * DIM + j, L.phi[j] * a[v] + (VIS ? hL * Gb[j][v] : 0.0));
+                    put(Q + 5 + v * DIM + j, R.phi[j] * b[v] + (VIS ? hR * Gb[j][v] : 0.0));
+                }
+        }
     }
-    // the front side has no state of its own
+    __syncthreads();
+    if (!on)
+        return;
+    const int nw = m.G < NW ? m.G : NW;
+    for (int q = w; q < 2 * Q; q += NW)
+    {
+        if (!uRec && q % Q >= 5)
+            continue;
+        real s = sm[0][q][lane];
+        for (int k = 1; k < nw; k++)
+            s += sm[k][q][lane];
+        fbuf[(size_t)q * F + f] = s;
+    }
+}
+
+// the boundary faces' rows of the back side, one thread per face
+template <int DIM, int RS, bool BATCH>
+__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
+kRHSBndFaceAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
+               const real *__restrict__ dlc, const real *__restrict__ fbar, real *__restrict__ fbuf, int vis)
+{
+    const idx t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= m.nBnd)
+        return;
+    const size_t N = m.N, F = m.F;
+    const idx f = m.bndFace[t];
+    const idx cL = m.f2c[f];
+    const real isc = m.iscale[cL];
+    real nm[3], uL[5], acc[5], ar[5][DIM];
+#pragma unroll
+    for (int r = 0; r < 3; r++)
+        nm[r] = m.fmeanN[(size_t)r * F + f];
 #pragma unroll
     for (int v = 0; v < 5; v++)
     {
-        pbuf[(size_t)(5 + v) * GF + t] = 0;
-        pbuf[(size_t)(15 + v) * GF + t] = 0;
+        uL[v] = u[(size_t)v * N + cL], acc[v] = 0;
+#pragma unroll
+        for (int j = 0; j < DIM; j++)
+            ar[v][j] = 0;
     }
-    if (vis)
-        for (int q = 0; q < 15; q++)
-            pbuf[(size_t)(35 + q) * GF + t] = 0;
+    const real dLambda = dlc ? dlc[cL] : 0.0;
+    for (int g = 0; g < m.G; g++)
+    {
+        real x[3], n[3], Fbar[5];
+#pragma unroll
+        for (int r = 0; r < 3; r++)
+        {
+            x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
+            n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
+        }
+        const real wj = m.fwj[(size_t)g * F + f];
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            Fbar[v] = -wj * fbar[(size_t)v * F + f];
+        AdjSide<DIM, DIM + 1> L;
+        L.load(m, cL, x, nullptr, uL, uRec, vis != 0);
+        real a[5], c[5], Gb[3][5];
+        bndPointBar<RS, BATCH>(m, gp, f, cL, uL, L.U, L.G, n, nm, dLambda, Fbar, vis, a, c, Gb);
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            acc[v] += a[v] + c[v];
+            if (uRec)
+#pragma unroll
+                for (int j = 0; j < DIM; j++)
+                    ar[v][j] += L.phi[j] * a[v] + isc * Gb[j][v];
+        }
+    }
+#pragma unroll
+    for (int v = 0; v < 5; v++)
+    {
+        fbuf[(size_t)v * F + f] = acc[v];
+        if (uRec)
+#pragma unroll
+            for (int j = 0; j < DIM; j++)
+                fbuf[(size_t)(5 + v * DIM + j) * F + f] = ar[v][j];
+    }
+}
+
+// one thread per cell: the sum of its faces' rows (in slot order)
+template <int DIM, int KM>
+__global__ void __launch_bounds__(256) kRHSGatherAdjLin(DevMesh m, const real *__restrict__ fbuf,
+                                                        real *__restrict__ ubar, real *__restrict__ urecbar)
+{
+    constexpr int Q = 5 + 5 * DIM;
+    const idx i = xcdTile(blockIdx.x, gridDim.x) * (idx)blockDim.x + threadIdx.x;
+    if (i >= m.N)
+        return;
+    const size_t N = m.N, F = m.F;
+    idx f[KM];
+    bool on[KM];
+    size_t base[KM];
+#pragma unroll
+    for (int k = 0; k < KM; k++)
+    {
+        const size_t q = (size_t)(k < m.K ? k : 0) * N + i;
+        f[k] = m.c2f[q];
+        on[k] = k < m.K && f[k] >= 0;
+        base[k] = on[k] ? ((m.c2flag[q] & 1) ? (size_t)Q * F : 0) + f[k] : 0;
+    }
+    const int nq = urecbar ? Q : 5;
+    for (int q = 0; q < nq; q++)
+    {
+        real r[KM], s = 0;
+#pragma unroll
+        for (int k = 0; k < KM; k++)
+            r[k] = fbuf[base[k] + (size_t)q * F];
+#pragma unroll
+        for (int k = 0; k < KM; k++)
+            s += on[k] ? r[k] : 0.0;
+        (q < 5 ? ubar + (size_t)q * N : urecbar + (size_t)(q - 5) * N)[i] = s;
+    }
 }
 
 // One thread per cell: collect the point sensitivities of the cell's faces into
@@ -389,7 +564,7 @@ __global__ void __launch_bounds__(128) kRHSGatherAdj(DevMesh m, const real *__re
         if (f < 0)
             continue;
         const bool back = m.f2c[f] == i;
-        const int rowU = back ? 0 : 5, rowM = back ? 10 : 15, rowG = back ? 20 : 35;
+        const int rowU = back ? 0 : 5, rowM = back ? 10 : 15;
         real sh[3];
 #pragma unroll
         for (int r = 0; r < 3; r++)
@@ -425,7 +600,7 @@ __global__ void __launch_bounds__(128) kRHSGatherAdj(DevMesh m, const real *__re
 #pragma unroll
                         for (int v = 0; v < 5; v++)
                         {
-                            const real gg = pbuf[(size_t)(rowG + 5 * d + v) * GF + t];
+                            const real gg = 0.5 * pbuf[(size_t)(20 + 5 * d + v) * GF + t];
 #pragma unroll
                             for (int j = 0; j < M; j++)
                                 ar[v][j] += dphi[d][j] * gg;
@@ -460,31 +635,55 @@ __global__ void __launch_bounds__(256) kFaceBar(DevMesh m, const real *__restric
                                           : rbar[(size_t)v * N + cL] / m.vol[cL];
 }
 
+// values of the sensitivity buffer for this mesh
+size_t adjBufferSize(const DevMesh &m, bool viscous)
+{
+    const size_t point = (size_t)(viscous ? 35 : 20) * m.G, face = 2 * (5 + 5 * m.dim);
+    return std::max(point, face) * m.F;
+}
+
+// rbar: the face-flux adjoint [5][F], formed by launchEvalRHSVJP
 template <int DIM, int NDOF, int RS, bool BATCH>
 static void rhsAdjLaunch(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc,
                          const real *rbar, real *ubar, real *urecbar)
 {
-    const size_t GF = (size_t)c.m.G * c.m.F;
+    const DevMesh &m = c.m;
     const int vis = gp.viscous ? 1 : 0;
-    kRHSPointAdj<DIM, NDOF, RS, BATCH><<<(unsigned)((GF + 127) / 128), 128, 0, c.stream>>>(c.m, gp, u, uRec, dlc,
-                                                                                          rbar, c.adjPoint);
-    // (rbar here is the face-flux adjoint [5][F], formed by launchEvalRHSVJP)
+    if constexpr (NDOF == DIM + 1)
+    {
+        const int g = gridFor(m.F, 64), bs = 64 * adjFaceWaves<DIM>();
+        if (vis)
+            kRHSFaceAdj<DIM, RS, BATCH, true><<<g, bs, 0, c.stream>>>(m, gp, u, uRec, dlc, rbar, c.adjPoint);
+        else
+            kRHSFaceAdj<DIM, RS, BATCH, false><<<g, bs, 0, c.stream>>>(m, gp, u, uRec, dlc, rbar, c.adjPoint);
+        DNDSR_HIP_CHECK(hipGetLastError());
+        if (m.nBnd > 0)
+        {
+            kRHSBndFaceAdj<DIM, RS, BATCH><<<gridFor(m.nBnd, 64), 64, 0, c.stream>>>(m, gp, u, uRec, dlc, rbar,
+                                                                                     c.adjPoint, vis);
+            DNDSR_HIP_CHECK(hipGetLastError());
+        }
+        const int cb = cellBlock(m.N), gc = gridFor(m.N, cb);
+        if (m.K <= 4)
+            kRHSGatherAdjLin<DIM, 4><<<gc, cb, 0, c.stream>>>(m, c.adjPoint, ubar, uRec ? urecbar : nullptr);
+        else
+            kRHSGatherAdjLin<DIM, kMaxFC><<<gc, cb, 0, c.stream>>>(m, c.adjPoint, ubar, uRec ? urecbar : nullptr);
+        DNDSR_HIP_CHECK(hipGetLastError());
+        return;
+    }
+    const size_t GF = (size_t)m.G * m.F;
+    kRHSPointAdj<DIM, NDOF, RS, BATCH><<<(unsigned)((GF + 127) / 128), 128, 0, c.stream>>>(m, gp, u, uRec, dlc, rbar,
+                                                                                          c.adjPoint, vis);
     DNDSR_HIP_CHECK(hipGetLastError());
-    if (vis)
+    if (m.nBnd > 0)
     {
-        kRHSPointAdjVis<DIM, NDOF><<<(unsigned)((GF + 127) / 128), 128, 0, c.stream>>>(c.m, gp, u, uRec, rbar,
-                                                                                      c.adjPoint);
-        DNDSR_HIP_CHECK(hipGetLastError());
-    }
-    if (c.m.nBnd > 0)
-    {
-        const size_t nb = (size_t)c.m.nBnd * c.m.G;
+        const size_t nb = (size_t)m.nBnd * m.G;
         kRHSBndPointAdj<DIM, NDOF, RS, BATCH><<<(unsigned)((nb + 127) / 128), 128, 0, c.stream>>>(
-            c.m, gp, u, uRec, dlc, rbar, c.adjPoint, vis);
+            m, gp, u, uRec, dlc, rbar, c.adjPoint, vis);
         DNDSR_HIP_CHECK(hipGetLastError());
     }
-    kRHSGatherAdj<DIM, NDOF><<<gridFor(c.m.N, 128), 128, 0, c.stream>>>(c.m, c.adjPoint, ubar, urecbar,
-                                                                        vis && uRec != nullptr);
+    kRHSGatherAdj<DIM, NDOF><<<gridFor(m.N, 128), 128, 0, c.stream>>>(m, c.adjPoint, ubar, urecbar,
+                                                                      vis && uRec != nullptr);
     DNDSR_HIP_CHECK(hipGetLastError());
 }
 
@@ -644,9 +843,9 @@ __global__ void __launch_bounds__(128) kVRIterT(DevMesh m, const real *__restric
 // Transposed boundary term of the VR sweep (forward: uRecNew_i += scale A_i^-1 BCC_i,
 // BCC_i = sum_{boundary faces, g} phi(x_g) (w0^2 (u_B(x_g) - u_i)) w_g JDet_g, u_B the ghost
 // of the compressed point state u_i + phi . uRec_i, or the given point value).  One
-// thread per boundary cell; BCCbar = scale A^-T ybar, then the derivatives of BCC to the
-// cell's mean and coefficients from dual-number passes (point values given: to the mean
-// only), added to ubar / xbar.
+// thread per boundary cell; BCCbar = scale A^-T ybar, then per point the adjoint of u_B - u_i and
+// through the ghost's Jacobian (five dual-number passes of the ghost) of the point state, i.e. of the
+// cell's mean and coefficients (point values given: of the mean only), added to ubar / xbar.
 template <int DIM, int NDOF, int NV>
 __global__ void __launch_bounds__(64) kVRBoundaryT(DevMesh m, const real *__restrict__ uRec,
                                                    const real *__restrict__ u, const real *__restrict__ ybar,
@@ -682,73 +881,104 @@ __global__ void __launch_bounds__(64) kVRBoundaryT(DevMesh m, const real *__rest
     for (int v = 0; v < NV; v++)
         um[v] = u[(size_t)v * N + i];
     const bool euler = NV == 5 && m.bcType != nullptr;
-    const int nDir = euler ? NV + NV * M : NV;
-#pragma unroll 1
-    for (int d = 0; d < nDir; d++)
+    real ub[NV], xb[NV][M];
+#pragma unroll
+    for (int v = 0; v < NV; v++)
     {
-        real total = 0;
-        for (int k = 0; k < m.K; k++)
+        ub[v] = 0;
+#pragma unroll
+        for (int j = 0; j < M; j++)
+            xb[v][j] = 0;
+    }
+    for (int k = 0; k < m.K; k++)
+    {
+        const idx f = m.c2f[(size_t)k * N + i];
+        if (f < 0 || m.c2c[(size_t)k * N + i] >= 0)
+            continue;
+        const int zone = m.fzone[f];
+        const real w0 = m.faceW[f];
+        for (int g = 0; g < m.G; g++)
         {
-            const idx f = m.c2f[(size_t)k * N + i];
-            if (f < 0 || m.c2c[(size_t)k * N + i] >= 0)
-                continue;
-            const int zone = m.fzone[f];
-            const real w0 = m.faceW[f];
-            const real w2 = w0 * w0;
-            for (int g = 0; g < m.G; g++)
+            real xs[3], phi[M], tv[NV];
+#pragma unroll
+            for (int r = 0; r < 3; r++)
             {
-                real xs[3], phi[M];
+                xs[r] = m.fpts[((size_t)g * 3 + r) * F + f] - cen[r];
+                if (DIM == 3 || r < 2)
+                    xs[r] *= isc;
+            }
+            basisRow0<DIM, NDOF>(xs, mom, phi);
+            const real fac = m.fwj[(size_t)g * F + f] * (w0 * w0);
+            // BCC_j += phi_j inc fac: the adjoint of inc
 #pragma unroll
-                for (int r = 0; r < 3; r++)
-                {
-                    xs[r] = m.fpts[((size_t)g * 3 + r) * F + f] - cen[r];
-                    if (DIM == 3 || r < 2)
-                        xs[r] *= isc;
-                }
-                basisRow0<DIM, NDOF>(xs, mom, phi);
-                const real fac = m.fwj[(size_t)g * F + f];
-                real incd[NV]; // d inc / d (direction d)
-                if (euler)
-                {
-                    Dual umD[5], uBL[5], ULf[5], uB[5];
-                    real n[3];
-#pragma unroll
-                    for (int v = 0; v < 5; v++)
-                    {
-                        umD[v] = Dual(um[v], d == v ? 1.0 : 0.0);
-                        Dual r = 0;
-#pragma unroll
-                        for (int j = 0; j < M; j++)
-                            r += phi[j] * Dual(uRec[((size_t)v * M + j) * N + i], d == NV + v * M + j ? 1.0 : 0.0);
-                        uBL[v] = r;
-                    }
-#pragma unroll
-                    for (int r = 0; r < 3; r++)
-                        n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
-                    compressRecPart(umD, uBL, ULf);
-                    bcGhost(m.bcType[zone], ULf, n, m.bcVal + (size_t)zone * 5, m.bcGamma, uB);
-#pragma unroll
-                    for (int v = 0; v < NV; v++)
-                        incd[v] = (uB[v] - umD[v]).d;
-                }
-                else
-#pragma unroll
-                    for (int v = 0; v < NV; v++)
-                        incd[v] = d == v ? -1.0 : 0.0; // given point values: inc = value - u_i
+            for (int v = 0; v < NV; v++)
+            {
+                real q = 0;
 #pragma unroll
                 for (int j = 0; j < M; j++)
+                    q += Bb[j][v] * phi[j];
+                tv[v] = q * fac;
+                ub[v] -= tv[v]; // inc = uB - u_i (given point values: value - u_i)
+            }
+            if (!euler)
+                continue;
+            real uBL[5], ULf[5], n[3];
 #pragma unroll
-                    for (int v = 0; v < NV; v++)
-                        total += Bb[j][v] * (((phi[j] * incd[v]) * w2) * fac);
+            for (int v = 0; v < 5; v++)
+            {
+                real r = 0;
+#pragma unroll
+                for (int j = 0; j < M; j++)
+                    r += phi[j] * uRec[((size_t)v * M + j) * N + i];
+                uBL[v] = r;
+            }
+#pragma unroll
+            for (int r = 0; r < 3; r++)
+                n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
+            // compressRecPart keeps the point state or falls back to the mean
+            real full[5];
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+                full[v] = um[v] + uBL[v];
+            compressRecPart(um, uBL, ULf);
+            bool kept = true;
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+                kept = kept && !(ULf[v] != full[v]);
+#pragma unroll 1
+            for (int c = 0; c < 5; c++)
+            {
+                Dual D[5], B[5];
+#pragma unroll
+                for (int v = 0; v < 5; v++)
+                    D[v] = Dual(ULf[v], v == c ? 1.0 : 0.0);
+                bcGhost(m.bcType[zone], D, n, m.bcVal + (size_t)zone * 5, m.bcGamma, B);
+                real q = 0;
+#pragma unroll
+                for (int v = 0; v < 5; v++)
+                    q += tv[v < NV ? v : 0] * B[v].d;
+#pragma unroll
+                for (int v = 0; v < NV; v++)
+                    if (v == c)
+                    {
+                        ub[v] += q;
+                        if (kept)
+#pragma unroll
+                            for (int j = 0; j < M; j++)
+                                xb[v][j] += phi[j] * q;
+                    }
             }
         }
-        if (d < NV)
-        {
-            if (ubar)
-                ubar[(size_t)d * N + i] += total;
-        }
-        else if (xbar)
-            xbar[(size_t)(d - NV) * N + i] += total;
+    }
+#pragma unroll
+    for (int v = 0; v < NV; v++)
+    {
+        if (ubar)
+            ubar[(size_t)v * N + i] += ub[v];
+        if (xbar && euler)
+#pragma unroll
+            for (int j = 0; j < M; j++)
+                xbar[((size_t)v * M + j) * N + i] += xb[v][j];
     }
 }
 

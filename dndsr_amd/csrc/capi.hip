@@ -105,6 +105,19 @@ static LinWork &linWork(dndsr_ctx *ctx, int k, bool fp32)
     return w;
 }
 
+// sensitivity and face-flux adjoint buffers of the residual's transpose
+static void adjointWork(Ctx &c, bool viscous)
+{
+    const size_t n = adjBufferSize(c.m, viscous);
+    if (c.adjPointCap < n)
+    {
+        c.adjPoint = devAlloc<real>(c, n);
+        c.adjPointCap = n;
+    }
+    if (!c.adjFaceBar)
+        c.adjFaceBar = devAlloc<real>(c, (size_t)5 * c.m.F);
+}
+
 // FP32 copies of the state, diagonal and face eigenvalues for an FP32 preconditioner
 static void fp32State(dndsr_ctx *ctx)
 {
@@ -1591,14 +1604,7 @@ int dndsr_eval_rhs_vjp(dndsr_ctx *ctx, const dndsr_euler_settings *es, const dou
     need(!uRecBar || uRec, "uRecBar needs uRec");
     Ctx &c = ctx->c;
     need(c.m.nBnd == 0 || c.m.bcType, "the mesh has boundary faces: set the boundary conditions first (dndsr_set_bc)");
-    const int rows = es->viscous ? 50 : 20;
-    if (c.adjPointRows < rows)
-    {
-        c.adjPoint = devAlloc<real>(c, (size_t)rows * c.m.G * c.m.F);
-        c.adjPointRows = rows;
-    }
-    if (!c.adjFaceBar)
-        c.adjFaceBar = devAlloc<real>(c, (size_t)5 * c.m.F);
+    adjointWork(c, es->viscous != 0);
     launchEvalRHSVJP(c, toGas(es), u, uRec, deltaLambdaCell, rhsBar, uBar, uRec ? uRecBar : nullptr);
     CAPI_END
 }
@@ -1635,14 +1641,7 @@ int dndsr_zone_force_vjp(dndsr_ctx *ctx, const dndsr_euler_settings *es, const d
     Ctx &c = ctx->c;
     need(zone >= 0 && zone < c.m.nBCZone, "zone out of range");
     need(c.m.bcType, "the mesh has boundary faces: set the boundary conditions first (dndsr_set_bc)");
-    const int rows = es->viscous ? 50 : 20;
-    if (c.adjPointRows < rows)
-    {
-        c.adjPoint = devAlloc<real>(c, (size_t)rows * c.m.G * c.m.F);
-        c.adjPointRows = rows;
-    }
-    if (!c.adjFaceBar)
-        c.adjFaceBar = devAlloc<real>(c, (size_t)5 * c.m.F);
+    adjointWork(c, es->viscous != 0);
     for (int d = 0; d < 3; d++)
         c.hostRed[d] = forceBar[d];
     real *dev = c.red + 5 * ((size_t)gridFor(c.m.N, 256) + c.m.nColor + 5);

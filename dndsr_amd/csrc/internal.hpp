@@ -137,8 +137,8 @@ struct Ctx
     size_t redCap = 0;
     real *hostRed = nullptr;    // pinned host mirror of reductions
     real *faceLamTmp = nullptr; // [2][F] (lambdaFace, deltaLambdaFace)
-    real *adjPoint = nullptr;   // [20 or 50][G F] point sensitivities of the RHS adjoint
-    int adjPointRows = 0;
+    real *adjPoint = nullptr;   // point or face sensitivities of the RHS adjoint (adjBufferSize values)
+    size_t adjPointCap = 0;
     real *adjFaceBar = nullptr; // [5][F] face-flux adjoint
     real *adj2ndQ = nullptr;    // [5][3][N] per-cell weights of the transposed second-order substitute
     real *adjRhs = nullptr;     // [5][N] residual of a functional's forward evaluation
@@ -367,6 +367,7 @@ void applyLUSGSPrecond(Ctx &c, const GasParams &gp, const LinWork &w, const real
 int gmresSolve(Ctx &c, const GasParams &gp, const LinWork &w, const real *b, real *x, int kSub, int nRestart,
                double *residualOut);
 // ---- launchers (adjoint.hip)
+size_t adjBufferSize(const DevMesh &m, bool viscous);
 // faceBar (optional, [5][F]): the adjoint of the face fluxes instead of the residual's
 // (rbar unused then); without it the face adjoint is formed from rbar
 void launchEvalRHSVJP(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc,
