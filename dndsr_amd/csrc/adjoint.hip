@@ -8,8 +8,8 @@
 //                 deltaLambdaCell frozen; a boundary face takes U_R = ghost(U_L), u_R = ghost(u_L) (at
 //                 the mean normal), G_R = G_L;
 //   VR sweep:     y_i = c0 x_i + c1 sum_k [A^-1B_{i,k} x_j + A^-1b_{i,k} (u_j - u_i)].
-// Flux derivatives are the reverse passes of gasadj.hpp, ghost states go through dual numbers (five
-// passes of the ghost alone); every branch is differentiated as executed.  Reconstruction is not
+// Derivatives of fluxes and ghost states are the reverse passes of gasadj.hpp; every branch is
+// differentiated as executed.  Reconstruction is not
 // stored: the caller passes the same uRec the forward pass used (the Python wrapper recomputes it).
 #include <algorithm>
 
@@ -25,19 +25,19 @@ __device__ inline void cellBasisAt(const DevMesh &m, idx c, const real *x, const
 {
     constexpr int M = NDOF - 1;
     const size_t N = m.N;
-    const real isc = m.iscale[c];
+    const real isc = ldu(m.iscale, (uint32_t)c);
     real xs[3], mom[M > 0 ? M : 1];
 #pragma unroll
     for (int r = 0; r < 3; r++)
     {
         real p = x[r] + (shift ? shift[r] : 0.0);
-        xs[r] = p - m.cent[(size_t)r * N + c];
+        xs[r] = p - ldu(m.cent + (size_t)r * N, (uint32_t)c);
         if (DIM == 3 || r < 2)
             xs[r] *= isc;
     }
 #pragma unroll
     for (int j = 0; j < M; j++)
-        mom[j] = m.moment[(size_t)j * N + c];
+        mom[j] = ldu(m.moment + (size_t)j * N, (uint32_t)c);
     basisRow0<DIM, NDOF>(xs, mom, phi);
 }
 
@@ -49,18 +49,18 @@ __device__ inline void cellBasisGradAt(const DevMesh &m, idx c, const real *x, c
 {
     constexpr int M = NDOF - 1;
     const size_t N = m.N;
-    const real s = m.scale[c];
+    const real s = ldu(m.scale, (uint32_t)c);
     real xs[3];
 #pragma unroll
     for (int r = 0; r < 3; r++)
-        xs[r] = (x[r] + (shift ? shift[r] : 0.0)) - m.cent[(size_t)r * N + c];
+        xs[r] = (x[r] + (shift ? shift[r] : 0.0)) - ldu(m.cent + (size_t)r * N, (uint32_t)c);
     xs[0] /= s, xs[1] /= s;
     if (DIM == 3)
         xs[2] /= s;
 #pragma unroll
     for (int j = 0; j < M; j++)
     {
-        phi[j] = basisDiff(DIM, 0, j + 1, xs, s) - m.moment[(size_t)j * N + c];
+        phi[j] = basisDiff(DIM, 0, j + 1, xs, s) - ldu(m.moment + (size_t)j * N, (uint32_t)c);
 #pragma unroll
         for (int d = 0; d < DIM; d++)
             dphi[d][j] = basisDiff(DIM, 1 + d, j + 1, xs, s);
@@ -96,7 +96,7 @@ __device__ inline void cellValGradAt(const DevMesh &m, idx c, const real *x, con
 #pragma unroll
         for (int j = 0; j < M; j++)
         {
-            const real r = uRec[(size_t)(v * M + j) * N + c];
+            const real r = ldu(uRec + (size_t)(v * M + j) * N, (uint32_t)c);
             a += phi[j] * r;
 #pragma unroll
             for (int d = 0; d < DIM; d++)
@@ -135,7 +135,7 @@ struct AdjSide
         {
             if constexpr (M == DIM) // linear: d phi_j / d x_d = delta / scale
             {
-                const real isc = m.iscale[c];
+                const real isc = ldu(m.iscale, (uint32_t)c);
 #pragma unroll
                 for (int d = 0; d < DIM; d++)
 #pragma unroll
@@ -152,7 +152,7 @@ struct AdjSide
 #pragma unroll
             for (int j = 0; j < M; j++)
             {
-                const real r = uRec[(size_t)(v * M + j) * N + c];
+                const real r = ldu(uRec + (size_t)(v * M + j) * N, (uint32_t)c);
                 s += phi[j] * r;
                 if (grad)
                 {
@@ -169,14 +169,12 @@ struct AdjSide
     }
 };
 
-// Sensitivities of an interior face point: s = Fbar . F(U_L, U_R, u_L, u_R) - Fbar . Fv, with respect to the
-// point states (UL, UR), the cell means (mL, mR) and the mean gradient of the two sides (Gb)
+// Sensitivities of an interior face point: Fbar . F(U_L, U_R, u_L, u_R) with respect to the point states
+// (ULb, URb) and the cell means (mLb, mRb)
 template <int RS, bool BATCH>
-__device__ __forceinline__ void facePointBar(const DevMesh &m, const GasParams &gp, idx f, idx cL, idx cR,
-                                             const real *sh, const real *uL, const real *uR, const real *UL,
-                                             const real *UR, const real (*GL)[5], const real (*GR)[5], const real *n,
-                                             const real *nm, real dLambda, const real *Fbar, bool vis, real *ULb,
-                                             real *URb, real *mLb, real *mRb, real (*Gb)[5])
+__device__ __forceinline__ void facePointBar(const GasParams &gp, const real *uL, const real *uR, const real *UL,
+                                             const real *UR, const real *n, const real *nm, real dLambda,
+                                             const real *Fbar, real *ULb, real *URb, real *mLb, real *mRb)
 {
 #pragma unroll
     for (int v = 0; v < 5; v++)
@@ -186,14 +184,19 @@ __device__ __forceinline__ void facePointBar(const DevMesh &m, const GasParams &
     roeAverage(uL, uR, gp.gamma, r);
     riemannFluxBar<RS, BATCH>(UL, UR, r, n, nm, gp, dLambda, Fbar, ULb, URb, rb);
     roeAverageBar(uL, uR, gp.gamma, r, rb, mLb, mRb);
-    if (!vis)
-        return;
+}
+// -Fbar . Fv with respect to the point states (added) and the mean gradient of the two sides (Gb)
+__device__ __forceinline__ void facePointVisBar(const DevMesh &m, const GasParams &gp, idx f, idx cL, idx cR,
+                                                const real *sh, const real *UL, const real *UR, const real (*GL)[5],
+                                                const real (*GR)[5], const real *n, const real *Fbar, real *ULb,
+                                                real *URb, real (*Gb)[5])
+{
     const size_t N = m.N;
     real dn = 0, Ga[3][5], Fvb[5];
 #pragma unroll
     for (int q = 0; q < 3; q++)
-        dn += ((m.bary[(size_t)q * N + cR] - sh[q]) - m.bary[(size_t)q * N + cL]) * n[q];
-    const real d0 = fmin(m.vol[cL], m.vol[cR]) / m.farea[f] * 2;
+        dn += ((ldu(m.bary + (size_t)q * N, (uint32_t)cR) - sh[q]) - ldu(m.bary + (size_t)q * N, (uint32_t)cL)) * n[q];
+    const real d0 = fmin(ldu(m.vol, (uint32_t)cL), ldu(m.vol, (uint32_t)cR)) / ldu(m.farea, (uint32_t)f) * 2;
     const real idist = 1.0 / fmax(fmin(fabs(dn), d0 * 2), d0 * 0.25);
 #pragma unroll
     for (int v = 0; v < 5; v++)
@@ -237,33 +240,16 @@ __device__ __forceinline__ void bndPointBar(const DevMesh &m, const GasParams &g
         real dn = 0, Fvb[5];
 #pragma unroll
         for (int q = 0; q < 3; q++)
-            dn += (m.fcent[(size_t)q * F + f] - m.bary[(size_t)q * N + cL]) * n[q];
-        const real d0 = m.vol[cL] / m.farea[f] * 2;
+            dn += (m.fcent[(size_t)q * F + f] - ldu(m.bary + (size_t)q * N, (uint32_t)cL)) * n[q];
+        const real d0 = ldu(m.vol, (uint32_t)cL) / ldu(m.farea, (uint32_t)f) * 2;
         const real idist = 1.0 / fmax(fmin(fabs(dn) * 2.0, d0 * 2), d0 * 0.25);
 #pragma unroll
         for (int v = 0; v < 5; v++)
             Fvb[v] = -Fbar[v];
         viscousPointBar(gp, UL, UR, GL, n, idist, type == BC_WALL, Fvb, ULb, URb, Gb);
     }
-    // the ghosts' Jacobians transposed, one column per pass
-#pragma unroll 1
-    for (int c = 0; c < 5; c++)
-    {
-        Dual D[5], E[5], DR[5], ER[5];
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            D[v] = Dual(UL[v], v == c ? 1.0 : 0.0), E[v] = Dual(uL[v], v == c ? 1.0 : 0.0);
-        bcGhost(type, D, n, far, gp.gamma, DR);
-        bcGhost(type, E, nm, far, gp.gamma, ER);
-        real a = 0, b = 0;
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            a += URb[v] * DR[v].d, b += mRb[v] * ER[v].d;
-#pragma unroll
-        for (int v = 0; v < 5; v++)
-            if (v == c)
-                ULb[v] += a, mLb[v] += b;
-    }
+    bcGhostBar(type, UL, n, far, gp.gamma, URb, ULb);
+    bcGhostBar(type, uL, nm, far, gp.gamma, mRb, mLb);
 }
 
 // Point-sensitivity rows (of the buffer pbuf[row][G F]): 0-4 d/dU_L, 5-9 d/dU_R, 10-14 d/du_L (cell mean),
@@ -271,7 +257,7 @@ __device__ __forceinline__ void bndPointBar(const DevMesh &m, const GasParams &g
 // each side takes half, and a boundary face, whose sides share one gradient, stores twice its value).
 // One thread per (face, point), point-major: t = g F + f.
 template <int DIM, int NDOF, int RS, bool BATCH>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1)))
 kRHSPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
              const real *__restrict__ dlc, const real *__restrict__ fbar, real *__restrict__ pbuf, int vis)
 {
@@ -288,25 +274,26 @@ kRHSPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__
 #pragma unroll
     for (int r = 0; r < 3; r++)
     {
-        x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
-        n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
-        sh[r] = m.fshift[(size_t)r * F + f];
-        nm[r] = BATCH ? m.fmeanN[(size_t)r * F + f] : 0.0;
+        x[r] = ldu(m.fpts + ((size_t)g * 3 + r) * F, (uint32_t)f);
+        n[r] = ldu(m.fnorm + ((size_t)g * 3 + r) * F, (uint32_t)f);
+        sh[r] = ldu(m.fshift + (size_t)r * F, (uint32_t)f);
+        nm[r] = BATCH ? ldu(m.fmeanN + (size_t)r * F, (uint32_t)f) : 0.0;
     }
-    const real wj = m.fwj[(size_t)g * F + f];
+    const real wj = ldu(m.fwj + (size_t)g * F, (uint32_t)f);
 #pragma unroll
     for (int v = 0; v < 5; v++)
     {
-        uL[v] = u[(size_t)v * N + cL], uR[v] = u[(size_t)v * N + cR];
-        Fbar[v] = -wj * fbar[(size_t)v * F + f];
+        uL[v] = ldu(u + (size_t)v * N, (uint32_t)cL), uR[v] = ldu(u + (size_t)v * N, (uint32_t)cR);
+        Fbar[v] = -wj * ldu(fbar + (size_t)v * F, (uint32_t)f);
     }
     const real dLambda = dlc ? fmax(dlc[cL], dlc[cR]) : 0.0;
     AdjSide<DIM, NDOF> L, R;
     L.load(m, cL, x, nullptr, uL, uRec, vis != 0);
     R.load(m, cR, x, sh, uR, uRec, vis != 0);
     real a[5], b[5], c[5], d[5], Gb[3][5];
-    facePointBar<RS, BATCH>(m, gp, f, cL, cR, sh, uL, uR, L.U, R.U, L.G, R.G, n, nm, dLambda, Fbar, vis != 0, a, b, c,
-                            d, Gb);
+    facePointBar<RS, BATCH>(gp, uL, uR, L.U, R.U, n, nm, dLambda, Fbar, a, b, c, d);
+    if (vis)
+        facePointVisBar(m, gp, f, cL, cR, sh, L.U, R.U, L.G, R.G, n, Fbar, a, b, Gb);
 #pragma unroll
     for (int v = 0; v < 5; v++)
     {
@@ -323,7 +310,7 @@ kRHSPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__
 
 // One thread per (boundary face, point): the rows of the back side (the front side has no state of its own)
 template <int DIM, int NDOF, int RS, bool BATCH>
-__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(128) __attribute__((amdgpu_waves_per_eu(1)))
 kRHSBndPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
                 const real *__restrict__ dlc, const real *__restrict__ fbar, real *__restrict__ pbuf, int vis)
 {
@@ -339,14 +326,14 @@ kRHSBndPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real 
 #pragma unroll
     for (int r = 0; r < 3; r++)
     {
-        x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
-        n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
-        nm[r] = m.fmeanN[(size_t)r * F + f];
+        x[r] = ldu(m.fpts + ((size_t)g * 3 + r) * F, (uint32_t)f);
+        n[r] = ldu(m.fnorm + ((size_t)g * 3 + r) * F, (uint32_t)f);
+        nm[r] = ldu(m.fmeanN + (size_t)r * F, (uint32_t)f);
     }
-    const real wj = m.fwj[(size_t)g * F + f];
+    const real wj = ldu(m.fwj + (size_t)g * F, (uint32_t)f);
 #pragma unroll
     for (int v = 0; v < 5; v++)
-        uL[v] = u[(size_t)v * N + cL], Fbar[v] = -wj * fbar[(size_t)v * F + f];
+        uL[v] = ldu(u + (size_t)v * N, (uint32_t)cL), Fbar[v] = -wj * ldu(fbar + (size_t)v * F, (uint32_t)f);
     AdjSide<DIM, NDOF> L;
     L.load(m, cL, x, nullptr, uL, uRec, vis != 0);
     real a[5], c[5], Gb[3][5];
@@ -372,7 +359,7 @@ kRHSBndPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real 
 template <int DIM>
 constexpr int adjFaceWaves() { return DIM == 2 ? 2 : 3; }
 template <int DIM, int RS, bool BATCH, bool VIS>
-__global__ void __launch_bounds__(64 * adjFaceWaves<DIM>()) __attribute__((amdgpu_waves_per_eu(2)))
+__global__ void __launch_bounds__(64 * adjFaceWaves<DIM>()) __attribute__((amdgpu_waves_per_eu(1)))
 kRHSFaceAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
             const real *__restrict__ dlc, const real *__restrict__ fbar, real *__restrict__ fbuf)
 {
@@ -383,36 +370,34 @@ kRHSFaceAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__r
     const idx f0 = xcdTile(blockIdx.x, gridDim.x) * 64, f = f0 + lane;
     const idx cL = f < m.F ? m.f2c[f] : -1, cR = f < m.F ? m.f2c[F + f] : -1;
     const bool on = cR >= 0; // boundary faces: kRHSBndFaceAdj
-    for (int g = w; g < m.G; g += NW)
+    for (int g = w; g < m.G && on; g += NW)
     {
-        if (!on)
-            continue;
         real x[3], n[3], nm[3], sh[3], uL[5], uR[5], Fbar[5];
 #pragma unroll
         for (int r = 0; r < 3; r++)
         {
-            x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
-            n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
-            sh[r] = m.fshift[(size_t)r * F + f];
-            nm[r] = BATCH ? m.fmeanN[(size_t)r * F + f] : 0.0;
+            x[r] = ldu(m.fpts + ((size_t)g * 3 + r) * F, (uint32_t)f);
+            n[r] = ldu(m.fnorm + ((size_t)g * 3 + r) * F, (uint32_t)f);
+            sh[r] = ldu(m.fshift + (size_t)r * F, (uint32_t)f);
+            nm[r] = BATCH ? ldu(m.fmeanN + (size_t)r * F, (uint32_t)f) : 0.0;
         }
-        const real wj = m.fwj[(size_t)g * F + f];
+        const real wj = ldu(m.fwj + (size_t)g * F, (uint32_t)f);
 #pragma unroll
         for (int v = 0; v < 5; v++)
         {
-            uL[v] = u[(size_t)v * N + cL], uR[v] = u[(size_t)v * N + cR];
-            Fbar[v] = -wj * fbar[(size_t)v * F + f];
+            uL[v] = ldu(u + (size_t)v * N, (uint32_t)cL), uR[v] = ldu(u + (size_t)v * N, (uint32_t)cR);
+            Fbar[v] = -wj * ldu(fbar + (size_t)v * F, (uint32_t)f);
         }
         const real dLambda = dlc ? fmax(dlc[cL], dlc[cR]) : 0.0;
         AdjSide<DIM, DIM + 1> L, R;
         L.load(m, cL, x, nullptr, uL, uRec, VIS);
         R.load(m, cR, x, sh, uR, uRec, VIS);
         real a[5], b[5], c[5], d[5], Gb[3][5];
-        facePointBar<RS, BATCH>(m, gp, f, cL, cR, sh, uL, uR, L.U, R.U, L.G, R.G, n, nm, dLambda, Fbar, VIS, a, b, c,
-                                d, Gb);
-        const real hL = 0.5 * m.iscale[cL], hR = 0.5 * m.iscale[cR];
-        const bool first = g == w;
-        auto put = [&](int q, real val) { sm[w][q][lane] = first ? val : sm[w][q][lane] + val; };
+        facePointBar<RS, BATCH>(gp, uL, uR, L.U, R.U, n, nm, dLambda, Fbar, a, b, c, d);
+        if constexpr (VIS)
+            facePointVisBar(m, gp, f, cL, cR, sh, L.U, R.U, L.G, R.G, n, Fbar, a, b, Gb);
+        const real hL = 0.5 * ldu(m.iscale, (uint32_t)cL), hR = 0.5 * ldu(m.iscale, (uint32_t)cR);
+        auto put = [&](int q, real val) { sm[w][q][lane] = g == w ? val : sm[w][q][lane] + val; };
 #pragma unroll
         for (int v = 0; v < 5; v++)
         {
@@ -442,67 +427,67 @@ kRHSFaceAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__r
     }
 }
 
-// the boundary faces' rows of the back side, one thread per face
+// the boundary faces' rows of the back side: a block is 64 faces, wavefront w the points w, w + NW, ...
 template <int DIM, int RS, bool BATCH>
-__global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1)))
+__global__ void __launch_bounds__(64 * adjFaceWaves<DIM>()) __attribute__((amdgpu_waves_per_eu(1)))
 kRHSBndFaceAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
                const real *__restrict__ dlc, const real *__restrict__ fbar, real *__restrict__ fbuf, int vis)
 {
-    const idx t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= m.nBnd)
-        return;
+    constexpr int NW = adjFaceWaves<DIM>(), Q = 5 + 5 * DIM;
+    __shared__ real sm[NW][Q][64];
+    const int lane = threadIdx.x % 64, w = waveIndex(64);
+    const idx t = blockIdx.x * 64 + lane;
+    const bool on = t < m.nBnd;
     const size_t N = m.N, F = m.F;
-    const idx f = m.bndFace[t];
+    const idx f = m.bndFace[on ? t : m.nBnd - 1];
     const idx cL = m.f2c[f];
-    const real isc = m.iscale[cL];
-    real nm[3], uL[5], acc[5], ar[5][DIM];
+    const real isc = ldu(m.iscale, (uint32_t)cL);
+    real nm[3], uL[5];
 #pragma unroll
     for (int r = 0; r < 3; r++)
-        nm[r] = m.fmeanN[(size_t)r * F + f];
+        nm[r] = ldu(m.fmeanN + (size_t)r * F, (uint32_t)f);
 #pragma unroll
     for (int v = 0; v < 5; v++)
-    {
-        uL[v] = u[(size_t)v * N + cL], acc[v] = 0;
-#pragma unroll
-        for (int j = 0; j < DIM; j++)
-            ar[v][j] = 0;
-    }
+        uL[v] = ldu(u + (size_t)v * N, (uint32_t)cL);
     const real dLambda = dlc ? dlc[cL] : 0.0;
-    for (int g = 0; g < m.G; g++)
+    for (int g = w; g < m.G; g += NW)
     {
         real x[3], n[3], Fbar[5];
 #pragma unroll
         for (int r = 0; r < 3; r++)
         {
-            x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
-            n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
+            x[r] = ldu(m.fpts + ((size_t)g * 3 + r) * F, (uint32_t)f);
+            n[r] = ldu(m.fnorm + ((size_t)g * 3 + r) * F, (uint32_t)f);
         }
-        const real wj = m.fwj[(size_t)g * F + f];
+        const real wj = ldu(m.fwj + (size_t)g * F, (uint32_t)f);
 #pragma unroll
         for (int v = 0; v < 5; v++)
-            Fbar[v] = -wj * fbar[(size_t)v * F + f];
+            Fbar[v] = -wj * ldu(fbar + (size_t)v * F, (uint32_t)f);
         AdjSide<DIM, DIM + 1> L;
         L.load(m, cL, x, nullptr, uL, uRec, vis != 0);
         real a[5], c[5], Gb[3][5];
         bndPointBar<RS, BATCH>(m, gp, f, cL, uL, L.U, L.G, n, nm, dLambda, Fbar, vis, a, c, Gb);
+        auto put = [&](int q, real val) { sm[w][q][lane] = g == w ? val : sm[w][q][lane] + val; };
 #pragma unroll
         for (int v = 0; v < 5; v++)
         {
-            acc[v] += a[v] + c[v];
+            put(v, a[v] + c[v]);
             if (uRec)
 #pragma unroll
                 for (int j = 0; j < DIM; j++)
-                    ar[v][j] += L.phi[j] * a[v] + isc * Gb[j][v];
+                    put(5 + v * DIM + j, L.phi[j] * a[v] + isc * Gb[j][v]);
         }
     }
-#pragma unroll
-    for (int v = 0; v < 5; v++)
+    __syncthreads();
+    if (!on)
+        return;
+    const int nw = m.G < NW ? m.G : NW;
+    for (int q = w; q < (uRec ? Q : 5); q += NW)
     {
-        fbuf[(size_t)v * F + f] = acc[v];
-        if (uRec)
-#pragma unroll
-            for (int j = 0; j < DIM; j++)
-                fbuf[(size_t)(5 + v * DIM + j) * F + f] = ar[v][j];
+        real s = sm[0][q][lane];
+        for (int k = 1; k < nw; k++)
+            s += sm[k][q][lane];
+        fbuf[(size_t)q * F + f] = s;
     }
 }
 
@@ -541,30 +526,29 @@ __global__ void __launch_bounds__(256) kRHSGatherAdjLin(DevMesh m, const real *_
     }
 }
 
-// One thread per cell: collect the point sensitivities of the cell's faces into
+// One thread per cell and variable (blockIdx.y): collect the point sensitivities of the cell's faces into
 // uBar (N x 5) and uRecBar (5 M x N), evaluating the cell's basis at each point.
 template <int DIM, int NDOF>
-__global__ void __launch_bounds__(128) kRHSGatherAdj(DevMesh m, const real *__restrict__ pbuf,
-                                                     real *__restrict__ ubar, real *__restrict__ urecbar, int vis)
+__global__ void __launch_bounds__(64) kRHSGatherAdj(DevMesh m, const real *__restrict__ pbuf,
+                                                    real *__restrict__ ubar, real *__restrict__ urecbar, int vis)
 {
     constexpr int M = NDOF - 1;
     const idx i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int v = blockIdx.y;
     if (i >= m.N)
         return;
     const size_t N = m.N, F = m.F, GF = (size_t)m.G * F;
-    real au[5] = {0, 0, 0, 0, 0}, ar[5][M > 0 ? M : 1];
+    real au = 0, ar[M > 0 ? M : 1];
 #pragma unroll
-    for (int v = 0; v < 5; v++)
-#pragma unroll
-        for (int j = 0; j < M; j++)
-            ar[v][j] = 0;
+    for (int j = 0; j < M; j++)
+        ar[j] = 0;
     for (int k = 0; k < m.K; k++)
     {
         const idx f = m.c2f[(size_t)k * N + i];
         if (f < 0)
             continue;
-        const bool back = m.f2c[f] == i;
-        const int rowU = back ? 0 : 5, rowM = back ? 10 : 15;
+        const bool back = (m.c2flag[(size_t)k * N + i] & 1) == 0;
+        const int rowU = (back ? 0 : 5) + v, rowM = (back ? 10 : 15) + v;
         real sh[3];
 #pragma unroll
         for (int r = 0; r < 3; r++)
@@ -572,13 +556,8 @@ __global__ void __launch_bounds__(128) kRHSGatherAdj(DevMesh m, const real *__re
         for (int g = 0; g < m.G; g++)
         {
             const size_t t = (size_t)g * F + f;
-            real gU[5];
-#pragma unroll
-            for (int v = 0; v < 5; v++)
-            {
-                gU[v] = pbuf[(size_t)(rowU + v) * GF + t];
-                au[v] += gU[v] + pbuf[(size_t)(rowM + v) * GF + t];
-            }
+            const real gU = pbuf[(size_t)rowU * GF + t];
+            au += gU + pbuf[(size_t)rowM * GF + t];
             if (urecbar)
             {
                 real x[3], phi[M > 0 ? M : 1];
@@ -587,37 +566,29 @@ __global__ void __launch_bounds__(128) kRHSGatherAdj(DevMesh m, const real *__re
                     x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
                 cellBasisAt<DIM, NDOF>(m, i, x, back ? nullptr : sh, phi);
 #pragma unroll
-                for (int v = 0; v < 5; v++)
-#pragma unroll
-                    for (int j = 0; j < M; j++)
-                        ar[v][j] += phi[j] * gU[v];
+                for (int j = 0; j < M; j++)
+                    ar[j] += phi[j] * gU;
                 if (vis)
                 {
                     real phi2[M > 0 ? M : 1], dphi[DIM][M > 0 ? M : 1];
                     cellBasisGradAt<DIM, NDOF>(m, i, x, back ? nullptr : sh, phi2, dphi);
 #pragma unroll
                     for (int d = 0; d < DIM; d++)
+                    {
+                        const real gg = 0.5 * pbuf[(size_t)(20 + 5 * d + v) * GF + t];
 #pragma unroll
-                        for (int v = 0; v < 5; v++)
-                        {
-                            const real gg = 0.5 * pbuf[(size_t)(20 + 5 * d + v) * GF + t];
-#pragma unroll
-                            for (int j = 0; j < M; j++)
-                                ar[v][j] += dphi[d][j] * gg;
-                        }
+                        for (int j = 0; j < M; j++)
+                            ar[j] += dphi[d][j] * gg;
+                    }
                 }
             }
         }
     }
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-        ubar[(size_t)v * N + i] = au[v];
+    ubar[(size_t)v * N + i] = au;
     if (urecbar)
 #pragma unroll
-        for (int v = 0; v < 5; v++)
-#pragma unroll
-            for (int j = 0; j < M; j++)
-                urecbar[(size_t)(v * M + j) * N + i] = ar[v][j];
+        for (int j = 0; j < M; j++)
+            urecbar[(size_t)(v * M + j) * N + i] = ar[j];
 }
 
 // adjoint of the face flux from the adjoint of the residual (the gather rhs_L += ff / V_L,
@@ -659,7 +630,7 @@ static void rhsAdjLaunch(Ctx &c, const GasParams &gp, const real *u, const real 
         DNDSR_HIP_CHECK(hipGetLastError());
         if (m.nBnd > 0)
         {
-            kRHSBndFaceAdj<DIM, RS, BATCH><<<gridFor(m.nBnd, 64), 64, 0, c.stream>>>(m, gp, u, uRec, dlc, rbar,
+            kRHSBndFaceAdj<DIM, RS, BATCH><<<gridFor(m.nBnd, 64), bs, 0, c.stream>>>(m, gp, u, uRec, dlc, rbar,
                                                                                      c.adjPoint, vis);
             DNDSR_HIP_CHECK(hipGetLastError());
         }
@@ -682,8 +653,8 @@ static void rhsAdjLaunch(Ctx &c, const GasParams &gp, const real *u, const real 
             m, gp, u, uRec, dlc, rbar, c.adjPoint, vis);
         DNDSR_HIP_CHECK(hipGetLastError());
     }
-    kRHSGatherAdj<DIM, NDOF><<<gridFor(m.N, 128), 128, 0, c.stream>>>(m, c.adjPoint, ubar, urecbar,
-                                                                      vis && uRec != nullptr);
+    kRHSGatherAdj<DIM, NDOF><<<dim3(gridFor(m.N, 64), 5), 64, 0, c.stream>>>(m, c.adjPoint, ubar, urecbar,
+                                                                             vis && uRec != nullptr);
     DNDSR_HIP_CHECK(hipGetLastError());
 }
 
@@ -769,83 +740,137 @@ void launchEvalRHSVJP(Ctx &c, const GasParams &gp, const real *u, const real *uR
 // i across slots kj see j across their slot ki = c2s[kj][j], so
 //   xbar_j = c0 ybar_j + c1 sum_kj B_{i,ki}^T ybar_i
 //   ubar_j = c1 sum_kj b_{i,ki} . ybar_i - c1 sum_k b_{j,k} . ybar_j     (per variable)
-// One thread per cell; the neighbour's matrix block is read column-wise.
+// Tile kernel as the forward sweep's (kVRIter, vr.hip): 64 cells per block, one wavefront per output row r
+// (two rows above 16), the neighbour's ybar block staged in LDS once per slot and shared by the row
+// wavefronts, each matrix entry (column r of the neighbour's block) read once.  The ubar rows are spread over
+// the wavefronts.  One thread per cell, which this replaces, re-read the block for every variable at one
+// wavefront per SIMD: 430 us on 10.6k p2 hexahedra.
 // ---------------------------------------------------------------------------
-template <int M, int NV>
-__global__ void __launch_bounds__(128) kVRIterT(DevMesh m, const real *__restrict__ ybar, real *__restrict__ xbar,
-                                                real *__restrict__ ubar, real c0, real c1, int useB, int useb)
+template <int M>
+struct VRTRows
 {
-    const idx jc = blockIdx.x * blockDim.x + threadIdx.x;
-    if (jc >= m.N)
-        return;
+    static constexpr int RW = M <= 16 ? M : (M + 1) / 2; // wavefronts per block
+    static constexpr int RPT = (M + RW - 1) / RW;        // rows per thread
+};
+template <int M, int NV>
+__global__ void __launch_bounds__(64 * VRTRows<M>::RW)
+kVRIterT(DevMesh m, const real *__restrict__ ybar, real *__restrict__ xbar, real *__restrict__ ubar, real c0, real c1,
+         int useB, int useb)
+{
+    constexpr int RW = VRTRows<M>::RW, RPT = VRTRows<M>::RPT, NR = NV * M;
+    constexpr int PER = (NR + RW - 1) / RW, VPT = (NV + RW - 1) / RW;
+    __shared__ real sY[2][PER * RW][64];
+    const int lane = threadIdx.x % 64, w = waveIndex(64);
+    const idx jc = xcdTile(blockIdx.x, gridDim.x) * 64 + lane;
+    const bool valid = jc < m.N;
     const size_t N = m.N;
-    real ax[NV][M];
-    real au[NV];
+    const idx j = valid ? jc : m.N - 1;
+    const bool rowsU = ubar && useb;
+    real ax[RPT][NV], au[VPT];
 #pragma unroll
-    for (int v = 0; v < NV; v++)
+    for (int t = 0; t < RPT; t++)
     {
-        au[v] = 0;
-#pragma unroll
-        for (int r = 0; r < M; r++)
-            ax[v][r] = c0 * ybar[(size_t)(v * M + r) * N + jc];
-    }
-    for (int kj = 0; kj < m.K; kj++)
-    {
-        const idx i = m.c2c[(size_t)kj * N + jc];
-        if (i < 0)
-            continue;
-        const int ki = m.c2s[(size_t)kj * N + jc];
-        const real *B = m.AinvB + (size_t)(1 + ki) * M * M * N + i;
-        const real *b = m.Ainvb + (size_t)ki * M * N + i;
-        const real *bj = m.Ainvb + (size_t)kj * M * N + jc;
-        real yi[M];
+        const int r = w + t * RW < M ? w + t * RW : M - 1;
 #pragma unroll
         for (int v = 0; v < NV; v++)
+            ax[t][v] = c0 * ldu(ybar + (size_t)(v * M + r) * N, (uint32_t)j);
+    }
+#pragma unroll
+    for (int t = 0; t < VPT; t++)
+        au[t] = 0;
+    auto stage = [&](int buf, idx o) {
+        real nb[PER];
+#pragma unroll
+        for (int t = 0; t < PER; t++)
         {
+            const int q = w + t * RW < NR ? w + t * RW : NR - 1;
+            nb[t] = ldu(ybar + (size_t)q * N, (uint32_t)(o >= 0 ? o : j));
+        }
 #pragma unroll
-            for (int q = 0; q < M; q++)
-                yi[q] = ybar[(size_t)(v * M + q) * N + i];
-            if (useB)
+        for (int t = 0; t < PER; t++)
+            sY[buf][w + t * RW][lane] = nb[t];
+    };
+    idx on = m.c2c[j];
+    for (int k = 0; k < m.K; k++)
+    {
+        const idx o = on;
+        const int ki = o >= 0 ? m.c2s[(size_t)k * N + j] : 0;
+        const size_t i = o >= 0 ? o : j;
+        const real *B = m.AinvB + (size_t)(1 + ki) * M * M * N + i;
+        const real *b = m.Ainvb + (size_t)ki * M * N + i;
+        const real *bj = m.Ainvb + (size_t)k * M * N;
+        real bc[RPT][M];
+        if (useB)
 #pragma unroll
-                for (int r = 0; r < M; r++)
+            for (int t = 0; t < RPT; t++)
+            {
+                const int r = w + t * RW < M ? w + t * RW : M - 1;
+#pragma unroll
+                for (int q = 0; q < M; q++)
+                    bc[t][q] = B[(size_t)(q * M + r) * N];
+            }
+        stage(k & 1, o);
+        on = k + 1 < m.K ? m.c2c[(size_t)(k + 1) * N + j] : idx(-1);
+        __syncthreads(); // sY[k & 1] complete; the other buffer no longer read
+        if (o < 0)
+            continue;
+        if (useB)
+#pragma unroll
+            for (int t = 0; t < RPT; t++)
+#pragma unroll
+                for (int v = 0; v < NV; v++)
                 {
                     real s = 0;
 #pragma unroll
                     for (int q = 0; q < M; q++)
-                        s += B[(size_t)(q * M + r) * N] * yi[q];
-                    ax[v][r] += c1 * s;
+                        s += bc[t][q] * sY[k & 1][v * M + q][lane];
+                    ax[t][v] += c1 * s;
                 }
-            if (useb)
+        if (rowsU)
+#pragma unroll
+            for (int t = 0; t < VPT; t++)
             {
+                const int v = w + t * RW;
+                if (v >= NV)
+                    continue;
                 real s = 0, sj = 0;
 #pragma unroll
                 for (int q = 0; q < M; q++)
                 {
-                    s += b[(size_t)q * N] * yi[q];
-                    sj += bj[(size_t)q * N] * ybar[(size_t)(v * M + q) * N + jc];
+                    s += b[(size_t)q * N] * sY[k & 1][v * M + q][lane];
+                    sj += ldu(bj + (size_t)q * N, (uint32_t)j) * ldu(ybar + (size_t)(v * M + q) * N, (uint32_t)j);
                 }
-                au[v] += c1 * (s - sj);
+                au[t] += c1 * (s - sj);
             }
-        }
     }
+    if (!valid)
+        return;
     if (xbar)
 #pragma unroll
-        for (int v = 0; v < NV; v++)
+        for (int t = 0; t < RPT; t++)
+        {
+            const int r = w + t * RW;
+            if (r < M)
 #pragma unroll
-            for (int r = 0; r < M; r++)
-                xbar[(size_t)(v * M + r) * N + jc] = ax[v][r];
+                for (int v = 0; v < NV; v++)
+                    stu(xbar + (size_t)(v * M + r) * N, (uint32_t)j, ax[t][v]);
+        }
     if (ubar)
 #pragma unroll
-        for (int v = 0; v < NV; v++)
-            ubar[(size_t)v * N + jc] = au[v];
+        for (int t = 0; t < VPT; t++)
+        {
+            const int v = w + t * RW;
+            if (v < NV)
+                stu(ubar + (size_t)v * N, (uint32_t)j, au[t]);
+        }
 }
 
 // Transposed boundary term of the VR sweep (forward: uRecNew_i += scale A_i^-1 BCC_i,
 // BCC_i = sum_{boundary faces, g} phi(x_g) (w0^2 (u_B(x_g) - u_i)) w_g JDet_g, u_B the ghost
 // of the compressed point state u_i + phi . uRec_i, or the given point value).  One
 // thread per boundary cell; BCCbar = scale A^-T ybar, then per point the adjoint of u_B - u_i and
-// through the ghost's Jacobian (five dual-number passes of the ghost) of the point state, i.e. of the
-// cell's mean and coefficients (point values given: of the mean only), added to ubar / xbar.
+// through the ghost (bcGhostBar) of the point state, i.e. of the cell's mean and coefficients (point
+// values given: of the mean only), added to ubar / xbar.
 template <int DIM, int NDOF, int NV>
 __global__ void __launch_bounds__(64) kVRBoundaryT(DevMesh m, const real *__restrict__ uRec,
                                                    const real *__restrict__ u, const real *__restrict__ ybar,
@@ -945,28 +970,18 @@ __global__ void __launch_bounds__(64) kVRBoundaryT(DevMesh m, const real *__rest
 #pragma unroll
             for (int v = 0; v < 5; v++)
                 kept = kept && !(ULf[v] != full[v]);
-#pragma unroll 1
-            for (int c = 0; c < 5; c++)
+            real sb[5] = {0, 0, 0, 0, 0}, tb[5];
+#pragma unroll
+            for (int v = 0; v < 5; v++)
+                tb[v] = tv[v < NV ? v : 0];
+            bcGhostBar(m.bcType[zone], ULf, n, m.bcVal + (size_t)zone * 5, m.bcGamma, tb, sb);
+#pragma unroll
+            for (int v = 0; v < NV; v++)
             {
-                Dual D[5], B[5];
+                ub[v] += sb[v];
 #pragma unroll
-                for (int v = 0; v < 5; v++)
-                    D[v] = Dual(ULf[v], v == c ? 1.0 : 0.0);
-                bcGhost(m.bcType[zone], D, n, m.bcVal + (size_t)zone * 5, m.bcGamma, B);
-                real q = 0;
-#pragma unroll
-                for (int v = 0; v < 5; v++)
-                    q += tv[v < NV ? v : 0] * B[v].d;
-#pragma unroll
-                for (int v = 0; v < NV; v++)
-                    if (v == c)
-                    {
-                        ub[v] += q;
-                        if (kept)
-#pragma unroll
-                            for (int j = 0; j < M; j++)
-                                xb[v][j] += phi[j] * q;
-                    }
+                for (int j = 0; j < M; j++)
+                    xb[v][j] += kept ? phi[j] * sb[v] : 0.0;
             }
         }
     }
@@ -998,11 +1013,11 @@ template <int M>
 static void vrTLaunch(Ctx &c, int nVars, const real *ybar, real *xbar, real *ubar, real c0, real c1, int useB,
                       int useb)
 {
-    const int g = gridFor(c.m.N, 128);
+    const int g = gridFor(c.m.N, 64), bs = 64 * VRTRows<M>::RW;
     if (nVars == 5)
-        kVRIterT<M, 5><<<g, 128, 0, c.stream>>>(c.m, ybar, xbar, ubar, c0, c1, useB, useb);
+        kVRIterT<M, 5><<<g, bs, 0, c.stream>>>(c.m, ybar, xbar, ubar, c0, c1, useB, useb);
     else if (nVars == 1)
-        kVRIterT<M, 1><<<g, 128, 0, c.stream>>>(c.m, ybar, xbar, ubar, c0, c1, useB, useb);
+        kVRIterT<M, 1><<<g, bs, 0, c.stream>>>(c.m, ybar, xbar, ubar, c0, c1, useB, useb);
     else
         throw std::runtime_error("nVars must be 1 or 5");
     DNDSR_HIP_CHECK(hipGetLastError());

@@ -233,6 +233,41 @@ __host__ __device__ inline void roeFixBar(const RoeAve &r, real vLm0, real vRm0,
     }
 }
 
+// bcGhost backwards: adds (d ghost / d UL)^T URb to ULb.  The linear ghosts (mirror, reversal, copy, given
+// state) are their own transposes; the others go through dual numbers, one column of the Jacobian per pass.
+__host__ __device__ inline void bcGhostBar(int type, const real *UL, const real *n, const real *far, real gamma,
+                                           const real *URb, real *ULb)
+{
+    if (type == BC_IN)
+        return;
+    if (type == BC_WALL_INVIS || type == BC_SYM || type == BC_WALL || type == BC_OUT)
+    {
+        const real mn = URb[1] * n[0] + URb[2] * n[1] + URb[3] * n[2];
+        ULb[0] += URb[0];
+#pragma unroll
+        for (int d = 0; d < 3; d++)
+            ULb[1 + d] += type == BC_OUT ? URb[1 + d] : (type == BC_WALL ? -URb[1 + d] : URb[1 + d] - 2 * mn * n[d]);
+        ULb[4] += URb[4];
+        return;
+    }
+#pragma unroll 1
+    for (int c = 0; c < 5; c++)
+    {
+        Dual D[5], DR[5];
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            D[v] = Dual(UL[v], v == c ? 1.0 : 0.0);
+        bcGhost(type, D, n, far, gamma, DR);
+        real a = 0;
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            a += URb[v] * DR[v].d;
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            ULb[v] += v == c ? a : 0.0;
+    }
+}
+
 // Riemann flux (riemannFluxR, or with BATCH roeBatchPoint on roeBatchSetup) backwards: adds to ULb, URb and
 // b.  n the point normal, nm the mean normal (BATCH).
 template <int RS, bool BATCH>
