@@ -30,7 +30,7 @@ struct dndsr_ctx
     double *scratchDev = nullptr; // this device's address of `scratch`
     hipStream_t own = nullptr;
     // device-resident time-loop workspace
-    real *wXLast = nullptr, *wURecNew = nullptr, *wLam = nullptr, *wDlc = nullptr, *wDtMin = nullptr;
+    real *wXLast = nullptr, *wStage = nullptr, *wURecNew = nullptr, *wLam = nullptr, *wDlc = nullptr, *wDtMin = nullptr;
     bool haveWork = false;
     // implicit dual-time workspace
     real *iXLast = nullptr, *iRhsF = nullptr, *iRhs = nullptr, *iDTau = nullptr, *iJd = nullptr, *iInc = nullptr,
@@ -64,6 +64,8 @@ static void timeLoopWork(dndsr_ctx *ctx)
     Ctx &c = ctx->c;
     const size_t N = c.m.N;
     ctx->wXLast = devAlloc<real>(c, 5 * N);
+    if (c.m.P == 1 && rhsCellSize(c.m))
+        ctx->wStage = devAlloc<real>(c, 5 * N);
     ctx->wURecNew = devAlloc<real>(c, 5 * (size_t)c.m.M * N);
     ctx->wLam = devAlloc<real>(c, 4 * (size_t)c.m.F);
     ctx->wDlc = devAlloc<real>(c, N);
@@ -1292,26 +1294,34 @@ int dndsr_ssprk3(dndsr_ctx *ctx, const dndsr_euler_settings *es, double *u, doub
     const size_t nU = 5 * N, nR = 5 * (size_t)m.M * N;
     timeLoopWork(ctx);
     real *rec = uRec, *recNew = ctx->wURecNew;
-    // one RK stage: VR sweeps at u, RHS(u), and u = a u + b xLast + cdt dt RHS in the gather pass
-    auto stage = [&](real a, real b, real cdt, const real *dtp, real *save) {
+    // one RK stage: VR sweeps at x, RHS(x), and out = a x + b y + cdt dt RHS in the gather pass.  In place
+    // the first stage saves u in wXLast; on small meshes, whose residual is one pass and cannot update what
+    // it reads, the three stages go u -> wXLast -> wStage -> u and the second and third combine with u,
+    // which the first leaves as it was.
+    real *x1 = ctx->wStage ? ctx->wXLast : u, *x2 = ctx->wStage ? ctx->wStage : u;
+    const real *y = ctx->wStage ? u : ctx->wXLast;
+    const real *dtp = ctx->wDtMin;
+    int nPart = 0;
+    auto stage = [&](real *x, real a, real b, real cdt, real *out, real *save) {
         for (int r = 0; r < nRec; r++)
-            solverVRSweep(c, rec, recNew, u);
-        StageUpdate st{a, b, cdt, b != 0.0 ? ctx->wXLast : nullptr, dtp, u, save};
-        launchEvalRHS(c, gp, u, rec, ctx->wDlc, nullptr, &st);
+            solverVRSweep(c, rec, recNew, x);
+        StageUpdate st{a, b, cdt, b != 0.0 ? y : nullptr, dtp, x, out, save, nPart};
+        launchEvalRHS(c, gp, x, rec, ctx->wDlc, nullptr, &st);
     };
     for (int step = 0; step < nStep; step++)
     {
-        launchEvalDt(c, gp, u, CFL, 1e100, 0, nullptr, ctx->wLam, ctx->wDlc, ctx->wDtMin); // global dt only
-        const real *dtp = ctx->wDtMin;
+        nPart = launchEvalDt(c, gp, u, CFL, 1e100, 0, nullptr, ctx->wLam, ctx->wDlc, ctx->wDtMin, true); // global dt only
+        dtp = nPart ? c.red : ctx->wDtMin;
         if (dtFixed > 0)
         {
             c.hostRed[0] = dtFixed;
             DNDSR_HIP_CHECK(hipMemcpyAsync(ctx->wDtMin, c.hostRed, sizeof(real), hipMemcpyHostToDevice, c.stream));
             DNDSR_HIP_CHECK(hipStreamSynchronize(c.stream));
+            nPart = 0, dtp = ctx->wDtMin;
         }
-        stage(1.0, 0.0, 1.0, dtp, ctx->wXLast); // xLast = u, then u1 = u + dt R(u)
-        stage(0.25, 0.75, 0.25, dtp, nullptr);
-        stage(2. / 3., 1. / 3., 2. / 3., dtp, nullptr);
+        stage(u, 1.0, 0.0, 1.0, x1, ctx->wStage ? nullptr : ctx->wXLast); // xLast = u, then u1 = u + dt R(u)
+        stage(x1, 0.25, 0.75, 0.25, x2, nullptr);
+        stage(x2, 2. / 3., 1. / 3., 2. / 3., u, nullptr);
     }
     if (rec != uRec) // odd number of VR sweeps in total: bring the result home
         launchCopy(c, nR, rec, uRec);

@@ -15,15 +15,15 @@ namespace dndsr
 // deltaLambdaCell = max over faces; then a two-stage min for dtMin.
 // lambdaFace layout [4][F]: lambdaFace, lambdaFaceC, lambdaFaceVis, lambdaFace0(=123=4).
 // ---------------------------------------------------------------------------
-__global__ void __launch_bounds__(256) kDtFace(DevMesh m, GasParams gp, const real *__restrict__ u,
-                                               real *__restrict__ lam, real *__restrict__ dLamF)
+struct DtFaceVals
+{
+    real lc, lcMean, visc, dLam; // lambda without viscosity, |mean normal velocity|, viscous part, deltaLambdaFace
+};
+__device__ __forceinline__ DtFaceVals dtFace(const DevMesh &m, const GasParams &gp, const real *__restrict__ u, idx f,
+                                             idx cL, idx cR)
 {
     const real gamma = gp.gamma;
-    idx f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= m.F)
-        return;
     const size_t N = m.N, F = m.F;
-    idx cL = m.f2c[f], cR = m.f2c[F + f];
     idx cR2 = cR >= 0 ? cR : cL;
     real UL[5], UR[5], n[3];
 #pragma unroll
@@ -41,8 +41,10 @@ __global__ void __launch_bounds__(256) kDtFace(DevMesh m, GasParams gp, const re
     real vs[3] = {vL[0] + vR[0], vL[1] + vR[1], vL[2] + vR[2]};
     real vnMean = 0.5 * dot3(vs, n);
     real aL = sqrt(aL2), aR = sqrt(aR2);
-    real lc = fmax(aL + fabs(vnL), aR + fabs(vnR));
-    real visc = 0.0; // inviscid: lamVis = 0
+    DtFaceVals o;
+    o.lc = fmax(aL + fabs(vnL), aR + fabs(vnR));
+    o.lcMean = fabs(vnMean);
+    o.visc = 0.0; // inviscid: lamVis = 0
     if (gp.viscous)
     {
         // lamVis at the mean of the two cell means (a boundary face has UR = UL),
@@ -52,15 +54,88 @@ __global__ void __launch_bounds__(256) kDtFace(DevMesh m, GasParams gp, const re
         for (int k = 0; k < 5; k++)
             uMean[k] = (UL[k] + UR[k]) * 0.5;
         const real lamVis = lamVisFace(gp, uMean, (pL + pR) * 0.5);
-        visc = lamVis * m.farea[f] * (1. / m.vol[cL] + 1. / m.vol[cR2]);
+        o.visc = lamVis * m.farea[f] * (1. / m.vol[cL] + 1. / m.vol[cR2]);
     }
-    lam[f] = lc + visc;
-    lam[F + f] = fabs(vnMean) + visc;
-    lam[2 * F + f] = visc;
-    lam[3 * F + f] = lc;
     real dv[3] = {vR[0] - vL[0], vR[1] - vL[1], vR[2] - vL[2]};
     real dvn = dot3(dv, n);
-    dLamF[f] = max3(fabs(dvn + aR - aL), fabs(dvn - aR + aL), fabs(aL - aR));
+    o.dLam = max3(fabs(dvn + aR - aL), fabs(dvn - aR + aL), fabs(aL - aR));
+    return o;
+}
+__device__ __forceinline__ void dtFaceStore(const DtFaceVals &v, size_t F, idx f, real *__restrict__ lam)
+{
+    lam[f] = v.lc + v.visc;
+    lam[F + f] = v.lcMean + v.visc;
+    lam[2 * F + f] = v.visc;
+    lam[3 * F + f] = v.lc;
+}
+__global__ void __launch_bounds__(256) kDtFace(DevMesh m, GasParams gp, const real *__restrict__ u,
+                                               real *__restrict__ lam, real *__restrict__ dLamF)
+{
+    const idx f = blockIdx.x * blockDim.x + threadIdx.x;
+    if (f >= m.F)
+        return;
+    const DtFaceVals v = dtFace(m, gp, u, f, m.f2c[f], m.f2c[m.F + f]);
+    dtFaceStore(v, m.F, f, lam);
+    dLamF[f] = v.dLam;
+}
+
+// Small meshes: both passes in one.  L (4 or 8) lanes per cell, one per face slot, evaluate the cell's
+// faces themselves, twice per face, instead of a second launch that reads them back; the slots are
+// combined in order by shuffles, as kDtCell does.  The face's left side stores its four values.
+template <int L>
+__global__ void __launch_bounds__(64 * L) kDtSmall(DevMesh m, GasParams gp, real CFL, real maxDt,
+                                                   const real *__restrict__ u, real *__restrict__ lam,
+                                                   real *__restrict__ dt, real *__restrict__ dlc,
+                                                   real *__restrict__ partMin)
+{
+    __shared__ real sm[L];
+    const int k = threadIdx.x % L;
+    const idx i = (idx)blockIdx.x * 64 + threadIdx.x / L;
+    const size_t N = m.N, F = m.F;
+    const bool in = i < m.N && k < m.K;
+    const size_t q = in ? (size_t)k * N + i : 0;
+    const idx f = in ? m.c2f[q] : idx(-1), o = m.c2c[q];
+    const bool right = (m.c2flag[q] & 1) != 0; // the cell is the face's right side
+    real l = 0, A = 0, dl = 0, d = 3e200, vs = 0;
+    if (i < m.N)
+        vs = CFL * m.vol[i] * m.smooth[i];
+    if (f >= 0)
+    {
+        const DtFaceVals v = dtFace(m, gp, u, f, right ? o : i, right ? i : o);
+        if (!right)
+            dtFaceStore(v, F, f, lam);
+        l = v.lc + v.visc, A = m.farea[f], dl = v.dLam;
+    }
+    real lc = 0, dm = 0;
+#pragma unroll
+    for (int s = 0; s < L; s++)
+    {
+        const real ls = __shfl(l, s, L), As = __shfl(A, s, L);
+        lc += ls * As, dm = fmax(dm, __shfl(dl, s, L));
+    }
+    if (i < m.N)
+    {
+        d = fmin(vs / (lc + 1e-100), maxDt);
+        if (k == 0)
+        {
+            if (dt)
+                dt[i] = d;
+            if (dlc)
+                dlc[i] = dm;
+        }
+    }
+#pragma unroll
+    for (int s = 32; s >= L; s >>= 1)
+        d = fmin(d, __shfl_xor(d, s));
+    if ((threadIdx.x & 63) == 0)
+        sm[threadIdx.x >> 6] = d;
+    __syncthreads();
+    if (threadIdx.x == 0)
+    {
+        for (int w = 1; w < L; w++)
+            d = fmin(d, sm[w]);
+        partMin[blockIdx.x] = d;
+    }
 }
 
 // Loads issued together as in kRHSGather; blockDim.x is a power of two of at most 256.
@@ -134,10 +209,45 @@ __global__ void kFillFromScalar(idx n, const real *s, real *out)
         out[i] = s[0];
 }
 
-void launchEvalDt(Ctx &c, const GasParams &gp, const real *u, real CFL, real maxDt, int useLocalDt, real *dt,
-                  real *lambdaFace, real *deltaLambdaCell, real *dtMinDev)
+static void finishDt(Ctx &c, int nPart, int useLocalDt, real *dt, real *dtMinDev)
+{
+    kReduceMin<<<1, 256, 0, c.stream>>>(c.red, nPart, dtMinDev);
+    DNDSR_HIP_CHECK(hipGetLastError());
+    if (!useLocalDt && dt)
+    {
+        kFillFromScalar<<<gridFor(c.m.N, 256), 256, 0, c.stream>>>(c.m.N, dtMinDev, dt);
+        DNDSR_HIP_CHECK(hipGetLastError());
+    }
+}
+
+// Cells up to which the one-pass time step is taken.  Below, a launch (about 4 us) costs more than
+// evaluating each face twice; ten SSP-RK3 steps, two passes against one: 4 096 quadrilaterals 555 / 487 us,
+// 16 384 591 / 537, 32 400 690 / 678, 65 536 884 / 963; three on hexahedra: 4 096 235 / 222,
+// 15 625 272 / 263, 32 768 341 / 353.
+constexpr idx kSmallDt = 16384;
+int launchEvalDt(Ctx &c, const GasParams &gp, const real *u, real CFL, real maxDt, int useLocalDt, real *dt,
+                 real *lambdaFace, real *deltaLambdaCell, real *dtMinDev, bool partials)
 {
     DevMesh &m = c.m;
+    // (dt and deltaLambdaCell apart from u: the one pass writes them while other blocks read)
+    const size_t N = m.N;
+    auto apart = [&](const real *w) { return !w || w + N <= u || u + 5 * N <= w; };
+    if (m.N <= kSmallDt && apart(dt) && apart(deltaLambdaCell))
+    {
+        const int nb = gridFor(m.N, 64);
+        {
+            KernelTimer kt(c, K_DT_FACE);
+            if (m.K <= 4)
+                kDtSmall<4><<<nb, 256, 0, c.stream>>>(m, gp, CFL, maxDt, u, lambdaFace, dt, deltaLambdaCell, c.red);
+            else
+                kDtSmall<8><<<nb, 512, 0, c.stream>>>(m, gp, CFL, maxDt, u, lambdaFace, dt, deltaLambdaCell, c.red);
+            DNDSR_HIP_CHECK(hipGetLastError());
+        }
+        if (partials)
+            return nb;
+        finishDt(c, nb, useLocalDt, dt, dtMinDev);
+        return 0;
+    }
     {
         KernelTimer kt(c, K_DT_FACE);
         kDtFace<<<gridFor(m.F, 256), 256, 0, c.stream>>>(m, gp, u, lambdaFace, c.faceLamTmp);
@@ -153,13 +263,8 @@ void launchEvalDt(Ctx &c, const GasParams &gp, const real *u, real CFL, real max
                                                      c.red);
         DNDSR_HIP_CHECK(hipGetLastError());
     }
-    kReduceMin<<<1, 256, 0, c.stream>>>(c.red, nb, dtMinDev);
-    DNDSR_HIP_CHECK(hipGetLastError());
-    if (!useLocalDt && dt)
-    {
-        kFillFromScalar<<<gridFor(m.N, 256), 256, 0, c.stream>>>(m.N, dtMinDev, dt);
-        DNDSR_HIP_CHECK(hipGetLastError());
-    }
+    finishDt(c, nb, useLocalDt, dt, dtMinDev);
+    return 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -484,6 +589,7 @@ __global__ void __launch_bounds__(256) kRHSGather(DevMesh m, const real *__restr
                                                   StageUpdate st, int *__restrict__ nonFinite)
 {
     const idx i = xcdTile(blockIdx.x, gridDim.x) * (idx)blockDim.x + threadIdx.x;
+    const real dt = st.u ? stageDtJoin(st, stageDtLane(st)) : 1.0;
     if (i >= m.N)
         return;
     const size_t N = m.N, F = m.F;
@@ -499,7 +605,6 @@ __global__ void __launch_bounds__(256) kRHSGather(DevMesh m, const real *__restr
             w[k] = 0, f[k] = 0;
     }
     const real vol = m.vol[i];
-    const real dt = st.u && st.dtDev ? st.dtDev[0] : 1.0;
     real fv[KM][5];
 #pragma unroll
     for (int k = 0; k < KM; k++)
@@ -526,20 +631,11 @@ __global__ void __launch_bounds__(256) kRHSGather(DevMesh m, const real *__restr
         for (int v = 0; v < 5; v++)
             rhs[v * N + i] = acc[v];
     }
-    if (st.u) // same arithmetic as kAxpby(a, u, b, y, cdt, rhs, dt)
+    if (st.u)
     {
 #pragma unroll
         for (int v = 0; v < 5; v++)
-        {
-            real xi = st.u[v * N + i];
-            if (st.save)
-                st.save[v * N + i] = xi;
-            real r = st.a * xi;
-            if (st.y)
-                r += st.b * st.y[v * N + i];
-            r += st.cdt * (acc[v] * dt);
-            st.u[v * N + i] = r;
-        }
+            stageStore(st, v * N + i, stageLoad(st, v * N + i), acc[v], dt);
     }
 }
 
@@ -1191,6 +1287,48 @@ static void rhsDispatch(Ctx &c, const GasParams &gp, const real *u, const real *
         throw std::runtime_error(kBadFaceRule);
 }
 
+void launchRHSViscous(Ctx &c, const GasParams &gp, const real *u, const real *uRec, real *ff, bool bndOnly)
+{
+    DevMesh &m = c.m;
+    if (bndOnly && m.nBnd == 0)
+        return;
+    KernelTimer kt(c, K_RHS_VISCOUS);
+    const idx *list = bndOnly ? m.bndFace : nullptr;
+    const idx nList = bndOnly ? m.nBnd : m.F;
+    const int nb = gridFor(nList, 128);
+    const int P = uRec ? m.P : 1;
+    // the gas-dependent ghosts only where the table has such a zone (their branch costs
+    // the kernel registers)
+    auto launchVis = [&](auto dimC, auto ndofC) {
+        constexpr int D = decltype(dimC)::value, ND = decltype(ndofC)::value;
+        if (m.gasBC)
+            kRHSViscous<D, ND, true><<<nb, 128, 0, c.stream>>>(m, gp, u, uRec, ff, list, nList);
+        else
+            kRHSViscous<D, ND, false><<<nb, 128, 0, c.stream>>>(m, gp, u, uRec, ff, list, nList);
+    };
+    using I2 = std::integral_constant<int, 2>;
+    using I3 = std::integral_constant<int, 3>;
+    if (m.dim == 2)
+    {
+        if (P == 1)
+            launchVis(I2{}, I3{});
+        else if (P == 2)
+            launchVis(I2{}, std::integral_constant<int, 6>{});
+        else
+            launchVis(I2{}, std::integral_constant<int, 10>{});
+    }
+    else
+    {
+        if (P == 1)
+            launchVis(I3{}, std::integral_constant<int, 4>{});
+        else if (P == 2)
+            launchVis(I3{}, std::integral_constant<int, 10>{});
+        else
+            launchVis(I3{}, std::integral_constant<int, 20>{});
+    }
+    DNDSR_HIP_CHECK(hipGetLastError());
+}
+
 void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *rhs,
                    const StageUpdate *stage, real *faceFluxBuf, bool flagNonFinite)
 {
@@ -1202,6 +1340,12 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
         throw std::runtime_error("viscous residual needs prGas > 0, Rgas > 0 and muGas >= 0");
     // first-order and linear reconstructions: the interior faces' whole flux in one pass
     const bool linear = (!uRec || m.P == 1) && rhsLinearRule(m);
+    if (linear && !faceFluxBuf && rhsCellRule(c, u, uRec, dlc, rhs, stage))
+    {
+        launchRHSCellLinear(c, gp, u, uRec, dlc, ff, rhs, stage ? *stage : StageUpdate{},
+                            flagNonFinite ? c.nonFinite : nullptr);
+        return;
+    }
     {
         KernelTimer kt(c, K_RHS_FACE); // inviscid interior, periodic and boundary faces
         if (linear)
@@ -1225,48 +1369,13 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
                 rhsDispatch<3, 20>(c, gp, u, uRec, dlc, ff);
         }
     }
-    const bool bndOnly = linear && rhsLinearViscous(m); // the interior faces have theirs
-    if (gp.viscous && (!bndOnly || m.nBnd > 0))
-    {
-        KernelTimer kt(c, K_RHS_VISCOUS);
-        const idx *list = bndOnly ? m.bndFace : nullptr;
-        const idx nList = bndOnly ? m.nBnd : m.F;
-        const int nb = gridFor(nList, 128);
-        const int P = uRec ? m.P : 1;
-        // the gas-dependent ghosts only where the table has such a zone (their branch costs
-        // the kernel registers)
-        auto launchVis = [&](auto dimC, auto ndofC) {
-            constexpr int D = decltype(dimC)::value, ND = decltype(ndofC)::value;
-            if (m.gasBC)
-                kRHSViscous<D, ND, true><<<nb, 128, 0, c.stream>>>(m, gp, u, uRec, ff, list, nList);
-            else
-                kRHSViscous<D, ND, false><<<nb, 128, 0, c.stream>>>(m, gp, u, uRec, ff, list, nList);
-        };
-        using I2 = std::integral_constant<int, 2>;
-        using I3 = std::integral_constant<int, 3>;
-        if (m.dim == 2)
-        {
-            if (P == 1)
-                launchVis(I2{}, I3{});
-            else if (P == 2)
-                launchVis(I2{}, std::integral_constant<int, 6>{});
-            else
-                launchVis(I2{}, std::integral_constant<int, 10>{});
-        }
-        else
-        {
-            if (P == 1)
-                launchVis(I3{}, std::integral_constant<int, 4>{});
-            else if (P == 2)
-                launchVis(I3{}, std::integral_constant<int, 10>{});
-            else
-                launchVis(I3{}, std::integral_constant<int, 20>{});
-        }
-        DNDSR_HIP_CHECK(hipGetLastError());
-    }
+    if (gp.viscous)
+        launchRHSViscous(c, gp, u, uRec, ff, linear && rhsLinearViscous(m)); // the interior faces have theirs
     KernelTimer kt2(c, K_RHS_GATHER);
     const int bs = cellBlock(m.N), nb2 = gridFor(m.N, bs);
-    const StageUpdate su = stage ? *stage : StageUpdate{};
+    StageUpdate su = stage ? *stage : StageUpdate{};
+    if (su.u && !su.out)
+        su.out = const_cast<real *>(su.u);
     int *flag = flagNonFinite ? c.nonFinite : nullptr;
     if (m.K <= 4)
         kRHSGather<4><<<nb2, bs, 0, c.stream>>>(m, ff, rhs, su, flag);

@@ -221,15 +221,21 @@ bool usesSubs2nd(const DevMesh &m);
 void launchVR2nd(Ctx &c, int nVars, const real *u, real *out);
 void launchVRIterDiff(Ctx &c, int nVars, const real *uRec, const real *u, const real *uRecDiff, real *uRecNew);
 // ---- launchers (euler.hip)
-void launchEvalDt(Ctx &c, const GasParams &gp, const real *u, real CFL, real maxDt, int useLocalDt, real *dt,
-                  real *lambdaFace, real *deltaLambdaCell, real *dtMinDev);
-// Optional stage combination fused into the RHS gather: u = a u + b y + cdt dt RHS (y, dtDev
-// optional; save receives u first).  The face pass reads u before the gather starts.
+// partials: dtMinDev may be left unwritten; the return value is then the number of partial minima in
+// the context's reduction buffer (0: dtMinDev holds the minimum)
+int launchEvalDt(Ctx &c, const GasParams &gp, const real *u, real CFL, real maxDt, int useLocalDt, real *dt,
+                 real *lambdaFace, real *deltaLambdaCell, real *dtMinDev, bool partials = false);
+// Optional stage combination fused into the RHS gather: out = a u + b y + cdt dt RHS (y optional; save
+// receives u first).  dt is dtDev[0], the least of the nPart values at dtDev where nPart > 0, or 1.
+// out null or u: in place, the face pass reading u before the gather starts; the one-pass form of small
+// meshes (rhsCellRule) needs another array.
 struct StageUpdate
 {
     real a = 0, b = 0, cdt = 0;
     const real *y = nullptr, *dtDev = nullptr;
-    real *u = nullptr, *save = nullptr;
+    const real *u = nullptr;
+    real *out = nullptr, *save = nullptr;
+    int nPart = 0;
 };
 // faceFluxBuf: the [5][F] face-flux scratch (NULL = the context's); flagNonFinite: raise the
 // context's non-finite flag from the gather
@@ -242,6 +248,15 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
 bool rhsLinearRule(const DevMesh &m);
 bool rhsLinearViscous(const DevMesh &m);
 void setupLinear(Ctx &c);
+// the one-pass form of small meshes: whether the mesh takes it, whether a call does (its output apart
+// from what it reads), and the launch
+bool rhsCellSize(const DevMesh &m);
+bool rhsCellRule(const Ctx &c, const real *u, const real *uRec, const real *dlc, const real *rhs,
+                 const StageUpdate *stage);
+void launchRHSCellLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff,
+                         real *rhs, const StageUpdate &stage, int *nonFinite);
+// the viscous flux (euler.hip) of all faces, or of the boundary faces only
+void launchRHSViscous(Ctx &c, const GasParams &gp, const real *u, const real *uRec, real *ff, bool bndOnly);
 void launchRHSFaceLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff,
                          bool pack);
 void launchLUSGSInit(Ctx &c, const real *dTau, real dt, real alphaDiag, const real *lambdaFace, real *jdiag);

@@ -5,6 +5,46 @@
 
 namespace dndsr
 {
+// the stage's time step (StageUpdate), in two steps: the lane's loads, and the minimum over the
+// wavefront, whose lanes all take part
+__device__ __forceinline__ real stageDtLane(const StageUpdate &st)
+{
+    if (st.nPart == 0)
+        return st.dtDev ? st.dtDev[0] : 1.0;
+    real d = 3e200;
+    for (int q = threadIdx.x & 63; q < st.nPart; q += 64)
+        d = fmin(d, st.dtDev[q]);
+    return d;
+}
+__device__ __forceinline__ real stageDtJoin(const StageUpdate &st, real d)
+{
+    if (st.nPart == 0)
+        return d;
+#pragma unroll
+    for (int s = 32; s > 0; s >>= 1)
+        d = fmin(d, __shfl_xor(d, s));
+    return d;
+}
+struct StageIn
+{
+    real x, y;
+};
+__device__ __forceinline__ StageIn stageLoad(const StageUpdate &st, size_t o)
+{
+    return {st.u ? st.u[o] : 0.0, st.u && st.y ? st.y[o] : 0.0};
+}
+// same arithmetic as kAxpby(a, u, b, y, cdt, rhs, dt) at offset o
+__device__ __forceinline__ void stageStore(const StageUpdate &st, size_t o, const StageIn &in, real rhs, real dt)
+{
+    if (st.save)
+        st.save[o] = in.x;
+    real r = st.a * in.x;
+    if (st.y)
+        r += st.b * in.y;
+    r += st.cdt * (rhs * dt);
+    st.out[o] = r;
+}
+
 // Boundary faces (EvaluateRHS.hxx:194-207, 336-345), run after the tile kernel and overwriting the
 // tile kernel's flux of that face.  The Roe average takes the cell mean and its ghost at the face
 // centre (mean normal); every point takes the reconstructed state and its ghost at the point normal;
