@@ -22,7 +22,10 @@
 // pass is about one round of waves).  So a neighbour costs 64 + 32 bytes in 16-byte loads, everything
 // a cell reads of its own is one record and coalesced rows, all K neighbour rows are in flight at
 // once, and the blocks of one XCD take a contiguous range of positions (its L2 then serves the rows
-// that several of them gather).
+// that several of them gather).  With three colours or more a visit gathers one side's neighbours only
+// (SGSVisit).  Average pass, in place: 945k tetrahedra (5 colours) 20.5 us (23.4 with all neighbours,
+// 4.9 TB/s of cache-line misses), 246k hexahedra (2 colours) 12.1 us (15.2 at three waves per SIMD, with
+// 16 registers in scratch).
 #include <utility>
 
 #include "internal.hpp"
@@ -83,7 +86,7 @@ __device__ __forceinline__ void rowStore(T *p, const T *in)
 // the mesh-only part: scaled normals and neighbour positions per position, A_f / (2 V_i) per cell
 template <typename T>
 __global__ void __launch_bounds__(256) kSGSMesh(DevMesh m, T *__restrict__ nq, idx *__restrict__ nbr,
-                                                real *__restrict__ half)
+                                                idx *__restrict__ face, real *__restrict__ half)
 {
     const idx p = blockIdx.x * blockDim.x + threadIdx.x;
     if (p >= m.N)
@@ -91,17 +94,20 @@ __global__ void __launch_bounds__(256) kSGSMesh(DevMesh m, T *__restrict__ nq, i
     const size_t N = m.N, F = m.F;
     const idx i = m.colorCells[p];
     const real vol = m.vol[i];
+    const uint32_t ranks = slotRanks(m, i, p);
     for (int k = 0; k < m.K; k++)
     {
         const idx f = m.c2f[(size_t)k * N + i];
         const idx o = m.c2c[(size_t)k * N + i];
         const real h = f >= 0 ? 0.5 * m.farea[f] / vol : 0.0;
         const real s = (m.c2flag[(size_t)k * N + i] & 1) ? -h : h;
+        const uint32_t to = (ranks >> (4 * k)) & 15;
 #pragma unroll
         for (int r = 0; r < 3; r++)
-            nq[((size_t)k * 3 + r) * N + p] = f >= 0 ? (T)(m.fmeanN[r * F + f] * s) : T(0);
-        nbr[(size_t)k * N + p] = (f < 0 || o < 0 || o == i) ? idx(-1) : m.cellPos[o];
-        half[(size_t)k * N + i] = h;
+            nq[((size_t)to * 3 + r) * N + p] = f >= 0 ? (T)(m.fmeanN[r * F + f] * s) : T(0);
+        nbr[(size_t)to * N + p] = (f < 0 || o < 0 || o == i) ? idx(-1) : m.cellPos[o];
+        face[(size_t)to * N + i] = f;
+        half[(size_t)to * N + i] = h;
     }
 }
 
@@ -115,8 +121,8 @@ template <typename T, int KM>
 __global__ void __launch_bounds__(256) kSGSPrep(DevMesh m, real gamma, real alpha, BDFTerms bt, real rdt,
                                                 const real *__restrict__ u, const real *__restrict__ rhsF,
                                                 const real *__restrict__ dTau, const real *__restrict__ lam,
-                                                const real *__restrict__ half, T *__restrict__ st,
-                                                T *__restrict__ rec, real *__restrict__ part)
+                                                const idx *__restrict__ face, const real *__restrict__ half,
+                                                T *__restrict__ st, T *__restrict__ rec, real *__restrict__ part)
 {
     __shared__ real sm[5][4];
     const idx i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -130,7 +136,7 @@ __global__ void __launch_bounds__(256) kSGSPrep(DevMesh m, real gamma, real alph
         for (int k = 0; k < KM; k++)
         {
             const size_t q = (size_t)(k < m.K ? k : 0) * N + i;
-            f[k] = m.c2f[q];
+            f[k] = face[q];
             h[k] = half[q];
             if (k >= m.K || f[k] < 0)
                 f[k] = 0, h[k] = 0;
@@ -192,18 +198,19 @@ __global__ void __launch_bounds__(256) kSGSPrep(DevMesh m, real gamma, real alph
 }
 
 // The positions [begin, end): xw = (rhs - alpha sum_k dF_k(x)) / D.  Gauss-Seidel: x and xw are the
-// same array, one colour per launch, so a neighbour's row is its newest value; first: the sweep that
-// starts from zero reads only the neighbours before p.  Jacobi: the whole mesh in one launch from the
-// other array; first reads none.
+// same array, one colour per launch, so a neighbour's row is its newest value; the neighbours of one
+// side are summed (side) and, with HALF, the other side's sum is the one the cell's last visit kept
+// (if any: read).  Jacobi: the whole mesh in one launch from the other array, all neighbours,
+// or none in the sweep that starts from zero.
 template <typename T, int K>
 constexpr int sgsPassWaves()
 {
-    return sizeof(T) == 8 ? (K <= 4 ? 4 : 3) : 1; // FP64: the rows of 4 (6) slots in 128 (168) VGPRs
+    return sizeof(T) == 8 ? (K <= 4 ? 3 : 2) : 1; // FP64: the rows of 4 (6) slots in 168 (256) VGPRs, no scratch
 }
-template <typename T, int K>
+template <typename T, int K, bool HALF>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(sgsPassWaves<T, K>())))
 kSGSPass(size_t N, real gammaD, T alpha, const T *x, T *xw, const T *__restrict__ st, const T *__restrict__ rec,
-         const T *__restrict__ nq, const idx *__restrict__ nbr, int gs, int first, idx begin, idx end)
+         const T *__restrict__ nq, const idx *__restrict__ nbr, T *half, int read, int side, idx begin, idx end)
 {
     const idx p = begin + xcdTile(blockIdx.x, gridDim.x) * 64 + (idx)threadIdx.x;
     if (p >= end)
@@ -213,22 +220,32 @@ kSGSPass(size_t N, real gammaD, T alpha, const T *x, T *xw, const T *__restrict_
 #pragma unroll
     for (int k = 0; k < K; k++)
         po[k] = nbr[(size_t)k * N + p];
+    bool use[K];
+#pragma unroll
+    for (int k = 0; k < K; k++)
+        use[k] = po[k] >= 0 && (side & (po[k] < p ? SGS_BEFORE : SGS_AFTER));
     T q[K][3], r[kRecRow];
     rowLoad<T, kRecRow>(rec + (size_t)p * kRecRow, r);
 #pragma unroll
     for (int k = 0; k < K; k++)
+    {
+        const size_t qp = !HALF || use[k] ? p : begin; // the slots not used share one line
 #pragma unroll
         for (int d = 0; d < 3; d++)
-            q[k][d] = nq[((size_t)k * 3 + d) * N + p];
-    // the gathers are unconditional (a slot that is not used reads the cell's own row, a valid
-    // address): a load under a branch makes the compiler wait for every earlier load at the join
-    bool use[K];
-    T du[K][5], s[K][4];
+            q[k][d] = nq[((size_t)k * 3 + d) * N + qp];
+    }
+    // the gathers are unconditional (the slots not used all read one row, of another colour if there is
+    // one): a load under a branch makes the compiler wait for every earlier load at the join
+    const size_t none = begin > 0 ? 0 : N - 1;
+    T du[K][5], s[K][4], hs[5];
+    if constexpr (HALF)
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+            hs[v] = half[(size_t)v * N + p];
 #pragma unroll
     for (int k = 0; k < K; k++)
     {
-        use[k] = po[k] >= 0 && !(first && !(gs && po[k] < p));
-        const size_t o = use[k] ? po[k] : p;
+        const size_t o = use[k] ? po[k] : none;
         T row[kIncRow];
         rowLoad<T, 4>(x + o * kIncRow, row);
         row[4] = x[o * kIncRow + 4];
@@ -256,6 +273,13 @@ kSGSPass(size_t N, real gammaD, T alpha, const T *x, T *xw, const T *__restrict_
             acc[1 + c] += d[1 + c] * vq + v[c] * rr + q[k][c] * dp - l * d[1 + c];
         acc[4] += (d[4] + dp) * vq + v[3] * rr - l * d[4];
     }
+    if constexpr (HALF)
+#pragma unroll
+        for (int v = 0; v < 5; v++)
+        {
+            half[(size_t)v * N + p] = acc[v];
+            acc[v] += read ? hs[v] : T(0);
+        }
     T out[kIncRow];
 #pragma unroll
     for (int v = 0; v < kIncRow; v++)
@@ -264,7 +288,7 @@ kSGSPass(size_t N, real gammaD, T alpha, const T *x, T *xw, const T *__restrict_
 }
 
 template <typename T>
-static void sgsPass(Ctx &c, const GasParams &gp, T alpha, SGSWork<T> &w, const T *x, T *xw, int gs, int first, idx b,
+static void sgsPass(Ctx &c, const GasParams &gp, T alpha, SGSWork<T> &w, const T *x, T *xw, const SGSVisit &sv, idx b,
                     idx e)
 {
     DevMesh &m = c.m;
@@ -272,16 +296,19 @@ static void sgsPass(Ctx &c, const GasParams &gp, T alpha, SGSWork<T> &w, const T
         return;
     KernelTimer kt(c, K_SGS);
     const int g = gridFor(e - b, 64);
-    auto go = [&](auto kern) {
-        kern<<<g, 64, 0, c.stream>>>((size_t)m.N, gp.gamma, alpha, x, xw, w.st, w.rec, w.nq, w.nbr, gs, first, b, e);
+    const bool half = sv.read || sv.keep;
+    auto go = [&](auto kHalf, auto kWhole) {
+        auto kern = half ? kHalf : kWhole;
+        kern<<<g, 64, 0, c.stream>>>((size_t)m.N, gp.gamma, alpha, x, xw, w.st, w.rec, w.nq, w.nbr,
+                                      w.half, sv.read, sv.side, b, e);
     };
     switch (m.K)
     {
-    case 3: go(kSGSPass<T, 3>); break;
-    case 4: go(kSGSPass<T, 4>); break;
-    case 5: go(kSGSPass<T, 5>); break;
-    case 6: go(kSGSPass<T, 6>); break;
-    case 2: go(kSGSPass<T, 2>); break;
+    case 3: go(kSGSPass<T, 3, true>, kSGSPass<T, 3, false>); break;
+    case 4: go(kSGSPass<T, 4, true>, kSGSPass<T, 4, false>); break;
+    case 5: go(kSGSPass<T, 5, true>, kSGSPass<T, 5, false>); break;
+    case 6: go(kSGSPass<T, 6, true>, kSGSPass<T, 6, false>); break;
+    case 2: go(kSGSPass<T, 2, true>, kSGSPass<T, 2, false>); break;
     default: throw std::runtime_error("unsupported number of faces per cell");
     }
     DNDSR_HIP_CHECK(hipGetLastError());
@@ -303,8 +330,11 @@ static void sgsSolve(Ctx &c, const GasParams &gp, real alphaD, const BDFTerms &b
         w.rec = devAlloc<T>(c, kRecRow * N);
         w.nq = devAlloc<T>(c, (size_t)3 * m.K * N);
         w.nbr = devAlloc<idx>(c, (size_t)m.K * N);
+        w.face = devAlloc<idx>(c, (size_t)m.K * N);
+        if (m.nColor > 2)
+            w.half = devAlloc<T>(c, 5 * N);
         w.st = devAlloc<T>(c, kStRow * N);
-        kSGSMesh<T><<<nb, 256, 0, c.stream>>>(m, w.nq, w.nbr, half);
+        kSGSMesh<T><<<nb, 256, 0, c.stream>>>(m, w.nq, w.nbr, w.face, half);
         DNDSR_HIP_CHECK(hipGetLastError());
     }
     if (!gsUpdate && !w.x[1])
@@ -312,11 +342,11 @@ static void sgsSolve(Ctx &c, const GasParams &gp, real alphaD, const BDFTerms &b
     {
         KernelTimer kt(c, K_LUSGS_INIT);
         if (m.K <= 4)
-            kSGSPrep<T, 4><<<nb, 256, 0, c.stream>>>(m, gp.gamma, alphaD, bt, 1.0 / dt, u, rhsF, dTau, lam, half, w.st,
-                                                     w.rec, c.red);
+            kSGSPrep<T, 4><<<nb, 256, 0, c.stream>>>(m, gp.gamma, alphaD, bt, 1.0 / dt, u, rhsF, dTau, lam, w.face, half,
+                                                     w.st, w.rec, c.red);
         else
-            kSGSPrep<T, kMaxFC><<<nb, 256, 0, c.stream>>>(m, gp.gamma, alphaD, bt, 1.0 / dt, u, rhsF, dTau, lam, half,
-                                                          w.st, w.rec, c.red);
+            kSGSPrep<T, kMaxFC><<<nb, 256, 0, c.stream>>>(m, gp.gamma, alphaD, bt, 1.0 / dt, u, rhsF, dTau, lam, w.face,
+                                                          half, w.st, w.rec, c.red);
         DNDSR_HIP_CHECK(hipGetLastError());
         launchReduceSum5(c, nb, resDev);
     }
@@ -327,7 +357,7 @@ static void sgsSolve(Ctx &c, const GasParams &gp, real alphaD, const BDFTerms &b
         T *y = w.x[1];
         for (int s = 0; s < 2 * (1 + sgsIter); s++)
         {
-            sgsPass<T>(c, gp, alpha, w, x, y, 0, s == 0, 0, m.N);
+            sgsPass<T>(c, gp, alpha, w, x, y, {s == 0 ? SGS_NONE : SGS_ALL, false, false}, 0, m.N);
             std::swap(x, y);
         }
     }
@@ -341,7 +371,8 @@ static void sgsSolve(Ctx &c, const GasParams &gp, real alphaD, const BDFTerms &b
                 for (int q = first || m.nColor < 2 ? 0 : 1; q < m.nColor; q++)
                 {
                     const int col = dir ? q : m.nColor - 1 - q;
-                    sgsPass<T>(c, gp, alpha, w, x, x, 1, first, m.colorPtrHost[col], m.colorPtrHost[col + 1]);
+                    sgsPass<T>(c, gp, alpha, w, x, x, sgsVisit(m, col, dir, first, s == sgsIter && !dir),
+                               m.colorPtrHost[col], m.colorPtrHost[col + 1]);
                 }
             }
     *result = x;
