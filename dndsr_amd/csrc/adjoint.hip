@@ -355,6 +355,9 @@ kRHSBndPointAdj(DevMesh m, GasParams gp, const real *__restrict__ u, const real 
 // only add their faces' rows.  A block is 64 faces; wavefront w takes the points w, w + NW, ... and sums
 // them in its own LDS rows (the reverse pass leaves no registers for 30 accumulators), which are then added in
 // wavefront order.  fbuf [2][5 + 5 DIM][F].
+// Bound by FP64 issue and registers: at one wavefront per SIMD what does not fit stays in accumulation
+// registers (143 us on the 333k faces of the mixed 2-D mesh, viscous); two per SIMD spill to scratch (328),
+// and inviscid and viscous parts in kernels of their own measured 178.
 // ---------------------------------------------------------------------------
 template <int DIM>
 constexpr int adjFaceWaves() { return DIM == 2 ? 2 : 3; }
@@ -744,7 +747,7 @@ void launchEvalRHSVJP(Ctx &c, const GasParams &gp, const real *u, const real *uR
 // (two rows above 16), the neighbour's ybar block staged in LDS once per slot and shared by the row
 // wavefronts, each matrix entry (column r of the neighbour's block) read once.  The ubar rows are spread over
 // the wavefronts.  One thread per cell, which this replaces, re-read the block for every variable at one
-// wavefront per SIMD: 430 us on 10.6k p2 hexahedra.
+// wavefront per SIMD: 430 us on 10.6k p2 hexahedra, against 52.
 // ---------------------------------------------------------------------------
 template <int M>
 struct VRTRows

@@ -584,6 +584,7 @@ kRHSFace(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__rest
 // with weight 0: a load under a branch would wait for every earlier one at the join), and divides
 // the sum by the volume once.  The side comes from the slot flags, not from a load that depends on
 // the face index.
+// 945k tetrahedra 44 us (one slot after the other 84), 4 096 quadrilaterals 4.4 us (6.3).
 template <int KM>
 __global__ void __launch_bounds__(256) kRHSGather(DevMesh m, const real *__restrict__ fflux, real *__restrict__ rhs,
                                                   StageUpdate st, int *__restrict__ nonFinite)
