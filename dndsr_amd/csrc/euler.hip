@@ -1115,7 +1115,8 @@ __global__ void __launch_bounds__(128) kRHSViscous(DevMesh m, GasParams gp, cons
     const idx t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= nList)
         return;
-    const idx f = list ? list[t] : t;
+    const idx f = list ? list[t] : t; // list: the boundary faces
+    const FacePts fp = list ? bndPts(m, t) : facePts(m, f);
     const size_t N = m.N, F = m.F;
     const idx cL = m.f2c[f], cR = m.f2c[F + f];
     const bool bnd = cR < 0;
@@ -1151,7 +1152,7 @@ __global__ void __launch_bounds__(128) kRHSViscous(DevMesh m, GasParams gp, cons
         real x[3], n[3];
 #pragma unroll
         for (int r = 0; r < 3; r++)
-            x[r] = m.fpts[((size_t)g * 3 + r) * F + f], n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
+            x[r] = fp.x(g, r), n[r] = fp.n(g, r);
         real UL[5], UR[5], GL[3][5], GR[3][5];
         L.eval(m, x, uRec, UL, GL);
         if (bnd)
@@ -1170,7 +1171,7 @@ __global__ void __launch_bounds__(128) kRHSViscous(DevMesh m, GasParams gp, cons
         }
         real Fv[5];
         viscousPointFlux(gp, UL, UR, GL, GR, n, dB, d0, bnd, bnd && type == BC_WALL, Fv);
-        const real wj = m.fwj[(size_t)g * F + f];
+        const real wj = fp.w(g);
 #pragma unroll
         for (int v = 0; v < 5; v++)
             acc[v] += Fv[v] * wj;

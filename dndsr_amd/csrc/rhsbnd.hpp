@@ -63,6 +63,7 @@ __global__ void __launch_bounds__(64 * G) kRHSBoundary(DevMesh m, GasParams gp, 
     const idx t = blockIdx.x * 64 + lane;
     const bool valid = t < m.nBnd;
     const idx f = m.bndFace[valid ? t : m.nBnd - 1];
+    const FacePts fp = bndPts(m, valid ? t : m.nBnd - 1);
     const size_t N = m.N, F = m.F;
     const idx cL = m.f2c[f];
     const int zone = m.fzone[f];
@@ -71,10 +72,10 @@ __global__ void __launch_bounds__(64 * G) kRHSBoundary(DevMesh m, GasParams gp, 
     for (int r = 0; r < 3; r++)
     {
         nm[r] = m.fmeanN[(size_t)r * F + f];
-        n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
-        x[r] = m.fpts[((size_t)g * 3 + r) * F + f];
+        n[r] = fp.n(g, r);
+        x[r] = fp.x(g, r);
     }
-    const real wj = m.fwj[(size_t)g * F + f];
+    const real wj = fp.w(g);
     const int type = m.bcType[zone];
     const real *far = m.bcVal + (size_t)zone * 5;
 #pragma unroll

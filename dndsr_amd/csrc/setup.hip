@@ -514,6 +514,31 @@ static void runSetup(Ctx &c)
     DNDSR_HIP_CHECK(hipFree(b));
 }
 
+// rows q of the face tables, in bndFace order
+__global__ void __launch_bounds__(256) kBndRows(DevMesh m, const real *__restrict__ src, real *__restrict__ dst, int rows)
+{
+    const idx t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= m.nBnd)
+        return;
+    const idx f = m.bndFace[t];
+    for (int q = 0; q < rows; q++)
+        dst[(size_t)q * m.nBnd + t] = src[(size_t)q * m.F + f];
+}
+static void setupBoundaryRows(Ctx &c)
+{
+    DevMesh &m = c.m;
+    if (m.nBnd == 0)
+        return;
+    const int nb = gridFor(m.nBnd, 256), G = m.G;
+    m.bpts = devAlloc<real>(c, (size_t)G * 3 * m.nBnd);
+    m.bnorm = devAlloc<real>(c, (size_t)G * 3 * m.nBnd);
+    m.bwj = devAlloc<real>(c, (size_t)G * m.nBnd);
+    kBndRows<<<nb, 256, 0, c.stream>>>(m, m.fpts, m.bpts, 3 * G);
+    kBndRows<<<nb, 256, 0, c.stream>>>(m, m.fnorm, m.bnorm, 3 * G);
+    kBndRows<<<nb, 256, 0, c.stream>>>(m, m.fwj, m.bwj, G);
+    DNDSR_HIP_CHECK(hipGetLastError());
+}
+
 void setupMetricsAndVR(Ctx &c)
 {
     const DevMesh &m = c.m;
@@ -539,6 +564,7 @@ void setupMetricsAndVR(Ctx &c)
         else
             throw std::runtime_error("maxOrder must be 1..3");
     }
+    setupBoundaryRows(c);
 }
 
 } // namespace dndsr

@@ -241,7 +241,7 @@ static void vrIterDiffM(Ctx &c, int nVars, const real *x, real *y)
 // mean): the basis values phi and inc = uB - u_i (LIN: the ghost's change along dx).  The own block
 // is read through rec(v, j) and, for LIN, the Jacobian direction through dx(v, j).
 template <int DIM, int NDOF, int NV, bool LIN, class Rec, class Dx>
-__device__ inline void boundaryPointInc(const DevMesh &m, idx f, int g, const real *mom, const real *cen, real isc,
+__device__ inline void boundaryPointInc(const DevMesh &m, idx f, const FacePts &fp, int g, const real *mom, const real *cen, real isc,
                                         const real *um, Rec rec, Dx dx, real (&phi)[NDOF - 1], real (&inc)[NV])
 {
     constexpr int M = NDOF - 1;
@@ -251,7 +251,7 @@ __device__ inline void boundaryPointInc(const DevMesh &m, idx f, int g, const re
 #pragma unroll
     for (int r = 0; r < 3; r++)
     {
-        xs[r] = m.fpts[((size_t)g * 3 + r) * F + f] - cen[r];
+        xs[r] = fp.x(g, r) - cen[r];
         if (DIM == 3 || r < 2)
             xs[r] *= isc;
     }
@@ -271,7 +271,7 @@ __device__ inline void boundaryPointInc(const DevMesh &m, idx f, int g, const re
         }
 #pragma unroll
         for (int r = 0; r < 3; r++)
-            n[r] = m.fnorm[((size_t)g * 3 + r) * F + f];
+            n[r] = fp.n(g, r);
         const real *far = m.bcVal + (size_t)zone * 5;
         const int type = m.bcType[zone];
         compressRecPart(um, uBL, ULf);
@@ -321,7 +321,7 @@ __device__ inline void boundaryFaceBCC(const DevMesh &m, idx f, const real *mom,
     for (int g = 0; g < m.G; g++)
     {
         real phi[M], inc[NV];
-        boundaryPointInc<DIM, NDOF, NV, false>(m, f, g, mom, cen, isc, um, rec, rec, phi, inc);
+        boundaryPointInc<DIM, NDOF, NV, false>(m, f, facePts(m, f), g, mom, cen, isc, um, rec, rec, phi, inc);
         const real fac = m.fwj[(size_t)g * m.F + f];
 #pragma unroll
         for (int j = 0; j < M; j++)
@@ -340,7 +340,8 @@ __device__ inline void boundaryFaceBCC(const DevMesh &m, idx f, const real *mom,
 // pass is bound by its chain of dependent loads and arithmetic, not by bandwidth.  A block is 64
 // faces with one wavefront per face point (two rounds of points above 8): the points' basis values
 // and increments go through LDS, then wavefront w forms the column v = w, w + NW, ... of BCC in point
-// order and applies A^-1.  35k triangles of a tetrahedral mesh at p1 38 us (one thread per face 51).
+// order and applies A^-1.  35k triangles of a tetrahedral mesh at p1: 38 us
+// with the points read from the face tables, one thread per face 51.
 template <int DIM, int NDOF, int NV, int MODE>
 __global__ void __launch_bounds__(512) kVRBndFace(DevMesh m, const real *__restrict__ uRec, const real *__restrict__ u,
                                                   const real *__restrict__ x, real *__restrict__ out)
@@ -351,6 +352,7 @@ __global__ void __launch_bounds__(512) kVRBndFace(DevMesh m, const real *__restr
     const idx t = blockIdx.x * 64 + lane;
     const bool valid = t < m.nBnd;
     const idx f = m.bndFace[valid ? t : m.nBnd - 1];
+    const FacePts fp = bndPts(m, valid ? t : m.nBnd - 1);
     const idx i = m.f2c[f];
     const size_t N = m.N, NB = m.nBnd;
     {
@@ -414,8 +416,8 @@ __global__ void __launch_bounds__(512) kVRBndFace(DevMesh m, const real *__restr
             if (g < m.G)
             {
                 real phi[M], inc[NV];
-                boundaryPointInc<DIM, NDOF, NV, MODE == 2>(m, f, g, mom, cen, isc, um, rec, dx, phi, inc);
-                const real fac = m.fwj[(size_t)g * m.F + f] * (w0 * w0);
+                boundaryPointInc<DIM, NDOF, NV, MODE == 2>(m, f, fp, g, mom, cen, isc, um, rec, dx, phi, inc);
+                const real fac = fp.w(g) * (w0 * w0);
                 real *row = sPt + (size_t)w * ROWS * 64 + lane;
 #pragma unroll
                 for (int j = 0; j < M; j++)
