@@ -598,6 +598,8 @@ int dndsr_vr_construct(dndsr_ctx *ctx, const dndsr_mesh_desc *md, const dndsr_vr
     m.globalVol = 0;
     for (real v : vol)
         m.globalVol += v;
+    if (m.s.SORInstead)
+        prepareSOR(c);
     c.haveMesh = true;
     CAPI_END
 }
@@ -752,7 +754,7 @@ int dndsr_set_vr_coeffs(dndsr_ctx *ctx, const double *AinvB, const double *Ainvb
     }
     upload(c, m.AinvB, B);
     upload(c, m.Ainvb, b);
-    c.sorFresh = false; // the copy in the order of the SOR lists is rebuilt
+    refreshSOR(c);
     DNDSR_HIP_CHECK(hipStreamSynchronize(c.stream));
     CAPI_END
 }

@@ -131,11 +131,11 @@ struct Ctx
     real *faceFlux = nullptr;   // [5][F]
     real *vrBnd = nullptr;      // [nVars][M][nBnd] A^-1 BCC of each boundary face (VR sweep boundary term)
     real *linRec = nullptr;     // [N][20] means and gradients (linear reconstruction on tetrahedra, facelin.hip)
-    // the SOR sweep's matrices in list order (vr.hip, sorMatrix): sweeps so far (up to 2), the copy,
-    // whether it matches the coefficients, and whether there was no memory for it
+    // the SOR sweep's matrices in list order (vr.hip, prepareSOR): sweeps before it was asked for, whether it
+    // was, and the copy, null without the memory for it
     int sorUse = 0;
+    bool sorTried = false;
     real *sorB = nullptr;
-    bool sorFresh = false, sorNoRoom = false;
     size_t faceFluxCap = 0;
     real *red = nullptr;        // reduction partials
     size_t redCap = 0;
@@ -221,6 +221,8 @@ void setupMetricsAndVR(Ctx &c);
 // ---- launchers (vr.hip)
 void launchVRIter(Ctx &c, int nVars, const real *uRec, real *uRecNew, const real *u, int mode, real relax);
 void launchVRSOR(Ctx &c, int nVars, real *uRec, const real *u, real relax);
+void prepareSOR(Ctx &c);
+void refreshSOR(Ctx &c);
 bool usesSubs2nd(const DevMesh &m);
 void launchVR2nd(Ctx &c, int nVars, const real *u, real *out);
 void launchVRIterDiff(Ctx &c, int nVars, const real *uRec, const real *u, const real *uRecDiff, real *uRecNew);

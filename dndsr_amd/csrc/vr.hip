@@ -493,7 +493,7 @@ __global__ void __launch_bounds__(64) kVRBndCell(DevMesh m, const real *__restri
 // streams each matrix row once in coalesced lines; the cells with one, whose boundary term depends
 // on the block accumulated so far, take one thread each (kVRSOR).  A colour is every other cell or
 // fewer, so in the caller's order each colour would fetch whole lines of A^-1 B for a part of their
-// cells: from its second sweep on a context keeps a copy of the matrices in list order (sorMatrix).
+// cells: a context that sweeps keeps a copy of the matrices in list order (prepareSOR).
 // ---------------------------------------------------------------------------
 template <int DIM, int NDOF, int NV>
 __global__ void __launch_bounds__(64) kVRSOR(DevMesh m, const idx *__restrict__ cells, idx nCells,
@@ -868,44 +868,64 @@ __global__ void __launch_bounds__(256) kPermuteRows(size_t N, int n, const idx *
         dst[(size_t)q * N + t] = src[(size_t)q * N + i];
 }
 
-// The matrices the SOR sweep streams.  The first sweep of a context reads them in the caller's cell
-// order; a context that sweeps again gets a copy in the order of the SOR lists, which it keeps (and
-// refreshes when the coefficients are replaced).  No copy while the stream is being captured (it would
-// allocate) or where the memory for it is not there.  61 x 53 x 47 hexahedra, p2: 309 us per sweep with
-// the copy and the tile form, 739 with a thread per cell on the caller's order.
-static CellList sorMatrix(Ctx &c)
+// The matrices the SOR sweep streams, copied to the order of the SOR lists once per context: at
+// construction with the setting SORInstead, else before its second sweep (one sweep does not earn the
+// copy: 585 us with the caller's order, 819 with the copy made first), but not under capture, which must
+// not allocate.  Until then, or without the memory, the sweep reads the caller's cell order.
+// prepareSOR returns with the copy complete, so sweeps on any stream may read it; replaced coefficients
+// refresh it in place (refreshSOR, synchronised by its caller), so a captured sweep reads them.
+// 61 x 53 x 47 hexahedra, p2: 309 us per sweep with the copy and the tile form, 739 with a thread per
+// cell on the caller's order.
+static void permuteSOR(Ctx &c, real *B)
 {
     const DevMesh &m = c.m;
     const size_t N = m.N, nB = (size_t)m.K * m.M * m.M, nb = (size_t)m.K * m.M;
-    CellList l;
-    l.B = m.AinvB + (size_t)m.M * m.M * N, l.b = m.Ainvb;
-    if (m.nColor < 2 || (c.sorUse < 2 && ++c.sorUse < 2))
-        return l;
-    if (!c.sorFresh)
+    const dim3 g(gridFor(m.N, 256), 8);
+    kPermuteRows<<<g, 256, 0, c.stream>>>(N, (int)nB, m.sorCells, m.AinvB + (size_t)m.M * m.M * N, B);
+    kPermuteRows<<<g, 256, 0, c.stream>>>(N, (int)nb, m.sorCells, m.Ainvb, B + nB * N);
+    DNDSR_HIP_CHECK(hipGetLastError());
+}
+void refreshSOR(Ctx &c)
+{
+    if (c.sorB)
+        permuteSOR(c, c.sorB);
+}
+void prepareSOR(Ctx &c)
+{
+    const DevMesh &m = c.m;
+    if (c.sorTried)
+        return;
+    c.sorTried = true;
+    if (m.nColor < 2 || usesSubs2nd(m))
+        return;
+    void *p = nullptr;
+    if (hipMalloc(&p, (size_t)m.K * m.M * (m.M + 1) * m.N * sizeof(real)) != hipSuccess)
+    {
+        (void)hipGetLastError();
+        return;
+    }
+    c.owned.push_back(p);
+    permuteSOR(c, static_cast<real *>(p));
+    DNDSR_HIP_CHECK(hipStreamSynchronize(c.stream));
+    c.sorB = static_cast<real *>(p);
+}
+
+static CellList sorMatrix(Ctx &c)
+{
+    const DevMesh &m = c.m;
+    const size_t N = m.N;
+    if (!c.sorTried && c.sorUse++ > 0)
     {
         hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
         DNDSR_HIP_CHECK(hipStreamIsCapturing(c.stream, &cap));
-        if (cap != hipStreamCaptureStatusNone || c.sorNoRoom)
-            return l;
-        if (!c.sorB)
-        {
-            void *p = nullptr;
-            if (hipMalloc(&p, (nB + nb) * N * sizeof(real)) != hipSuccess)
-            {
-                (void)hipGetLastError();
-                c.sorNoRoom = true;
-                return l;
-            }
-            c.owned.push_back(p);
-            c.sorB = static_cast<real *>(p);
-        }
-        const dim3 g(gridFor(m.N, 256), 8);
-        kPermuteRows<<<g, 256, 0, c.stream>>>(N, (int)nB, m.sorCells, m.AinvB + (size_t)m.M * m.M * N, c.sorB);
-        kPermuteRows<<<g, 256, 0, c.stream>>>(N, (int)nb, m.sorCells, m.Ainvb, c.sorB + nB * N);
-        DNDSR_HIP_CHECK(hipGetLastError());
-        c.sorFresh = true;
+        if (cap == hipStreamCaptureStatusNone)
+            prepareSOR(c);
     }
-    l.B = c.sorB, l.b = c.sorB + nB * N, l.byPos = true;
+    CellList l;
+    if (c.sorB)
+        l.B = c.sorB, l.b = c.sorB + (size_t)m.K * m.M * m.M * N, l.byPos = true;
+    else
+        l.B = m.AinvB + (size_t)m.M * m.M * N, l.b = m.Ainvb;
     return l;
 }
 

@@ -81,7 +81,8 @@ typedef struct
     const double *zoneDirWeight; /* host, [nBCZone][maxOrder+1] */
     /* SORInstead (VRSettings.hpp:43): the solver loops (dndsr_ssprk3, dndsr_implicit_euler_step)
      * sweep the reconstruction in place, multicolour SOR (dndsr_vr_iter mode 4), instead of
-     * by relaxed Jacobi.  0 = Jacobi. */
+     * by relaxed Jacobi.  0 = Jacobi.  The sweep's own copy of A^-1 B_f and A^-1 b_f (see
+     * dndsr_vr_iter) is then made by dndsr_vr_construct. */
     int SORInstead;
     /* subs2ndOrder (VRSettings.hpp:49-50), maxOrder 1 only: 0 = VR; 1 = Gauss rule, 2 = least
      * squares: every VR sweep (dndsr_vr_iter, any mode, and the solver loops) is replaced by a
@@ -168,6 +169,10 @@ int dndsr_d2h_cellfield(dndsr_ctx *ctx, const double *dev, double *hostRows, int
  *   uRec_i = (1-relax) uRec_i, then per face in cell-face order uRec_i += relax (...), the
  *   boundary term evaluated on the uRec_i accumulated so far; uRecNew is not used (may be
  *   NULL).  Equals the reference's serial sweep when cells are numbered colour by colour.
+ *   The sweep streams a copy of A^-1 B_f and A^-1 b_f in its own cell order, 8 K M (M + 1) bytes a
+ *   cell for K face slots and M coefficients: made at construction with SORInstead, else by the
+ *   context's second mode 4 call (which then synchronises its stream once), kept with the context and
+ *   refreshed in place by dndsr_set_vr_coeffs.  A call under capture makes no copy.
  * relax < 0 uses settings.jacobiRelax.
  * Replaces VariationalReconstruction<dim>::DoReconstructionIter,
  * src/CFV/VariationalReconstruction.hpp:984-992. */
