@@ -6,6 +6,7 @@
 // DoReconstructionIterDiff, :617-670.
 #include "gas.hpp"
 #include "internal.hpp"
+#include "memrule.hpp"
 
 namespace dndsr
 {
@@ -871,7 +872,7 @@ __global__ void __launch_bounds__(256) kPermuteRows(size_t N, int n, const idx *
 // The matrices the SOR sweep streams, copied to the order of the SOR lists once per context: at
 // construction with the setting SORInstead, else before its second sweep (one sweep does not earn the
 // copy: 585 us with the caller's order, 819 with the copy made first), but not under capture, which must
-// not allocate.  Until then, or without the memory, the sweep reads the caller's cell order.
+// not allocate.  Until then, or without room for it (roomForCopy), the sweep reads the caller's cell order.
 // prepareSOR returns with the copy complete, so sweeps on any stream may read it; replaced coefficients
 // refresh it in place (refreshSOR, synchronised by its caller), so a captured sweep reads them.
 // 61 x 53 x 47 hexahedra, p2: 309 us per sweep with the copy and the tile form, 739 with a thread per
@@ -889,6 +890,8 @@ void refreshSOR(Ctx &c)
 {
     if (c.sorB)
         permuteSOR(c, c.sorB);
+    else
+        c.sorTried = false; // there may be room now
 }
 void prepareSOR(Ctx &c)
 {
@@ -899,7 +902,12 @@ void prepareSOR(Ctx &c)
     if (m.nColor < 2 || usesSubs2nd(m))
         return;
     void *p = nullptr;
-    if (hipMalloc(&p, (size_t)m.K * m.M * (m.M + 1) * m.N * sizeof(real)) != hipSuccess)
+    const size_t bytes = (size_t)m.K * m.M * (m.M + 1) * m.N * sizeof(real);
+    size_t free = 0, total = 0;
+    DNDSR_HIP_CHECK(hipMemGetInfo(&free, &total));
+    if (!roomForCopy(free, bytes, m.N))
+        return;
+    if (hipMalloc(&p, bytes) != hipSuccess)
     {
         (void)hipGetLastError();
         return;

@@ -172,7 +172,8 @@ int dndsr_d2h_cellfield(dndsr_ctx *ctx, const double *dev, double *hostRows, int
  *   The sweep streams a copy of A^-1 B_f and A^-1 b_f in its own cell order, 8 K M (M + 1) bytes a
  *   cell for K face slots and M coefficients: made at construction with SORInstead, else by the
  *   context's second mode 4 call (which then synchronises its stream once), kept with the context and
- *   refreshed in place by dndsr_set_vr_coeffs.  A call under capture makes no copy.
+ *   refreshed in place by dndsr_set_vr_coeffs.  A call under capture makes no copy, nor
+ *   one that would not leave three times its size and 16 KB a cell of device memory free.
  * relax < 0 uses settings.jacobiRelax.
  * Replaces VariationalReconstruction<dim>::DoReconstructionIter,
  * src/CFV/VariationalReconstruction.hpp:984-992. */
