@@ -6,20 +6,23 @@
 // per side: the basis row times the coefficients is G (x - cent - scale moment), G = uRec / scale, so a
 // side is its mean u, the gradient G and the offset (26 values in 3-D, 23 on tetrahedra), read once and
 // reduced at once to its states at the face's points (on a triangle, whose points are affine
-// combinations of its vertices, to the state at one vertex and its changes along two sides); of the
-// gradients only the mean of the two sides lives on, for the viscous flux.  The tile kernels of the higher orders, one wavefront per point
+// combinations of its vertices, to the mean, the offset at one vertex and the changes along two sides: the
+// mean is added point by point, a state rounded once for all six points shifted the whole face's flux and
+// raised the residual's error by half); of the gradients only the mean of the two sides lives on, for the
+// viscous flux.  The tile kernels of the higher orders, one wavefront per point
 // and the sides staged in LDS, re-read 80 rows of it there and left the viscous flux to a second pass
 // with all its gathers.
 //
-// On a triangle the unit normal is one for the face and the points come from the vertices, so 13
-// values per face (vertices, mean normal, area) replace the 42 of the point tables; neighbours of an
+// On a triangle the unit normal is one for the face, its six weights are two values, and the points come
+// from the vertices, so 14 values per face replace the 42 of the point tables (normal and weights are
+// read from those tables: the mean normal and the area carry a rounding of their own); neighbours of an
 // unstructured mesh are gathered from cell records of 160 + 32 bytes in 16-byte loads, one or two
 // cache lines each, instead of 27 scattered rows (the address pipeline, one line per lane and load,
 // was the tile kernel's bound there).  The records are written by a pass over the cells (kLinPack).
 // Meshes of quadrilaterals or hexahedra are numbered so that neighbouring faces have neighbouring
 // cells: their rows are coalesced as they stand.
 //
-// Measured: 945k tetrahedra (1.9M faces), viscous Roe: 171 us + 72 us for the records, against 288 us
+// Measured: 945k tetrahedra (1.9M faces), viscous Roe: 175 us + 76 us for the records, against 288 us
 // (tile kernel) + 424 us (viscous pass); 333k faces of a mixed 2-D mesh, viscous Roe: 26 us against
 // 33 + 37 us; 744k hexahedral faces, inviscid Roe: 69 us against 84 us.
 #include "geom.hpp"
@@ -208,14 +211,18 @@ struct LinSide
         }
         c[0] = c[1] = c[2] = 0;
     }
-    // the state at x: u + G (x - centre - scale moment), the small offset formed first
-    __device__ __forceinline__ void at(const real *x, real *U) const
+    // the state at x: u + off, off = G (x - centre - scale moment), the small difference formed first
+    __device__ __forceinline__ void off(const real *x, real *U) const
     {
         real e[DIM];
 #pragma unroll
         for (int k = 0; k < DIM; k++)
             e[k] = (x[k] - c[k]) - d[k];
         along(e, U);
+    }
+    __device__ __forceinline__ void at(const real *x, real *U) const
+    {
+        off(x, U);
 #pragma unroll
         for (int v = 0; v < 5; v++)
             U[v] += u[v];
@@ -234,13 +241,9 @@ struct LinSide
     }
 };
 
-constexpr real triWeightSum()
-{
-    real s = 0;
-    for (int g = 0; g < 6; g++)
-        s += kTri6[2][g];
-    return s;
-}
+static_assert(kTri6[2][0] == kTri6[2][1] && kTri6[2][0] == kTri6[2][2] && kTri6[2][3] == kTri6[2][4] &&
+                  kTri6[2][3] == kTri6[2][5],
+              "the weights of points 0-2 and 3-5");
 
 // flux forms that read deltaLambdaCell (the H-correction fixes and HLLE+)
 constexpr bool readsDeltaLambda(int rs) { return rs == RS_HLLEP || rs == RS_HLLEP_V1 || rs == RS_Roe_M6 || rs == RS_Roe_M8; }
@@ -256,7 +259,8 @@ __device__ __forceinline__ bool linFace(const DevMesh &m, const GasParams &gp, c
     constexpr int NS = TRI ? 3 : G;
     const size_t F = m.F;
     const uint32_t fu = (uint32_t)f;
-    // the points (or the vertices of a triangle), the normal and the shift into the right cell's frame
+    // the points (or the vertices of a triangle), the (first point's) normal and the shift into the right
+    // cell's frame
     real x[NS][3], n[3], sh[3];
     if constexpr (TRI)
     {
@@ -281,16 +285,16 @@ __device__ __forceinline__ bool linFace(const DevMesh &m, const GasParams &gp, c
     {
         sh[r] = ldu(m.fshift + (size_t)r * F, fu);
         if constexpr (ONE_N || BATCH)
-            n[r] = ldu(m.fmeanN + (size_t)r * F, fu);
+            n[r] = ldu((ONE_N ? m.fnorm : m.fmeanN) + (size_t)r * F, fu);
     }
-    real wArea = 0, idist = 0;
+    real w0 = 0, w1 = 0, idist = 0;
     if constexpr (TRI)
-        wArea = ldu(m.farea, fu) * (1.0 / triWeightSum());
+        w0 = ldu(m.fwj, fu), w1 = ldu(m.fwj + (size_t)3 * F, fu);
     if constexpr (VIS)
         idist = ldu(m.linDist, fu);
     if (cR < 0) // boundary faces: kRHSBoundary and the viscous pass over the boundary list
         return false;
-    real SL[NS][5], SR[NS][5], Gm[DIM][5];
+    real SL[NS][5], SR[NS][5], Gm[DIM][5], mL[5], mR[5];
     RoeBatchFace bf;
     {
         LinSide<DIM, TRI> L, R;
@@ -299,7 +303,7 @@ __device__ __forceinline__ bool linFace(const DevMesh &m, const GasParams &gp, c
 #pragma unroll
         for (int k = 0; k < NS; k++)
         {
-            if (TRI && k > 0) // a triangle: the state at its first vertex and its changes along two sides
+            if (TRI && k > 0) // a triangle: the offset at its first vertex and the changes along two sides
             {
                 const real e[3] = {x[k][0] - x[0][0], x[k][1] - x[0][1], x[k][2] - x[0][2]};
                 L.along(e, SL[k]);
@@ -307,11 +311,22 @@ __device__ __forceinline__ bool linFace(const DevMesh &m, const GasParams &gp, c
                 continue;
             }
             real xr[3];
-            L.at(x[k], SL[k]);
 #pragma unroll
             for (int r = 0; r < DIM; r++)
                 xr[r] = x[k][r] + sh[r];
-            R.at(xr, SR[k]);
+            if constexpr (TRI)
+            {
+                L.off(x[k], SL[k]);
+                R.off(xr, SR[k]);
+#pragma unroll
+                for (int v = 0; v < 5; v++)
+                    mL[v] = L.u[v], mR[v] = R.u[v];
+            }
+            else
+            {
+                L.at(x[k], SL[k]);
+                R.at(xr, SR[k]);
+            }
         }
         if constexpr (VIS)
 #pragma unroll
@@ -339,10 +354,10 @@ __device__ __forceinline__ bool linFace(const DevMesh &m, const GasParams &gp, c
 #pragma unroll
             for (int v = 0; v < 5; v++)
             {
-                UL[v] = SL[0][v] + (b1 * SL[1][v] + b2 * SL[2][v]);
-                UR[v] = SR[0][v] + (b1 * SR[1][v] + b2 * SR[2][v]);
+                UL[v] = mL[v] + (SL[0][v] + (b1 * SL[1][v] + b2 * SL[2][v]));
+                UR[v] = mR[v] + (SR[0][v] + (b1 * SR[1][v] + b2 * SR[2][v]));
             }
-            wj = kTri6[2][g] * wArea;
+            wj = g < 3 ? w0 : w1;
         }
         else
         {
