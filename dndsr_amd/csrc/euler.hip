@@ -1351,7 +1351,7 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
     {
         KernelTimer kt(c, K_RHS_FACE); // inviscid interior, periodic and boundary faces
         if (linear)
-            launchRHSFaceLinear(c, gp, u, uRec, dlc, ff, faceFluxBuf == nullptr);
+            launchRHSFaceLinear(c, gp, u, uRec, dlc, ff);
         else if (m.dim == 2)
         {
             if (!uRec || m.P == 1)

@@ -15,23 +15,19 @@
 //
 // On a triangle the unit normal is one for the face, its six weights are two values, and the points come
 // from the vertices, so 14 values per face replace the 42 of the point tables (normal and weights are
-// read from those tables: the mean normal and the area carry a rounding of their own); neighbours of an
-// unstructured mesh are gathered from cell records of 160 + 32 bytes in 16-byte loads, one or two
-// cache lines each, instead of 27 scattered rows (the address pipeline, one line per lane and load,
-// was the tile kernel's bound there).  The records are written by a pass over the cells (kLinPack).
-// Meshes of quadrilaterals or hexahedra are numbered so that neighbouring faces have neighbouring
-// cells: their rows are coalesced as they stand.
+// read from those tables: the mean normal and the area carry a rounding of their own).  Each side's rows of
+// u and uRec are read as they stand: 160-byte cell records written by a pass of their own before were
+// slower in every cell order (384k tetrahedra, viscous residual: Morton order 151 us with records, 121
+// with rows; grouped by colour 178 / 165; reverse Cuthill-McKee 166 / 131).
 //
-// Measured: 945k tetrahedra (1.9M faces), viscous Roe: 175 us + 76 us for the records, against 288 us
-// (tile kernel) + 424 us (viscous pass); 333k faces of a mixed 2-D mesh, viscous Roe: 26 us against
-// 33 + 37 us; 744k hexahedral faces, inviscid Roe: 69 us against 84 us.
+// Measured: 945k tetrahedra (1.9M faces), viscous Roe: 199 us, against 288 us (tile kernel) + 424 us
+// (viscous pass); 333k faces of a mixed 2-D mesh, viscous Roe: 26 us against 33 + 37 us; 744k hexahedral
+// faces, inviscid Roe: 77 us against 84 us.
 #include "geom.hpp"
 #include "rhsbnd.hpp"
 
 namespace dndsr
 {
-constexpr int kLinRow = 20;
-
 struct ViscGas
 {
     real g1, Cp, kOverMu;
@@ -90,30 +86,6 @@ __device__ __forceinline__ void viscousPointLin(const GasParams &gp, const ViscG
     Fv[4] = e;
 }
 
-// u [5] and G [3][5] of every cell, cell-major
-__global__ void __launch_bounds__(256) kLinPack(DevMesh m, const real *__restrict__ u, const real *__restrict__ uRec,
-                                                real *__restrict__ out)
-{
-    const idx i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m.N)
-        return;
-    const size_t N = m.N;
-    const real isc = m.iscale[i];
-    real r[kLinRow];
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-    {
-        r[v] = u[(size_t)v * N + i];
-#pragma unroll
-        for (int d = 0; d < 3; d++)
-            r[5 + d * 5 + v] = uRec[((size_t)v * 3 + d) * N + i] * isc;
-    }
-    double2 *o = reinterpret_cast<double2 *>(out + (size_t)i * kLinRow);
-#pragma unroll
-    for (int q = 0; q < kLinRow / 2; q++)
-        o[q] = make_double2(r[2 * q], r[2 * q + 1]);
-}
-
 // the cells' constants: rows of 4 (tetrahedra, whose vertex mean is their barycentre: centre, 1 / scale) or
 // of 8 (centre, 1 / scale, scale times moment, 0)
 __global__ void __launch_bounds__(256) kLinCentre(DevMesh m, real *__restrict__ linC, int row)
@@ -151,9 +123,8 @@ template <int DIM, bool TRI>
 struct LinSide
 {
     real u[5], G[DIM][5], c[3], d[DIM];
-    // rec: the cell records (linRec), or null: the rows of u and uRec
     __device__ __forceinline__ void load(const DevMesh &m, idx i, const real *__restrict__ u_,
-                                         const real *__restrict__ uRec, const real *__restrict__ rec)
+                                         const real *__restrict__ uRec)
     {
         const size_t N = m.N;
 #pragma unroll
@@ -170,26 +141,6 @@ struct LinSide
                 d[0] = e.x, d[1] = e.y;
                 if constexpr (DIM == 3)
                     d[DIM - 1] = reinterpret_cast<const real *>(q)[6];
-            }
-            if (TRI && rec)
-            {
-                real r[kLinRow];
-                const double2 *p = reinterpret_cast<const double2 *>(rec + (size_t)i * kLinRow);
-#pragma unroll
-                for (int k = 0; k < kLinRow / 2; k++)
-                {
-                    const double2 t = p[k];
-                    r[2 * k] = t.x, r[2 * k + 1] = t.y;
-                }
-#pragma unroll
-                for (int v = 0; v < 5; v++)
-                {
-                    u[v] = r[v];
-#pragma unroll
-                    for (int k = 0; k < DIM; k++)
-                        G[k][v] = r[5 + k * 5 + v];
-                }
-                return;
             }
 #pragma unroll
             for (int v = 0; v < 5; v++)
@@ -251,8 +202,7 @@ constexpr bool readsDeltaLambda(int rs) { return rs == RS_HLLEP || rs == RS_HLLE
 // the flux of face f, times -1 and the area, summed over its points; false for a boundary face
 template <int DIM, int G, int RS, bool BATCH, bool VIS, bool TRI>
 __device__ __forceinline__ bool linFace(const DevMesh &m, const GasParams &gp, const real *__restrict__ u,
-                                        const real *__restrict__ uRec, const real *__restrict__ rec,
-                                        const real *__restrict__ dlc, idx f, idx cL, idx cR, real (&acc)[5])
+                                        const real *__restrict__ uRec, const real *__restrict__ dlc, idx f, idx cL, idx cR, real (&acc)[5])
 {
     constexpr bool ONE_N = TRI || DIM == 2; // one normal per face
     static_assert(ONE_N || !VIS, "quadrilateral faces keep their own viscous pass");
@@ -298,8 +248,8 @@ __device__ __forceinline__ bool linFace(const DevMesh &m, const GasParams &gp, c
     RoeBatchFace bf;
     {
         LinSide<DIM, TRI> L, R;
-        L.load(m, cL, u, uRec, rec);
-        R.load(m, cR, u, uRec, rec);
+        L.load(m, cL, u, uRec);
+        R.load(m, cR, u, uRec);
 #pragma unroll
         for (int k = 0; k < NS; k++)
         {
@@ -405,14 +355,14 @@ __device__ __forceinline__ bool linFace(const DevMesh &m, const GasParams &gp, c
 template <int DIM, int G, int RS, bool BATCH, bool VIS, bool TRI>
 __global__ void __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(2)))
 kRHSFaceLin(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__restrict__ uRec,
-            const real *__restrict__ rec, const real *__restrict__ dlc, real *__restrict__ fflux)
+            const real *__restrict__ dlc, real *__restrict__ fflux)
 {
     const idx f = xcdTile(blockIdx.x, gridDim.x) * 64 + (idx)threadIdx.x;
     if (f >= m.F)
         return;
     const idx cL = ldu(m.f2c, (uint32_t)f), cR = ldu(m.f2c + m.F, (uint32_t)f);
     real acc[5];
-    if (!linFace<DIM, G, RS, BATCH, VIS, TRI>(m, gp, u, uRec, rec, dlc, f, cL, cR, acc))
+    if (!linFace<DIM, G, RS, BATCH, VIS, TRI>(m, gp, u, uRec, dlc, f, cL, cR, acc))
         return;
 #pragma unroll
     for (int v = 0; v < 5; v++)
@@ -448,7 +398,7 @@ kRHSCellLin(DevMesh m, GasParams gp, const real *__restrict__ u, const real *__r
     if (f >= 0)
     {
         w = right ? -1.0 : 1.0;
-        if (!linFace<DIM, G, RS, BATCH, VIS, TRI>(m, gp, u, uRec, nullptr, dlc, f, right ? o : i, right ? i : o, t))
+        if (!linFace<DIM, G, RS, BATCH, VIS, TRI>(m, gp, u, uRec, dlc, f, right ? o : i, right ? i : o, t))
 #pragma unroll
             for (int v = 0; v < 5; v++)
                 t[v] = fflux[v * F + f];
@@ -497,7 +447,7 @@ bool rhsLinearRule(const DevMesh &m)
     return m.dim == 2 ? (m.G == 2 || m.G == 3) : (m.faceType == E_TRI3 ? m.G == 6 : m.G == 4);
 }
 
-// mesh constants and the cell records' memory, with the metrics
+// mesh constants, with the metrics
 void setupLinear(Ctx &c)
 {
     DevMesh &m = c.m;
@@ -508,8 +458,6 @@ void setupLinear(Ctx &c)
         const int row = m.faceType == E_TRI3 ? 4 : 8;
         m.linC = devAlloc<real>(c, row * (size_t)m.N);
         kLinCentre<<<gridFor(m.N, 256), 256, 0, c.stream>>>(m, m.linC, row);
-        if (m.faceType == E_TRI3)
-            c.linRec = devAlloc<real>(c, kLinRow * (size_t)m.N);
     }
     if (rhsLinearViscous(m))
     {
@@ -521,7 +469,7 @@ void setupLinear(Ctx &c)
 
 struct LinArgs
 {
-    const real *u, *uRec, *rec, *dlc;
+    const real *u, *uRec, *dlc;
     real *ff;
     // the one-pass form of small meshes
     real *rhs = nullptr;
@@ -551,7 +499,7 @@ static void linLaunch(Ctx &c, const GasParams &gp, const LinArgs &a)
     if constexpr (TRI || DIM == 2)
         if (gp.viscous)
             kern = kRHSFaceLin<DIM, G, RS, BATCH, true, TRI>;
-    kern<<<gridFor(c.m.F, 64), 64, 0, c.stream>>>(c.m, gp, a.u, a.uRec, a.rec, a.dlc, a.ff);
+    kern<<<gridFor(c.m.F, 64), 64, 0, c.stream>>>(c.m, gp, a.u, a.uRec, a.dlc, a.ff);
     DNDSR_HIP_CHECK(hipGetLastError());
     rhsBoundaryLaunch<DIM, DIM + 1, G, RS, BATCH>(c, gp, a.u, a.uRec, a.dlc, a.ff);
 }
@@ -606,25 +554,16 @@ static void linRule(Ctx &c, const GasParams &gp, const LinArgs &a)
         linDispatch<3, 4, false>(c, gp, a);
 }
 
-void launchRHSFaceLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff,
-                         bool pack)
+void launchRHSFaceLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff)
 {
-    DevMesh &m = c.m;
-    LinArgs a{u, uRec, nullptr, dlc, ff};
-    if (uRec && pack && c.linRec)
-    {
-        kLinPack<<<gridFor(m.N, 256), 256, 0, c.stream>>>(m, u, uRec, c.linRec);
-        DNDSR_HIP_CHECK(hipGetLastError());
-        a.rec = c.linRec;
-    }
-    linRule(c, gp, a);
+    linRule(c, gp, LinArgs{u, uRec, dlc, ff});
 }
 
 // Cells up to which the one-pass residual is taken (up to four faces per cell, the viscous flux in the
-// linear pass).  Ten SSP-RK3 steps, face pass and gather against one pass: 4 096 quadrilaterals
-// 487 / 431 us, 16 384 537 / 545, 32 400 678 / 656, 65 536 963 / 1208; 8 192 triangles 512 / 427, 32 768
-// 648 / 608; three steps on tetrahedra, whose records it also saves: 3 072 244 / 184, 16 464 304 / 261,
-// 34 992 418 / 388, 63 888 530 / 548.
+// linear pass).  Ten SSP-RK3 steps, face pass and gather against one pass: 9 000 quadrilaterals
+// 503 / 459 us, 16 384 508 / 520, 24 000 584 / 615, 32 400 648 / 620, 65 536 963 / 1208; 16 256 triangles
+// 515 / 478, 32 512 629 / 584; three steps on tetrahedra: 1 296 201 / 169, 10 368 224 / 196, 29 478
+// 306 / 294.
 constexpr idx kSmallRHS = 32768;
 bool rhsCellSize(const DevMesh &m)
 {
@@ -644,8 +583,7 @@ bool rhsCellRule(const Ctx &c, const real *u, const real *uRec, const real *dlc,
 void launchRHSCellLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff,
                          real *rhs, const StageUpdate &stage, int *nonFinite)
 {
-    LinArgs a{u, uRec, nullptr, dlc, ff, rhs, &stage, nonFinite};
-    linRule(c, gp, a);
+    linRule(c, gp, LinArgs{u, uRec, dlc, ff, rhs, &stage, nonFinite});
 }
 
 } // namespace dndsr

@@ -130,7 +130,6 @@ struct Ctx
     // scratch owned by the context (grown on demand, freed at destroy)
     real *faceFlux = nullptr;   // [5][F]
     real *vrBnd = nullptr;      // [nVars][M][nBnd] A^-1 BCC of each boundary face (VR sweep boundary term)
-    real *linRec = nullptr;     // [N][20] means and gradients (linear reconstruction on tetrahedra, facelin.hip)
     // the SOR sweep's matrices in list order (vr.hip, prepareSOR): sweeps before it was asked for, whether it
     // was, and the copy, null without the memory for it
     int sorUse = 0;
@@ -249,8 +248,7 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
                    real *rhs, const StageUpdate *stage = nullptr, real *faceFluxBuf = nullptr,
                    bool flagNonFinite = true);
 // ---- launchers (facelin.hip): fluxes (inviscid and viscous) of the interior faces and inviscid boundary
-// fluxes with a linear or no reconstruction, for the face rules rhsLinearRule names; pack: the
-// context's cell records may be used (else the cell rows are read directly)
+// fluxes with a linear or no reconstruction, for the face rules rhsLinearRule names
 bool rhsLinearRule(const DevMesh &m);
 bool rhsLinearViscous(const DevMesh &m);
 void setupLinear(Ctx &c);
@@ -263,8 +261,7 @@ void launchRHSCellLinear(Ctx &c, const GasParams &gp, const real *u, const real 
                          real *rhs, const StageUpdate &stage, int *nonFinite);
 // the viscous flux (euler.hip) of all faces, or of the boundary faces only
 void launchRHSViscous(Ctx &c, const GasParams &gp, const real *u, const real *uRec, real *ff, bool bndOnly);
-void launchRHSFaceLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff,
-                         bool pack);
+void launchRHSFaceLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff);
 void launchLUSGSInit(Ctx &c, const real *dTau, real dt, real alphaDiag, const real *lambdaFace, real *jdiag);
 // a sweep of the transposed scalar LU-SGS matrix (the adjoint preconditioner), FP64
 void launchSGSSweepT64(Ctx &c, const GasParams &gp, real alphaDiag, const real *rhs, const real *u, const real *uInc,
