@@ -1342,7 +1342,7 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
         throw std::runtime_error("viscous residual needs prGas > 0, Rgas > 0 and muGas >= 0");
     // first-order and linear reconstructions: the interior faces' whole flux in one pass
     const bool linear = (!uRec || m.P == 1) && rhsLinearRule(m);
-    if (linear && !faceFluxBuf && rhsCellRule(c, u, uRec, dlc, rhs, stage))
+    if (linear && !faceFluxBuf && rhsCellRule(c, gp.viscous != 0, u, uRec, dlc, rhs, stage))
     {
         launchRHSCellLinear(c, gp, u, uRec, dlc, ff, rhs, stage ? *stage : StageUpdate{},
                             flagNonFinite ? c.nonFinite : nullptr);

@@ -563,17 +563,21 @@ void launchRHSFaceLinear(Ctx &c, const GasParams &gp, const real *u, const real 
 // linear pass).  Ten SSP-RK3 steps, face pass and gather against one pass: 9 000 quadrilaterals
 // 503 / 459 us, 16 384 508 / 520, 24 000 584 / 615, 32 400 648 / 620, 65 536 963 / 1208; 16 256 triangles
 // 515 / 478, 32 512 629 / 584; three steps on tetrahedra: 1 296 201 / 169, 10 368 224 / 196, 29 478
-// 306 / 294.
-constexpr idx kSmallRHS = 32768;
+// 306 / 294.  In 2-D the viscous flux moves the crossover by no more than the spread of the mesh kinds (single
+// residuals: 18 200 quadrilaterals 11.1 / 9.7 us, 24 000 10.5 / 11.8; 24 576 triangles 10.5 / 9.9, 32 512
+// 10.5 / 10.9; mixed bounded cells 9 000 21.2 / 19.5, 25 500 23.7 / 24.5).  On tetrahedra, whose viscous
+// one-pass kernel fills the registers, the line is one wavefront (16 cells) per SIMD: 13 182 cells
+// 13.0 / 13.1, 16 464 13.5 / 17.4, 29 478 16.5 / 21.1; bounded 16 464 38.6 / 42.2.
+constexpr idx kSmallRHS = 32768, kSmallRHSTetVisc = 16384;
 bool rhsCellSize(const DevMesh &m)
 {
     return m.N <= kSmallRHS && m.K <= 4 && rhsLinearRule(m) && rhsLinearViscous(m);
 }
-bool rhsCellRule(const Ctx &c, const real *u, const real *uRec, const real *dlc, const real *rhs,
+bool rhsCellRule(const Ctx &c, bool viscous, const real *u, const real *uRec, const real *dlc, const real *rhs,
                  const StageUpdate *stage)
 {
     const DevMesh &m = c.m;
-    if (!rhsCellSize(m) || (stage && stage->u && (!stage->out || stage->out == stage->u)))
+    if (!rhsCellSize(m) || (viscous && m.dim == 3 && m.N > kSmallRHSTetVisc) || (stage && stage->u && (!stage->out || stage->out == stage->u)))
         return false;
     // an array that is read must not be written before every block has read it
     const size_t N = m.N;

@@ -252,10 +252,10 @@ void launchEvalRHS(Ctx &c, const GasParams &gp, const real *u, const real *uRec,
 bool rhsLinearRule(const DevMesh &m);
 bool rhsLinearViscous(const DevMesh &m);
 void setupLinear(Ctx &c);
-// the one-pass form of small meshes: whether the mesh takes it, whether a call does (its output apart
-// from what it reads), and the launch
+// the one-pass form of small meshes: whether the mesh may take it, whether a call does (its flux and its
+// output apart from what it reads), and the launch
 bool rhsCellSize(const DevMesh &m);
-bool rhsCellRule(const Ctx &c, const real *u, const real *uRec, const real *dlc, const real *rhs,
+bool rhsCellRule(const Ctx &c, bool viscous, const real *u, const real *uRec, const real *dlc, const real *rhs,
                  const StageUpdate *stage);
 void launchRHSCellLinear(Ctx &c, const GasParams &gp, const real *u, const real *uRec, const real *dlc, real *ff,
                          real *rhs, const StageUpdate &stage, int *nonFinite);

@@ -32,8 +32,9 @@ def _mesh(kind):
                            seed=3), [bc.BC_WALL, bc.BC_WALL_INVIS]
     if kind == "quad33k":  # above both limits
         return mm.periodic_quad_grid(183, 181, 1.0, 0.8, jitter=0.1, seed=3), None
-    return mm.tet_grid(18, 18, 17, 1.0, 1.0, 1.0, periodic=(True, False, True), zones=zones, jitter=0.05,
-                       seed=3), [bc.BC_WALL, bc.BC_WALL_INVIS]  # 33 048 cells
+    n = dict(tet16k=(14, 14, 14), tet33k=(18, 18, 17))[kind]  # above the viscous limit of tetrahedra, above both
+    return mm.tet_grid(*n, 1.0, 1.0, 1.0, periodic=(True, False, True), zones=zones, jitter=0.05,
+                       seed=3), [bc.BC_WALL, bc.BC_WALL_INVIS]
 
 
 def _setup(kind, rs, viscous):
@@ -51,7 +52,7 @@ def _setup(kind, rs, viscous):
 
 @pytest.mark.parametrize("viscous", [False, True])
 @pytest.mark.parametrize("rs", ["Roe", "HLLEP"])
-@pytest.mark.parametrize("kind", ["quad1", "tri", "mixed", "tet", "quad33k", "tet33k"])
+@pytest.mark.parametrize("kind", ["quad1", "tri", "mixed", "tet", "quad33k", "tet16k", "tet33k"])
 def test_same_as_two_passes(require_gpu, kind, rs, viscous):
     from dndsr_amd._lib import check, lib
     from dndsr_amd.cfv import _ptr
@@ -76,7 +77,7 @@ def test_same_as_two_passes(require_gpu, kind, rs, viscous):
         assert rel_l2(g.to_host(over), b) <= TOL
 
 
-@pytest.mark.parametrize("kind", ["quad1", "mixed", "tet", "quad33k"])
+@pytest.mark.parametrize("kind", ["quad1", "mixed", "tet", "tet16k", "quad33k"])
 def test_steps_match_oracle(require_gpu, kind):
     import pyoracle as po
     print(f"\n[small pass] steps {kind}", flush=True)
