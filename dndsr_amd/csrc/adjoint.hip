@@ -67,48 +67,6 @@ __device__ inline void cellBasisGradAt(const DevMesh &m, idx c, const real *x, c
     }
 }
 
-// value and gradient of cell c's reconstruction at x (+ shift), as the viscous pass
-template <int DIM, int NDOF>
-__device__ inline void cellValGradAt(const DevMesh &m, idx c, const real *x, const real *shift, const real *u,
-                                     const real *uRec, real *U, real (*G)[5])
-{
-    constexpr int M = NDOF - 1;
-    const size_t N = m.N;
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-    {
-        U[v] = u[(size_t)v * N + c];
-#pragma unroll
-        for (int d = 0; d < 3; d++)
-            G[d][v] = 0;
-    }
-    if (!uRec)
-        return;
-    real phi[M > 0 ? M : 1], dphi[DIM][M > 0 ? M : 1];
-    cellBasisGradAt<DIM, NDOF>(m, c, x, shift, phi, dphi);
-#pragma unroll
-    for (int v = 0; v < 5; v++)
-    {
-        real a = 0, g[DIM];
-#pragma unroll
-        for (int d = 0; d < DIM; d++)
-            g[d] = 0;
-#pragma unroll
-        for (int j = 0; j < M; j++)
-        {
-            const real r = ldu(uRec + (size_t)(v * M + j) * N, (uint32_t)c);
-            a += phi[j] * r;
-#pragma unroll
-            for (int d = 0; d < DIM; d++)
-                g[d] += dphi[d][j] * r;
-        }
-        U[v] += a;
-#pragma unroll
-        for (int d = 0; d < DIM; d++)
-            G[d][v] = g[d];
-    }
-}
-
 // value, gradient and geometry of an interior face point, shared by the point and face kernels
 template <int DIM, int NDOF>
 struct AdjSide

@@ -1274,19 +1274,18 @@ static void rhsDispatch(Ctx &c, const GasParams &gp, const real *u, const real *
 {
     constexpr int G1 = DIM == 2 ? 2 : 4, G2 = DIM == 2 ? 3 : 9;
     constexpr bool LIN = NDOF == DIM + 1; // linear: all rules but the 9-point one take the kernel of facelin.hip
-    if (c.m.G == G2 && (!LIN || DIM == 3))
-        rhsDispatchRS<DIM, NDOF, G2>(c, gp, u, uRec, dlc, ff);
-    else if constexpr (!LIN)
+    if constexpr (!LIN || DIM == 3)
+        if (c.m.G == G2)
+            return rhsDispatchRS<DIM, NDOF, G2>(c, gp, u, uRec, dlc, ff);
+    if constexpr (!LIN)
     {
         if (c.m.G == G1)
-            rhsDispatchRS<DIM, NDOF, G1>(c, gp, u, uRec, dlc, ff);
-        else if (DIM == 3 && c.m.G == 6)
-            rhsDispatchRS<DIM, NDOF, 6>(c, gp, u, uRec, dlc, ff);
-        else
-            throw std::runtime_error(kBadFaceRule);
+            return rhsDispatchRS<DIM, NDOF, G1>(c, gp, u, uRec, dlc, ff);
+        if constexpr (DIM == 3)
+            if (c.m.G == 6)
+                return rhsDispatchRS<DIM, NDOF, 6>(c, gp, u, uRec, dlc, ff);
     }
-    else
-        throw std::runtime_error(kBadFaceRule);
+    throw std::runtime_error(kBadFaceRule);
 }
 
 void launchRHSViscous(Ctx &c, const GasParams &gp, const real *u, const real *uRec, real *ff, bool bndOnly)

@@ -236,10 +236,8 @@ __host__ __device__ inline void sideFlux(const T *U, const real *n, real gamma, 
     physFlux(U, v, n, p, F);
 }
 
-// Full Riemann flux at one point with its own Roe average of the mean states.
-// Returns lam0/123/4 (after entropy fix) like the reference.
-// Point part of the Riemann flux, given the face's Roe average of the mean states
-// (the average depends only on ULm / URm, so a face computes it once).
+// Point part of the Riemann flux (lam0/123/4 after the entropy fix, like the reference), given the
+// face's Roe average of the mean states (it depends only on ULm / URm, so a face computes it once).
 template <int RS, typename T>
 __host__ __device__ inline void riemannFluxR(const T *UL, const T *UR, const RoeAveT<T> &r, const real *n,
                                              const GasParams &gp, real dLambda, T *F, T &lam0, T &lam123, T &lam4)
@@ -363,15 +361,6 @@ __host__ __device__ inline void riemannFluxR(const T *UL, const T *UR, const Roe
             }
         }
     }
-}
-
-template <int RS, typename T>
-__host__ __device__ inline void riemannFlux(const T *UL, const T *UR, const T *ULm, const T *URm, const real *n,
-                                            const GasParams &gp, real dLambda, T *F, T &lam0, T &lam123, T &lam4)
-{
-    RoeAveT<T> r;
-    roeAverage(ULm, URm, gp.gamma, r);
-    riemannFluxR<RS>(UL, UR, r, n, gp, dLambda, F, lam0, lam123, lam4);
 }
 
 // Batched Roe flux: eigenvalues from the cell-mean Roe average on the mean face
