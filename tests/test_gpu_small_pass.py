@@ -1,6 +1,7 @@
 """The one-pass residual and time step of small meshes against the two-pass form (the no-allocation
 entry keeps it) and the oracle, over the face rules, partly filled blocks and slots, boundary faces,
-a residual written over the state, whole SSP-RK3 steps, and meshes just above the limits."""
+a residual written over the state, whole SSP-RK3 steps, and meshes just above the limits, whose default
+form is the two-pass one: those against the oracle."""
 from __future__ import annotations
 
 import ctypes as C
@@ -32,6 +33,9 @@ def _mesh(kind):
                            seed=3), [bc.BC_WALL, bc.BC_WALL_INVIS]
     if kind == "quad33k":  # above both limits
         return mm.periodic_quad_grid(183, 181, 1.0, 0.8, jitter=0.1, seed=3), None
+    if kind == "mixed33k":
+        return mm.mixed_grid(180, 123, 1.0, 1.0, periodic=(True, False), zones=zones, jitter=0.05,
+                             seed=3), [bc.BC_WALL, bc.BC_SYM]
     n = dict(tet16k=(14, 14, 14), tet33k=(18, 18, 17))[kind]  # above the viscous limit of tetrahedra, above both
     return mm.tet_grid(*n, 1.0, 1.0, 1.0, periodic=(True, False, True), zones=zones, jitter=0.05,
                        seed=3), [bc.BC_WALL, bc.BC_WALL_INVIS]
@@ -52,7 +56,7 @@ def _setup(kind, rs, viscous):
 
 @pytest.mark.parametrize("viscous", [False, True])
 @pytest.mark.parametrize("rs", ["Roe", "HLLEP"])
-@pytest.mark.parametrize("kind", ["quad1", "tri", "mixed", "tet", "quad33k", "tet16k", "tet33k"])
+@pytest.mark.parametrize("kind", ["quad1", "tri", "mixed", "tet", "quad33k", "mixed33k", "tet16k", "tet33k"])
 def test_same_as_two_passes(require_gpu, kind, rs, viscous):
     from dndsr_amd._lib import check, lib
     from dndsr_amd.cfv import _ptr
@@ -62,8 +66,20 @@ def test_same_as_two_passes(require_gpu, kind, rs, viscous):
     du, dr, rhs, two = g.to_device(u), g.to_device(rec), g.BuildUDof(5), g.BuildUDof(5)
     dt = g.BuildUDof(1)[0]
     ev.EvaluateDt(dt, du, None, CFL=0.7)
+    o = None
+    if kind.endswith("k"):
+        import pyoracle as po
+        o = po.OracleVR(m, **s, **zw)
+        if types:
+            o.set_bc(types, np.ones((len(types), 5)), 1.4)
+        es = po.OracleVR.euler_settings(1.4, RS[rs], 0, 1.0, 1.0, viscous=int(viscous), muModel=1, **GAS)
+        dlc = o.eval_dt(es, u, 1.0, 1e100, True)[2]
+    assert (g.nCell > 32768) == kind.endswith("33k") and (16384 < g.nCell <= 32768) == (kind == "tet16k")
     for r in (dr, None):
         ev.EvaluateRHS(rhs, None, du, r, r)
+        if o is not None:
+            want = o.eval_rhs(es, u, None if r is None else rec, dlc)
+            assert rel_l2(g.to_host(rhs), want) <= 1e-12
         check(lib().dndsr_eval_rhs_noalloc(ev.ctx.h, C.byref(ev.es), _ptr(du), None if r is None else _ptr(r),
                                            _ptr(ev.deltaLambdaCell), _ptr(two)))
         ev.ctx.sync()
