@@ -356,9 +356,10 @@ def laminar_kernel_rooflines(g, run, iters, sgsIter):
     """Per-kernel averages of `iters` implicit iterations (per-launch HIP events) with FP64 and
     with FP32 sweeps, against the algorithmic bytes per cell of the tetrahedral p1 case:
     EvaluateRHS (face + viscous + gather passes) B_RHS, the VR sweep B_VR, one SGS sweep over
-    all colours 8 (5 nV + 1) + f_c (4 + s (2 + d)) + s (5 nV + 1) with s the sweep's precision
-    (rhs, JDiag, the cell's increment in and out; per face the neighbour, its state and
-    increment, the face geometry)."""
+    all colours s (3 nV + 1 + d + 1) + f_c (4 + s (1 + d)) with s the sweep's precision: every
+    array once (rhs, the increment in and out, 1 / JDiag, the state's velocity and enthalpy; per
+    face lambda, the scaled normal and the neighbour's index).  A visit sums one side's neighbours
+    and keeps the other half, so a neighbour's rows are not counted again per visit."""
     from dndsr_amd import _lib
     L_ = _lib.lib()
     nk = len(_lib.KERNEL_IDS)
@@ -384,7 +385,7 @@ def laminar_kernel_rooflines(g, run, iters, sgsIter):
         processed = sweeps * N - (1 + sgsIter) * int(cs[-1]) - sgsIter * int(cs[0])
         sgs_ms = per_it("sgs_colour") * N / processed
         s_ = 4 if fp32 else 8
-        b_sgs = 8 * (5 * 5 + 1) + f_c * (4 + s_ * (2 + 3)) + s_ * (5 * 5 + 1)
+        b_sgs = s_ * (3 * 5 + 1 + 3 + 1) + f_c * (4 + s_ * (1 + 3))
         ent = {}
         for key, t, b in (("eval_rhs", rhs_ms, b_rhs), ("vr_iter", vr_ms, b_vr), ("sgs_sweep", sgs_ms, b_sgs)):
             if t > 0:
