@@ -290,7 +290,8 @@ void launchLUSGSInitBlock(Ctx &c, const GasParams &gp, const real *dTau, real dt
 // The first and the last colour have neighbours on one side only and keep nothing.  Two implicit
 // iterations, all neighbours in each visit against one side (5 colours on tetrahedra, 3 on the mixed 2-D
 // mesh, 5 extra sweeps there): 24 576 tetrahedra 457 / 442 us, 279 936 1141 / 1120 us, 944 784 in FP32
-// 2401 / 2318 us; blocks on 50k cells of the 2-D mesh 652 / 596 us, on 97k 795 / 729 us.
+// 2401 / 2318 us; blocks on 50k cells of the 2-D mesh 652 / 596 us, on 97k 795 / 729 us; the scalar solve
+// on 200k cells of it, where they do not pay, 746 / 747 us.
 enum SGSSide { SGS_NONE = 0, SGS_BEFORE = 1, SGS_AFTER = 2, SGS_ALL = 3 };
 struct SGSVisit
 {

@@ -245,8 +245,8 @@ __device__ inline void faceLambdas(const T *lam, const T *lamRoe, size_t F, idx 
 // JacobianDiagBlock::GetInvert (EulerJacobian.hpp:153-190): J^-1 = (D^-1 J)^-1 D^-1 with the
 // scaled block inverted by Gauss-Jordan elimination with complete pivoting.  Returns false for a
 // zero diagonal or a singular block.  Every index is a compile-time constant (the row and column
-// exchanges are selects over the candidates), so both blocks stay in registers: indexed by the pivot
-// they lived in scratch memory, which bound the kernels that call this.
+// exchanges are selects over the candidates), so that the blocks need no indexed scratch memory, which
+// bound the kernels that call this (kSGSBlkPrep keeps 60 B of spills, 400 with gas-dependent ghosts).
 __device__ inline bool invertBlock5(const real (&J)[25], real (&Jinv)[25])
 {
     real P[5][5], X[5][5], dinv[5];

@@ -341,8 +341,8 @@ __device__ inline void boundaryFaceBCC(const DevMesh &m, idx f, const real *mom,
 // pass is bound by its chain of dependent loads and arithmetic, not by bandwidth.  A block is 64
 // faces with one wavefront per face point (two rounds of points above 8): the points' basis values
 // and increments go through LDS, then wavefront w forms the column v = w, w + NW, ... of BCC in point
-// order and applies A^-1.  35k triangles of a tetrahedral mesh at p1: 38 us
-// with the points read from the face tables, one thread per face 51.
+// order and applies A^-1.  35k triangles of a tetrahedral mesh at p1: 25 us (38 with the points read from
+// the face tables, 51 with one thread per face).
 template <int DIM, int NDOF, int NV, int MODE>
 __global__ void __launch_bounds__(512) kVRBndFace(DevMesh m, const real *__restrict__ uRec, const real *__restrict__ u,
                                                   const real *__restrict__ x, real *__restrict__ out)
